@@ -116,15 +116,14 @@ __global__ void k_bbounce_end(uint32_t* c, unsigned long long* stats) {
 }
 
 // Closest hit of the queued rays, each against its own scene's BVH8:
-// persistent waves with ray refill over a contiguous slice each.
-template <int STACK, int TB>
-__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(STACK <= 10 ? 8 : 1, 8))) void k_btrace(SceneMany ss, const float4* __restrict__ org,
-                                               const float4* __restrict__ dir, const uint32_t* __restrict__ q_path,
-                                               const uint32_t* __restrict__ count, HitArrays hit) {
-    __shared__ uint2 stk[STACK * TB];
+// persistent waves with ray refill.
+template <int STACK>
+__global__ __launch_bounds__(64 * kBatchWaves)
+    __attribute__((amdgpu_waves_per_eu(trace_waves_per_simd(STACK), 8))) void k_btrace(
+        SceneMany ss, const float4* __restrict__ org, const float4* __restrict__ dir,
+        const uint32_t* __restrict__ q_path, const uint32_t* __restrict__ count, HitArrays hit) {
+    __shared__ TraceLds<STACK, kBatchWaves> lds;
     const uint32_t n = *count;
-    const uint32_t nwaves = gridDim.x * (TB / 64);
-    const uint32_t wave = blockIdx.x * (TB / 64) + (threadIdx.x >> 6);
     auto load = [&](uint32_t i, Ray& ray, const uint4*& nd, const float4*& tr) {
         float4 a = org[i], d = dir[i];
         ray = Ray{a.x, a.y, a.z, a.w, d.x, d.y, d.z, d.w};
@@ -137,10 +136,8 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(STACK <= 10 
         if (res.rec != 0xFFFFFFFFu) {
             const float4* tris = ss.at(q_path[i]).leaf;
             float4 r2 = tris[(size_t)res.rec * kTriWords + 2];
-            float4 a = org[i], d = dir[i];
-            Ray ray{a.x, a.y, a.z, a.w, d.x, d.y, d.z, d.w};
             float u, v;
-            hit_uv(tris, res.rec, ray, u, v);
+            hit_uv(tris, res.rec, st.p, u, v);
             hit.t[i] = res.t;
             hit.inst[i] = __float_as_uint(r2.y);
             hit.prim[i] = __float_as_uint(r2.z);
@@ -154,7 +151,7 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(STACK <= 10 
             hit.v[i] = 0.0f;
         }
     };
-    refill_trace<false, false, STACK, kRefillLanes>(n, wave, nwaves, &stk[threadIdx.x], TB, load, done);
+    refill_trace<false, false, STACK, kStepsPerRefill>(n, lds, kRefillLanes, load, done);
 }
 
 // The late bounces of the batch, one thread per path (tail_paths).
@@ -303,13 +300,12 @@ __global__ void k_bq_apply(const float4* __restrict__ meta, const float4* __rest
                             r.w);
 }
 
-template <int STACK, int TB>
-__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(STACK <= 10 ? 8 : 1, 8))) void k_bshadow(SceneMany ss, ShadowQueue sq, const uint32_t* __restrict__ counts,
-                                                float4* __restrict__ rad) {
-    __shared__ uint2 stk[STACK * TB];
+template <int STACK>
+__global__ __launch_bounds__(64 * kBatchWaves)
+    __attribute__((amdgpu_waves_per_eu(trace_waves_per_simd(STACK), 8))) void k_bshadow(
+        SceneMany ss, ShadowQueue sq, const uint32_t* __restrict__ counts, float4* __restrict__ rad) {
+    __shared__ TraceLds<STACK, kBatchWaves> lds;
     const uint32_t n = counts[2];
-    const uint32_t nwaves = gridDim.x * (TB / 64);
-    const uint32_t wave = blockIdx.x * (TB / 64) + (threadIdx.x >> 6);
     auto load = [&](uint32_t i, Ray& ray, const uint4*& nd, const float4*& tr) {
         ray = shadow_ray(sq, i);
         const SceneDev& S = ss.at(__float_as_uint(sq.contrib[i].w));
@@ -317,7 +313,7 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(STACK <= 10 
         tr = S.leaf;
     };
     auto done = [&](uint32_t i, const TravState& st, uint32_t, uint32_t) { shadow_done(sq, i, st.res, rad); };
-    refill_trace<true, false, STACK, kRefillLanes>(n, wave, nwaves, &stk[threadIdx.x], TB, load, done);
+    refill_trace<true, false, STACK, kStepsPerRefill>(n, lds, kRefillLanes, load, done);
 }
 
 // Radiance of the group's paths -> each view's output (and running mean).
@@ -375,7 +371,7 @@ struct snkpt_batch {
     std::vector<Group> groups;
     snkpt_batch_tuning tuning{128, 16, 8, 0, 0.0f, 0, {0, 0}};
     bool tables_dirty = true;
-    uint32_t stack = 16;  // traversal stack entries (deepest scene)
+    uint32_t stack = 16;  // traversal stack entries the deepest scene needs
     uint32_t cap = 0;     // queue capacity allocated (paths)
     uint64_t accum_total = 0;
     uint64_t camera_rays = 0;
@@ -440,12 +436,8 @@ snkpt_status bfail(snkpt_batch* B, snkpt_status code, const std::string& msg) {
             return bfail(B, SNKPT_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
-// Smallest traversal stack for the deepest scene: 10 and 12 entries let 16
-// and 13 blocks of 128 lanes share a CU's 160 KB of LDS, against 10 for 16.
-uint32_t stack_for(uint32_t depth) {
-    uint32_t need = depth > 0 ? depth - 1 : 0;
-    return need <= 10 ? 10u : need <= 12 ? 12u : need <= 16 ? 16u : need <= 32 ? 32u : 64u;
-}
+// Traversal stack entries for a BVH8 of this depth.
+uint32_t stack_for(uint32_t depth) { return depth > 0 ? depth - 1 : 0; }
 
 // Scene table, view table (group-relative path offsets), groups, buffers.
 snkpt_status prepare(snkpt_batch* B, hipStream_t st) {
@@ -539,31 +531,23 @@ snkpt_status prepare(snkpt_batch* B, hipStream_t st) {
     return SNKPT_OK;
 }
 
-template <int STACK, int TB>
-void launch_traces(snkpt_batch* B, const SceneMany& ss, int cur, uint32_t grid, hipStream_t st, bool shadow) {
-    if (!shadow) {
-        HitArrays hit{B->h_t.as<float>(), B->h_inst.as<uint32_t>(), B->h_prim.as<uint32_t>(), B->h_u.as<float>(),
-                      B->h_v.as<float>()};
-        k_btrace<STACK, TB><<<grid, TB, 0, st>>>(ss, B->q_org[cur].as<float4>(), B->q_dir[cur].as<float4>(),
-                                                 B->q_path[cur].as<uint32_t>(), B->counts.as<uint32_t>() + cur, hit);
-    } else {
-        ShadowQueue sq{B->s_org.as<float4>(), B->s_dir.as<float4>(), B->s_contrib.as<float4>()};
-        k_bshadow<STACK, TB><<<grid, TB, 0, st>>>(ss, sq, B->counts.as<uint32_t>(), B->rad.as<float4>());
-    }
-}
-
-template <int TB>
-void launch_traces_tb(snkpt_batch* B, const SceneMany& ss, int cur, uint32_t grid, hipStream_t st, bool shadow) {
-    if (B->stack <= 10)
-        launch_traces<10, TB>(B, ss, cur, grid, st, shadow);
-    else if (B->stack <= 12)
-        launch_traces<12, TB>(B, ss, cur, grid, st, shadow);
-    else if (B->stack <= 16)
-        launch_traces<16, TB>(B, ss, cur, grid, st, shadow);
-    else if (B->stack <= 32)
-        launch_traces<32, TB>(B, ss, cur, grid, st, shadow);
-    else
-        launch_traces<64, TB>(B, ss, cur, grid, st, shadow);
+void launch_traces(snkpt_batch* B, const SceneMany& ss, int cur, hipStream_t st, bool shadow) {
+    // trace_block lanes x trace_blocks_per_cu blocks, as waves per CU
+    const uint32_t waves = (B->tuning.trace_block == 64 ? 1u : 2u) * std::max(1u, B->tuning.trace_blocks_per_cu);
+    with_stack(B->stack, [&](auto s) {
+        constexpr int S = decltype(s)::value;
+        const TraceGrid g = trace_grid(S, kBatchWaves, waves, (uint32_t)B->cus, B->cap);
+        if (!shadow) {
+            HitArrays hit{B->h_t.as<float>(), B->h_inst.as<uint32_t>(), B->h_prim.as<uint32_t>(),
+                          B->h_u.as<float>(), B->h_v.as<float>()};
+            k_btrace<S><<<g.blocks, g.threads, 0, st>>>(ss, B->q_org[cur].as<float4>(), B->q_dir[cur].as<float4>(),
+                                                        B->q_path[cur].as<uint32_t>(),
+                                                        B->counts.as<uint32_t>() + cur, hit);
+        } else {
+            ShadowQueue sq{B->s_org.as<float4>(), B->s_dir.as<float4>(), B->s_contrib.as<float4>()};
+            k_bshadow<S><<<g.blocks, g.threads, 0, st>>>(ss, sq, B->counts.as<uint32_t>(), B->rad.as<float4>());
+        }
+    });
 }
 
 void launch_btail(snkpt_batch* B, const SceneMany& ss, const PtParams& P, int cur, hipStream_t st) {
@@ -600,8 +584,6 @@ snkpt_status record_frame(snkpt_batch* B, const snkpt_settings* s, hipStream_t s
                   B->h_v.as<float>()};
     uint32_t* counts = B->counts.as<uint32_t>();
     unsigned long long* stats = B->stats.as<unsigned long long>();
-    const uint32_t tb = B->tuning.trace_block == 64 ? 64u : 128u;
-    const uint32_t tgrid = (uint32_t)B->cus * std::max(1u, B->tuning.trace_blocks_per_cu);
     const uint32_t sgrid = (uint32_t)B->cus * std::max(1u, B->tuning.shade_blocks_per_cu);
     const uint32_t ggrid = (uint32_t)B->cus * 8u;
     const uint32_t tail = batch_tail_from(B->tuning, P);
@@ -619,18 +601,12 @@ snkpt_status record_frame(snkpt_batch* B, const snkpt_settings* s, hipStream_t s
                 launch_btail(B, ss, P, cur, st);
                 break;
             }
-            if (tb == 64)
-                launch_traces_tb<64>(B, ss, cur, tgrid, st, false);
-            else
-                launch_traces_tb<128>(B, ss, cur, tgrid, st, false);
+            launch_traces(B, ss, cur, st, false);
             Queue qin{B->q_org[cur].as<float4>(), B->q_dir[cur].as<float4>(), B->q_path[cur].as<uint32_t>()};
             Queue qout{B->q_org[nxt].as<float4>(), B->q_dir[nxt].as<float4>(), B->q_path[nxt].as<uint32_t>()};
             k_bshade<0><<<sgrid, kBBlock, 0, st>>>(ss, P, qin, hit, qout, sq, ps, B->rad.as<float4>(), counts,
                                                    (uint32_t)cur, (uint32_t)nxt, ShadeHooks{});
-            if (tb == 64)
-                launch_traces_tb<64>(B, ss, cur, tgrid, st, true);
-            else
-                launch_traces_tb<128>(B, ss, cur, tgrid, st, true);
+            launch_traces(B, ss, cur, st, true);
             cur = nxt;
         }
         k_bbounce_end<<<1, 64, 0, st>>>(counts, stats);
@@ -812,8 +788,6 @@ snkpt_status record_cache_render(snkpt_batch* B, const snkpt_settings* s, hipStr
     H.q_samples = B->q_samples.as<float>();
     H.q_meta = B->q_meta.as<float4>();
     H.q_count = counts + 3;
-    const uint32_t tb = B->tuning.trace_block == 64 ? 64u : 128u;
-    const uint32_t tgrid = (uint32_t)B->cus * std::max(1u, B->tuning.trace_blocks_per_cu);
     const uint32_t sgrid = (uint32_t)B->cus * std::max(1u, B->tuning.shade_blocks_per_cu);
     const uint32_t ggrid = (uint32_t)B->cus * 8u;
     uint32_t* d_hist = B->hist.as<uint32_t>();
@@ -831,18 +805,12 @@ snkpt_status record_cache_render(snkpt_batch* B, const snkpt_settings* s, hipStr
         for (uint32_t b = 0; b < P.max_depth; ++b) {
             const int nxt = cur ^ 1;
             k_bbounce<<<1, 64, 0, st>>>(counts, (uint32_t)cur, (uint32_t)nxt, stats, b > 0 ? 1u : 0u);
-            if (tb == 64)
-                launch_traces_tb<64>(B, ss, cur, tgrid, st, false);
-            else
-                launch_traces_tb<128>(B, ss, cur, tgrid, st, false);
+            launch_traces(B, ss, cur, st, false);
             Queue qin{B->q_org[cur].as<float4>(), B->q_dir[cur].as<float4>(), B->q_path[cur].as<uint32_t>()};
             Queue qout{B->q_org[nxt].as<float4>(), B->q_dir[nxt].as<float4>(), B->q_path[nxt].as<uint32_t>()};
             k_bshade<1><<<sgrid, kBBlock, 0, st>>>(ss, P, qin, hit, qout, sq, ps, B->rad.as<float4>(), counts,
                                                    (uint32_t)cur, (uint32_t)nxt, H);
-            if (tb == 64)
-                launch_traces_tb<64>(B, ss, cur, tgrid, st, true);
-            else
-                launch_traces_tb<128>(B, ss, cur, tgrid, st, true);
+            launch_traces(B, ss, cur, st, true);
             cur = nxt;
         }
         k_bbounce_end<<<1, 64, 0, st>>>(counts, stats);

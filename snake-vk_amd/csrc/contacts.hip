@@ -14,8 +14,6 @@
 namespace snkpt {
 namespace {
 
-constexpr int kBlock = 128;
-
 struct ContactScene {
     const InstD* inst;
     const float4* xf;       // per instance: 3x4 object->world rows, then 3 normal-matrix rows
@@ -25,24 +23,15 @@ struct ContactScene {
     const float* nrm;
 };
 
-// Waves per SIMD the stacks' LDS leaves room for (8-byte entries, 128 lanes a block,
-// 160 KiB a CU): 8 for 10 entries (16 blocks), 6 for 12 (13 blocks, 12 launched).  The
-// register budget is held to that count: what spills is the contact record of the
-// completion handler, run once per ray, not the traversal loop.
 template <int STACK>
-constexpr int contact_waves() { return STACK <= 10 ? 8 : STACK <= 12 ? 6 : 1; }
-
-template <int STACK>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(contact_waves<STACK>(), 8))) void k_contacts(const float4* __restrict__ org_tmin,
-                                                     const float4* __restrict__ dir_tmax, uint32_t n,
-                                                     const uint4* __restrict__ nodes, const float4* __restrict__ tris,
-                                                     ContactScene C, float timestep, float* __restrict__ t_out,
-                                                     float4* __restrict__ n_out, float4* __restrict__ p_out,
-                                                     float4* __restrict__ v_out, uint32_t* __restrict__ inst_out,
-                                                     uint32_t* __restrict__ prim_out, uint32_t refill) {
-    __shared__ uint2 stk[STACK * kBlock];
-    const uint32_t nwaves = gridDim.x * (kBlock / 64);
-    const uint32_t wave = blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6);
+__global__ __launch_bounds__(64 * trace_waves(STACK))
+    __attribute__((amdgpu_waves_per_eu(trace_waves_per_simd(STACK), 8))) void k_contacts(
+        const float4* __restrict__ org_tmin, const float4* __restrict__ dir_tmax, uint32_t n,
+        const uint4* __restrict__ nodes, const float4* __restrict__ tris, ContactScene C, float timestep,
+        float* __restrict__ t_out, float4* __restrict__ n_out, float4* __restrict__ p_out,
+        float4* __restrict__ v_out, uint32_t* __restrict__ inst_out, uint32_t* __restrict__ prim_out,
+        uint32_t refill) {
+    __shared__ TraceLds<STACK> lds;
     auto load = [&](uint32_t id, Ray& ray, const uint4*& nd, const float4*& tr) {
         const float4 a = org_tmin[id], d = dir_tmax[id];
         ray = Ray{a.x, a.y, a.z, a.w, d.x, d.y, d.z, d.w};
@@ -66,7 +55,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(contact_
         const float4 r2 = tris[(size_t)res.rec * kTriWords + 2];
         const uint32_t ii = __float_as_uint(r2.y), prim = __float_as_uint(r2.z);
         float u, v;
-        hit_uv(tris, res.rec, ray, u, v);
+        hit_uv(tris, res.rec, st.p, u, v);
         // ParticleUpdate.rchit:40-62
         const InstD in = C.inst[ii];
         const uint32_t* ix = C.idx + in.index_offset + 3 * prim;
@@ -95,8 +84,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(contact_
         if (inst_out) inst_out[id] = ii;
         if (prim_out) prim_out[id] = prim;
     };
-    refill_trace_tuned<true, false, STACK, kStepsPerRefill>(n, wave, nwaves, &stk[threadIdx.x], kBlock, refill, load,
-                                                             done);
+    refill_trace<true, false, STACK, kStepsPerRefill>(n, lds, refill, load, done);
 }
 
 __global__ void k_contacts_empty(uint32_t n, float* t_out, float4* n_out, float4* p_out, float4* v_out,
@@ -129,9 +117,6 @@ snkpt_status trace_contacts(snkpt_ctx* ctx, const float4* org_tmin, const float4
         const uint32_t need = A.depth > 0 ? A.depth - 1 : 0;
         if (need > 64) return fail(ctx, SNKPT_ERR_CAPACITY, "trace_contacts: BVH8 deeper than the 64-entry stack");
         const uint32_t cus = ctx->props.multiProcessorCount > 0 ? (uint32_t)ctx->props.multiProcessorCount : 256u;
-        // resident blocks per CU by the stacks' LDS, an even count (two waves per block over four SIMDs)
-        const uint32_t per_cu = need <= 10 ? 16u : need <= 12 ? 12u : need <= 16 ? 10u : need <= 32 ? 4u : 2u;
-        const uint32_t grid = std::min((n + kBlock - 1) / kBlock, cus * per_cu);
         // the any-hit refill threshold the build's autotuner picked
         const uint32_t refill = A.shape[1].refill ? A.shape[1].refill : 16u;
         const ContactScene C{ctx->d_inst.as<InstD>(), ctx->d_inst_xf.as<float4>(),
@@ -140,20 +125,12 @@ snkpt_status trace_contacts(snkpt_ctx* ctx, const float4* org_tmin, const float4
         if (!C.prev_xf) return fail(ctx, SNKPT_ERR_NOT_BUILT, "trace_contacts: no previous-frame transforms");
         const uint4* nodes = A.nodes.as<uint4>();
         const float4* tris = A.leaf_tris.as<float4>();
-#define SNKPT_CONTACTS(S)                                                                                     \
-    k_contacts<S><<<grid, kBlock, 0, st>>>(org_tmin, dir_tmax, n, nodes, tris, C, timestep, out.t, nrm, pos, vel, \
-                                           out.inst, out.prim, refill)
-        if (need <= 10)
-            SNKPT_CONTACTS(10);
-        else if (need <= 12)
-            SNKPT_CONTACTS(12);
-        else if (need <= 16)
-            SNKPT_CONTACTS(16);
-        else if (need <= 32)
-            SNKPT_CONTACTS(32);
-        else
-            SNKPT_CONTACTS(64);
-#undef SNKPT_CONTACTS
+        with_stack(need, [&](auto s) {
+            constexpr int S = decltype(s)::value;
+            const TraceGrid g = trace_grid(S, trace_waves(S), (uint32_t)cu_waves(S), cus, n);
+            k_contacts<S><<<g.blocks, g.threads, 0, st>>>(org_tmin, dir_tmax, n, nodes, tris, C, timestep, out.t, nrm,
+                                                         pos, vel, out.inst, out.prim, refill);
+        });
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(ctx, e, "trace_contacts launch");

@@ -285,7 +285,7 @@ __device__ __forceinline__ float4 whole_path(const SceneDev& S, const CamDev& ca
 }
 
 // Lanes a persistent traversal wave waits for before refilling idle lanes.
-constexpr int kRefillLanes = 16;
+constexpr uint32_t kRefillLanes = 16;
 
 // Shadow-queue entry i as a ray; its contribution, added when unoccluded.
 __device__ __forceinline__ Ray shadow_ray(const ShadowQueue& sq, uint32_t i) {

@@ -30,7 +30,6 @@ namespace snkpt {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kShadowBlock = 128;
 
 __global__ void k_fill_f4(float4* p, uint32_t n, float4 v) {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -157,24 +156,21 @@ __global__ void k_gbuf_stats(const uint32_t* c, unsigned long long* stats) {
     }
 }
 
-// Shadow rays: persistent any-hit traversal with ray refill; each wave owns a
-// contiguous slice of the shadow queue.
+// Shadow rays: persistent any-hit traversal with ray refill.
 template <int STACK>
-__global__ __launch_bounds__(kShadowBlock) __attribute__((amdgpu_waves_per_eu(STACK <= 10 ? 8 : 1, 8))) void k_shadow(const uint4* __restrict__ nodes,
-                                                         const float4* __restrict__ tris, ShadowQueue sq,
-                                                         const uint32_t* __restrict__ counts,
-                                                         float4* __restrict__ rad) {
-    __shared__ uint2 stk[STACK * kShadowBlock];
+__global__ __launch_bounds__(64 * trace_waves(STACK))
+    __attribute__((amdgpu_waves_per_eu(trace_waves_per_simd(STACK), 8))) void k_shadow(
+        const uint4* __restrict__ nodes, const float4* __restrict__ tris, ShadowQueue sq,
+        const uint32_t* __restrict__ counts, float4* __restrict__ rad) {
+    __shared__ TraceLds<STACK> lds;
     const uint32_t nn = counts[2];
-    const uint32_t nwaves = gridDim.x * (kShadowBlock / 64);
-    const uint32_t wave = blockIdx.x * (kShadowBlock / 64) + (threadIdx.x >> 6);
     auto load = [&](uint32_t i, Ray& ray, const uint4*& nd, const float4*& tr) {
         ray = shadow_ray(sq, i);
         nd = nodes;
         tr = tris;
     };
     auto done = [&](uint32_t i, const TravState& st, uint32_t, uint32_t) { shadow_done(sq, i, st.res, rad); };
-    refill_trace<true, false, STACK, kRefillLanes>(nn, wave, nwaves, &stk[threadIdx.x], kShadowBlock, load, done);
+    refill_trace<true, false, STACK, kStepsPerRefill>(nn, lds, kRefillLanes, load, done);
 }
 
 // Whole paths, one per thread (KIND 0: radiance into rad[i]; KIND 2: training
@@ -445,27 +441,13 @@ snkpt_status launch_shadow(snkpt_ctx* ctx, RenderState& R, float4* rad, hipStrea
     if (A.num_tris == 0) return SNKPT_OK;  // no hits, so no shadow rays were queued
     uint32_t need = A.depth > 0 ? A.depth - 1 : 0;
     const uint32_t cus = ctx->props.multiProcessorCount > 0 ? (uint32_t)ctx->props.multiProcessorCount : 256u;
-    // persistent grid: as many blocks as the LDS of the stack size lets stay resident
-    // (an even count: two waves per block spread evenly over the four SIMDs)
-    const uint32_t resident = need <= 10 ? 16u : need <= 12 ? 12u : need <= 16 ? 10u : need <= 32 ? 4u : 2u;
-    uint32_t grid = std::min(nblk(n_max ? n_max : R.w * R.h, kShadowBlock), cus * resident);
-    if (need <= 10)
-        k_shadow<10><<<grid, kShadowBlock, 0, st>>>(A.nodes.as<uint4>(), A.leaf_tris.as<float4>(), shadow_of(R),
-                                                     R.counts.as<uint32_t>(), rad);
-    else if (need <= 12)
-        k_shadow<12><<<grid, kShadowBlock, 0, st>>>(A.nodes.as<uint4>(), A.leaf_tris.as<float4>(), shadow_of(R),
-                                                     R.counts.as<uint32_t>(), rad);
-    else if (need <= 16)
-        k_shadow<16><<<grid, kShadowBlock, 0, st>>>(A.nodes.as<uint4>(), A.leaf_tris.as<float4>(), shadow_of(R),
-                                                     R.counts.as<uint32_t>(), rad);
-    else if (need <= 32)
-        k_shadow<32><<<grid, kShadowBlock, 0, st>>>(A.nodes.as<uint4>(), A.leaf_tris.as<float4>(), shadow_of(R),
-                                                     R.counts.as<uint32_t>(), rad);
-    else if (need <= 64)
-        k_shadow<64><<<grid, kShadowBlock, 0, st>>>(A.nodes.as<uint4>(), A.leaf_tris.as<float4>(), shadow_of(R),
-                                                     R.counts.as<uint32_t>(), rad);
-    else
-        return fail(ctx, SNKPT_ERR_CAPACITY, "shadow: BVH8 deeper than the 64-entry traversal stack");
+    const bool ok = with_stack(need, [&](auto s) {
+        constexpr int S = decltype(s)::value;
+        const TraceGrid g = trace_grid(S, trace_waves(S), (uint32_t)cu_waves(S), cus, n_max ? n_max : R.w * R.h);
+        k_shadow<S><<<g.blocks, g.threads, 0, st>>>(A.nodes.as<uint4>(), A.leaf_tris.as<float4>(), shadow_of(R),
+                                                    R.counts.as<uint32_t>(), rad);
+    });
+    if (!ok) return fail(ctx, SNKPT_ERR_CAPACITY, "shadow: BVH8 deeper than the 64-entry traversal stack");
     return SNKPT_OK;
 }
 

@@ -24,7 +24,9 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
+#include <type_traits>
 
 namespace snkpt {
 
@@ -45,20 +47,29 @@ struct RayPre {
     float ox, oy, oz;
     float ix, iy, iz;  // 1/d, NaN on a parallel axis
     float Sx, Sy, Sz;
-    // kx | ky << 2 | kz << 4 | oct << 6 | par << 9 in one register: the traversal
+    // the axis permutation, octant and parallel axes in one register: the traversal
     // loop keeps all of RayPre live, and as five registers they made the 64-VGPR
-    // closest-hit loop spill one register to scratch on every step
+    // closest-hit loop spill one register to scratch on every step.  Bits 0-5: kx
+    // is 0, kx is 1, ky is 0, ky is 1, kz is 0, kz is 1; oct << 6 | par << 9.
     uint32_t bits;
-    __device__ __forceinline__ int kx() const { return (int)(bits & 3u); }
-    __device__ __forceinline__ int ky() const { return (int)((bits >> 2) & 3u); }
-    __device__ __forceinline__ int kz() const { return (int)((bits >> 4) & 3u); }
+    // all ones where bit b is set
+    __device__ __forceinline__ uint32_t mask(int b) const { return (uint32_t)((int32_t)(bits << (31 - b)) >> 31); }
     // bit a set: the ray runs towards -a
     __device__ __forceinline__ uint32_t oct() const { return (bits >> 6) & 7u; }
     // bit a set: axis a is parallel
     __device__ __forceinline__ uint32_t par() const { return (bits >> 9) & 7u; }
 };
 
-__device__ __forceinline__ float sel3(float x, float y, float z, int k) { return k == 0 ? x : (k == 1 ? y : z); }
+// a where the mask's bits are set, else b.  V_BITOP3 issues in 2 cycles per wave
+// beside the other pipe; V_CNDMASK takes 4, and a run of them on one VCC measured
+// 15-22 cycles each (the near / far choice and the axis permutation are such runs).
+__device__ __forceinline__ uint32_t bit_sel(uint32_t a, uint32_t b, uint32_t m) {
+    return __builtin_amdgcn_bitop3_b32(a, b, m, 0xE4);
+}
+// x, y or z by the masks of "is x" and "is y".
+__device__ __forceinline__ float sel3(float x, float y, float z, uint32_t mx, uint32_t my) {
+    return __uint_as_float(bit_sel(__float_as_uint(x), bit_sel(__float_as_uint(y), __float_as_uint(z), my), mx));
+}
 __device__ __forceinline__ float ubyte_f(uint32_t w, int b) { return (float)((w >> (8 * b)) & 0xFFu); }
 
 // 0xFF in byte i for every set bit i of a 4-bit mask.
@@ -76,31 +87,57 @@ __device__ __forceinline__ float safe_inv(float d) {
     return fabsf(d) < kParallelEps ? __builtin_nanf("") : 1.0f / d;
 }
 
+// 1 / d and x / d rounded as IEEE division rounds them, for 2^-60 <= |d| <= 2^60
+// and (quotient) 2^-60 <= |x| <= |d|: one Newton step on V_RCP_F32 gave the
+// correctly rounded reciprocal for each of the 2^23 mantissas, and Markstein's
+// correction then rounds the quotient correctly (no off result in 5e8 random
+// pairs).  3 + 3 instructions where the general division takes about 10.
+__device__ __forceinline__ float rcp_exact(float d) {
+    const float r = __builtin_amdgcn_rcpf(d);
+    return fmaf(fmaf(-d, r, 1.0f), r, r);
+}
+__device__ __forceinline__ float div_exact(float x, float d, float r) {
+    const float q = x * r;
+    return fmaf(fmaf(-q, d, x), r, q);
+}
+
 __device__ __forceinline__ RayPre ray_setup(const Ray& r) {
     RayPre p;
     p.ox = r.ox;
     p.oy = r.oy;
     p.oz = r.oz;
-    p.ix = safe_inv(r.dx);
-    p.iy = safe_inv(r.dy);
-    p.iz = safe_inv(r.dz);
-    float ax = fabsf(r.dx), ay = fabsf(r.dy), az = fabsf(r.dz);
-    int kz = (ax >= ay && ax >= az) ? 0 : (ay >= az ? 1 : 2);
+    const float ax = fabsf(r.dx), ay = fabsf(r.dy), az = fabsf(r.dz);
+    const int kz = (ax >= ay && ax >= az) ? 0 : (ay >= az ? 1 : 2);
     int kx = kz == 2 ? 0 : kz + 1;
     int ky = kx == 2 ? 0 : kx + 1;
-    float dkz = sel3(r.dx, r.dy, r.dz, kz);
+    const float dkz = kz == 0 ? r.dx : (kz == 1 ? r.dy : r.dz);
     if (dkz < 0.0f) {
         int t = kx;
         kx = ky;
         ky = t;
     }
-    p.Sx = sel3(r.dx, r.dy, r.dz, kx) / dkz;
-    p.Sy = sel3(r.dx, r.dy, r.dz, ky) / dkz;
-    p.Sz = 1.0f / dkz;
+    const float dkx = kx == 0 ? r.dx : (kx == 1 ? r.dy : r.dz);
+    const float dky = ky == 0 ? r.dx : (ky == 1 ? r.dy : r.dz);
+    constexpr float kLo = 0x1p-60f, kHi = 0x1p60f;
+    if (fminf(fminf(ax, ay), az) >= kLo && fmaxf(fmaxf(ax, ay), az) <= kHi) {
+        p.ix = rcp_exact(r.dx);
+        p.iy = rcp_exact(r.dy);
+        p.iz = rcp_exact(r.dz);
+        p.Sz = kz == 0 ? p.ix : (kz == 1 ? p.iy : p.iz);
+        p.Sx = div_exact(dkx, dkz, p.Sz);
+        p.Sy = div_exact(dky, dkz, p.Sz);
+    } else {
+        p.ix = safe_inv(r.dx);
+        p.iy = safe_inv(r.dy);
+        p.iz = safe_inv(r.dz);
+        p.Sx = dkx / dkz;
+        p.Sy = dky / dkz;
+        p.Sz = 1.0f / dkz;
+    }
     const uint32_t oct = (p.ix < 0.0f ? 1u : 0u) | (p.iy < 0.0f ? 2u : 0u) | (p.iz < 0.0f ? 4u : 0u);
-    const uint32_t par = (fabsf(r.dx) < kParallelEps ? 1u : 0u) | (fabsf(r.dy) < kParallelEps ? 2u : 0u) |
-                         (fabsf(r.dz) < kParallelEps ? 4u : 0u);
-    p.bits = (uint32_t)kx | (uint32_t)ky << 2 | (uint32_t)kz << 4 | oct << 6 | par << 9;
+    const uint32_t par = (ax < kParallelEps ? 1u : 0u) | (ay < kParallelEps ? 2u : 0u) | (az < kParallelEps ? 4u : 0u);
+    p.bits = (kx == 0 ? 1u : 0u) | (kx == 1 ? 2u : 0u) | (ky == 0 ? 4u : 0u) | (ky == 1 ? 8u : 0u) |
+             (kz == 0 ? 16u : 0u) | (kz == 1 ? 32u : 0u) | oct << 6 | par << 9;
     return p;
 }
 
@@ -114,13 +151,14 @@ __device__ __forceinline__ bool intersect_tri(const RayPre& p, float v0x, float 
     float Ax_ = v0x - p.ox, Ay_ = v0y - p.oy, Az_ = v0z - p.oz;
     float Bx_ = v1x - p.ox, By_ = v1y - p.oy, Bz_ = v1z - p.oz;
     float Cx_ = v2x - p.ox, Cy_ = v2y - p.oy, Cz_ = v2z - p.oz;
-    float Akz = sel3(Ax_, Ay_, Az_, p.kz()), Bkz = sel3(Bx_, By_, Bz_, p.kz()), Ckz = sel3(Cx_, Cy_, Cz_, p.kz());
-    float Ax = sel3(Ax_, Ay_, Az_, p.kx()) - p.Sx * Akz;
-    float Ay = sel3(Ax_, Ay_, Az_, p.ky()) - p.Sy * Akz;
-    float Bx = sel3(Bx_, By_, Bz_, p.kx()) - p.Sx * Bkz;
-    float By = sel3(Bx_, By_, Bz_, p.ky()) - p.Sy * Bkz;
-    float Cx = sel3(Cx_, Cy_, Cz_, p.kx()) - p.Sx * Ckz;
-    float Cy = sel3(Cx_, Cy_, Cz_, p.ky()) - p.Sy * Ckz;
+    const uint32_t x0 = p.mask(0), x1 = p.mask(1), y0 = p.mask(2), y1 = p.mask(3), z0 = p.mask(4), z1 = p.mask(5);
+    float Akz = sel3(Ax_, Ay_, Az_, z0, z1), Bkz = sel3(Bx_, By_, Bz_, z0, z1), Ckz = sel3(Cx_, Cy_, Cz_, z0, z1);
+    float Ax = sel3(Ax_, Ay_, Az_, x0, x1) - p.Sx * Akz;
+    float Ay = sel3(Ax_, Ay_, Az_, y0, y1) - p.Sy * Akz;
+    float Bx = sel3(Bx_, By_, Bz_, x0, x1) - p.Sx * Bkz;
+    float By = sel3(Bx_, By_, Bz_, y0, y1) - p.Sy * Bkz;
+    float Cx = sel3(Cx_, Cy_, Cz_, x0, x1) - p.Sx * Ckz;
+    float Cy = sel3(Cx_, Cy_, Cz_, y0, y1) - p.Sy * Ckz;
     U = Cx * By - Cy * Bx;
     V = Ax * Cy - Ay * Cx;
     W = Bx * Ay - By * Ax;
@@ -199,9 +237,9 @@ __device__ __forceinline__ bool trav_init(const Ray& ray, TravState& s) {
 }
 
 // Tests the next pending leaf triangle of the ray (st.tg_hits must be non-zero);
-// true when ANY and it is a hit.
-template <bool ANY, bool COUNT>
-__device__ __forceinline__ bool trav_tri(const float4* __restrict__ tris, TravState& st, uint32_t& tvis) {
+// true when `any` and it is a hit.
+template <bool COUNT>
+__device__ __forceinline__ bool trav_tri(const float4* __restrict__ tris, TravState& st, bool any, uint32_t& tvis) {
     const uint32_t j = __builtin_ctz(st.tg_hits);
     st.tg_hits &= st.tg_hits - 1u;
     const uint32_t rec = st.tg_base + j;
@@ -215,7 +253,7 @@ __device__ __forceinline__ bool trav_tri(const float4* __restrict__ tris, TravSt
             st.res.t = t;
             st.res.gid = gid;
             st.res.rec = rec;
-            if (ANY) return true;
+            if (any) return true;
         }
     }
     return false;
@@ -235,17 +273,18 @@ constexpr int kTrisPerStep = 1;
 // none is left, the next node of the current group (its 8 child boxes, which
 // sets the pending triangles of its hit leaves); pops the stack when the group
 // is empty.  Returns true when the ray is finished.  `stk` points to this lane's
-// first stack entry in LDS; consecutive entries are `stride` uint2 apart.
-template <bool ANY, bool COUNT, int STACK>
+// first stack entry in LDS; consecutive entries are `stride` uint2 apart.  `any`:
+// the first hit found ends the ray (a constant, or per lane in the path kernels).
+template <bool COUNT>
 __device__ __forceinline__ bool trav_step(const uint4* __restrict__ nodes, const float4* __restrict__ tris,
-                                          TravState& st, uint2* stk, int stride, uint32_t& nvis, uint32_t& tvis) {
+                                          TravState& st, uint2* stk, int stride, bool any, uint32_t& nvis,
+                                          uint32_t& tvis) {
     const RayPre& p = st.p;
     const float tmin = st.tmin;
 #pragma unroll
     for (int i = 0; i < kTrisPerStep; ++i)
-        if (st.tg_hits && trav_tri<ANY, COUNT>(tris, st, tvis)) return true;
+        if (st.tg_hits && trav_tri<COUNT>(tris, st, any, tvis)) return true;
     if (!st.tg_hits && (st.ng_hits & 0xFF000000u)) {
-        const bool nx = p.ix < 0.0f, ny = p.iy < 0.0f, nz = p.iz < 0.0f;
         uint32_t k = __builtin_ctz(st.ng_hits >> 24);
         st.ng_hits &= ~(1u << (24 + k));
         uint32_t s = k ^ p.oct();
@@ -265,12 +304,15 @@ __device__ __forceinline__ bool trav_step(const uint4* __restrict__ nodes, const
         float az = (__uint_as_float(w0.z) - p.oz) * p.iz;
         uint32_t imask = w0.w >> 24;
         // near / far plane bytes per axis (qlo first for a positive direction)
-        uint32_t nx0 = nx ? w3.z : w2.x, nx1 = nx ? w3.w : w2.y;
-        uint32_t fx0 = nx ? w2.x : w3.z, fx1 = nx ? w2.y : w3.w;
-        uint32_t ny0 = ny ? w4.x : w2.z, ny1 = ny ? w4.y : w2.w;
-        uint32_t fy0 = ny ? w2.z : w4.x, fy1 = ny ? w2.w : w4.y;
-        uint32_t nz0 = nz ? w4.z : w3.x, nz1 = nz ? w4.w : w3.y;
-        uint32_t fz0 = nz ? w3.x : w4.z, fz1 = nz ? w3.y : w4.w;
+        const uint32_t nx = (uint32_t)((int32_t)__float_as_uint(p.ix) >> 31);  // all ones: the ray runs towards -x
+        const uint32_t ny = (uint32_t)((int32_t)__float_as_uint(p.iy) >> 31);
+        const uint32_t nz = (uint32_t)((int32_t)__float_as_uint(p.iz) >> 31);
+        const uint32_t nx0 = bit_sel(w3.z, w2.x, nx), nx1 = bit_sel(w3.w, w2.y, nx);
+        const uint32_t fx0 = bit_sel(w2.x, w3.z, nx), fx1 = bit_sel(w2.y, w3.w, nx);
+        const uint32_t ny0 = bit_sel(w4.x, w2.z, ny), ny1 = bit_sel(w4.y, w2.w, ny);
+        const uint32_t fy0 = bit_sel(w2.z, w4.x, ny), fy1 = bit_sel(w2.w, w4.y, ny);
+        const uint32_t nz0 = bit_sel(w4.z, w3.x, nz), nz1 = bit_sel(w4.w, w3.y, nz);
+        const uint32_t fz0 = bit_sel(w3.x, w4.z, nz), fz1 = bit_sel(w3.y, w4.w, nz);
         // meta bytes of slots 0-3 and 4-7; a parallel-axis miss clears the slot's
         // byte, so it reads as empty below
         uint32_t m0 = w1.z, m1 = w1.w;
@@ -332,101 +374,198 @@ __device__ __forceinline__ TraceResult traverse(const uint4* __restrict__ nodes,
                                                 uint32_t& tvis) {
     TravState st;
     if (!trav_init(ray, st)) return st.res;
-    while (!trav_step<ANY, COUNT, STACK>(nodes, tris, st, stk, stride, nvis, tvis)) {
+    while (!trav_step<COUNT>(nodes, tris, st, stk, stride, ANY, nvis, tvis)) {
     }
     return st.res;
 }
 
-// Persistent traversal with ray refill (after Aila & Laine 2009, "Understanding
-// the efficiency of ray traversal on GPUs"), for the calling wave.  The rays
-// [0, n) are cut into bands of nwaves x 64 rays.  In every whole band wave w
-// owns the 64-ray chunk w (so the waves in flight trace one band of
-// neighbouring rays at a time and share its BVH nodes in L2); the last, partial
-// band is split evenly, wave w taking its [w rest / nwaves, (w+1) rest / nwaves)
-// slice, so no wave gets a whole chunk more than another.  Its rays are handed
-// out in order to idle lanes whenever at least REFILL lanes
-// are idle (or all are), so a wave does not wait for its slowest ray with the
-// other lanes masked off; between two such checks a lane takes up to
-// kStepsPerRefill traversal steps.  load(id, ray, nodes, tris) fetches ray `id` and the
-// BVH it is traced against; done(id, state, nvis, tvis) is called once per ray
-// with its finished state, also for invalid rays (which miss).  Every ray's
-// traversal is the one of traverse(), so results are identical.  All 64 lanes
-// of the wave must call it; no atomics (a wave's cursor is uniform and private).
-// Traversal steps between two refill checks: the check (a ballot and the ray
-// hand-out) costs as much as a light step.  C2 incoherent rays, Grays/s: 1 step
-// 3.21, 2: 3.33, 3: 3.37, 4: 3.35, 6: 3.31; the config-5 batch frame 15.6, 14.4,
-// 13.9, 13.6, 13.7 ms.
-constexpr int kStepsPerRefill = 4;
+// Waves of a persistent traversal kernel that reside on a CU: the LDS of the
+// stacks (a wave's take STACK x 512 B of the 160 KB), and at most the waves whose
+// VGPRs fit.
+__host__ __device__ constexpr int cu_waves(int stack) {
+    return stack <= 8 ? 32 : stack <= 10 ? 28 : stack <= 12 ? 24 : stack <= 16 ? 18 : stack <= 32 ? 8 : 4;
+}
+// Waves per block, which share one ray cursor: half a CU's, so that few rays are
+// left when a block's waves drain (1.24M bounce rays of 1.02M triangles: 12 waves
+// 221 us, 6: 233, 4: 243, 2: 250).  Batches take pairs: frames of several batches
+// on streams of their own share a CU with finer blocks (64 views, three batches
+// at once / alone: pairs 9.41 / 11.55 ms per frame, 4 waves 9.48 / 11.58, 12 waves
+// 10.24 / 11.13).
+__host__ __device__ constexpr int trace_waves(int stack) {
+    return stack <= 8 ? 16 : stack <= 10 ? 14 : stack <= 12 ? 12 : stack <= 16 ? 9 : stack <= 32 ? 4 : 2;
+}
+constexpr int kBatchWaves = 2;
+__host__ __device__ constexpr int trace_waves_per_simd(int stack) { return stack <= 12 ? cu_waves(stack) / 4 : 1; }
+
+// Calls f(integral_constant<int, STACK>) with the smallest stack variant that holds
+// `need` entries; false when none does.
+template <class F>
+bool with_stack(uint32_t need, F f) {
+    if (need <= 8)
+        f(std::integral_constant<int, 8>{});
+    else if (need <= 10)
+        f(std::integral_constant<int, 10>{});
+    else if (need <= 12)
+        f(std::integral_constant<int, 12>{});
+    else if (need <= 16)
+        f(std::integral_constant<int, 16>{});
+    else if (need <= 32)
+        f(std::integral_constant<int, 32>{});
+    else if (need <= 64)
+        f(std::integral_constant<int, 64>{});
+    else
+        return false;
+    return true;
+}
+
+// Grid of a persistent traversal launch with `waves_per_cu` waves on each of
+// `cus` CUs (capped by what resides), in blocks of w waves, for at most n rays:
+// not more blocks than groups of 8 rays.
+struct TraceGrid {
+    uint32_t blocks, threads;
+};
+inline TraceGrid trace_grid(int stack, int w, uint32_t waves_per_cu, uint32_t cus, uint32_t n) {
+    const uint32_t most = std::min((uint32_t)cu_waves(stack), std::max(1u, waves_per_cu));
+    // large blocks: two on a CU, narrower when fewer waves are asked for
+    const uint32_t waves = std::min((uint32_t)w, (most + 1) / 2);
+    const uint32_t per_cu = std::max(1u, most / waves);
+    return TraceGrid{std::min(cus * per_cu, std::max(1u, (n + 7) / 8)), waves * 64u};
+}
+
+// LDS of a persistent traversal block: each wave's stacks (entries 64 lanes
+// apart, so lanes at equal depth hit distinct banks) and the block's ray cursor.
+template <int STACK, int W = trace_waves(STACK)>
+struct TraceLds {
+    uint2 stk[STACK * 64 * W];
+    uint32_t cursor;
+    __device__ __forceinline__ uint2* lane_stack() {
+        return stk + (threadIdx.x >> 6) * (STACK * 64u) + (threadIdx.x & 63u);
+    }
+};
+
+constexpr uint32_t kSpreadWaves = 3;
+
+// Rays handed out by one block: of the rays [0, n), block b of nb owns the
+// 64-ray chunk b of every whole band of nb x 64 rays (so the blocks in flight
+// trace one band of neighbouring rays at a time and share its BVH nodes in L2)
+// and the [b rest / nb, (b + 1) rest / nb) slice of the last, partial band.
+struct RayShare {
+    uint32_t block, nblocks, full64, base, end;  // end: rays of this block
+    __device__ __forceinline__ RayShare(uint32_t n, uint32_t b, uint32_t nb) : block(b), nblocks(nb) {
+        const uint32_t band = nb * 64u, full = n / band;
+        base = full * band;
+        full64 = full * 64u;
+        const uint32_t rest = n - base;
+        const uint32_t lo = (uint32_t)(((uint64_t)b * rest) / nb);
+        end = full64 + (uint32_t)(((uint64_t)(b + 1u) * rest) / nb) - lo;
+        base += lo;
+    }
+    // the block's k-th ray
+    __device__ __forceinline__ uint32_t id(uint32_t k) const {
+        return k < full64 ? ((k >> 6) * nblocks + block) * 64u + (k & 63u) : base + (k - full64);
+    }
+    // Lanes of a wave that take rays: all of them, or, when the block's rays do not
+    // fill kSpreadWaves waves, an even part of them (at least 8): a small call then
+    // uses more SIMDs, and a wave waits for fewer rays.  Waves per block, 65k paths of
+    // a 256 x 256 room frame / 16k collision rays: 2: 455 / 33.6 us, 3: 457 / 35.7,
+    // 4: 471 / 32.9, 6: 500 / 31.4; one 64-ray chunk per wave over the chip 478 / 39.5.
+    __device__ __forceinline__ uint32_t lanes() const {
+        const uint32_t waves = min(kSpreadWaves, blockDim.x >> 6);
+        return min(64u, max(8u, (end + waves - 1u) / waves));
+    }
+};
 
 // Up to N traversal steps; true as soon as one finishes the ray.
-template <bool ANY, bool COUNT, int STACK, int N>
+template <bool COUNT, int N>
 __device__ __forceinline__ bool trav_steps(const uint4* __restrict__ nodes, const float4* __restrict__ tris,
-                                           TravState& st, uint2* stk, int stride, uint32_t& nvis, uint32_t& tvis) {
-    if (trav_step<ANY, COUNT, STACK>(nodes, tris, st, stk, stride, nvis, tvis)) return true;
-    if constexpr (N > 1) return trav_steps<ANY, COUNT, STACK, N - 1>(nodes, tris, st, stk, stride, nvis, tvis);
+                                           TravState& st, uint2* stk, int stride, bool any, uint32_t& nvis,
+                                           uint32_t& tvis) {
+    if (trav_step<COUNT>(nodes, tris, st, stk, stride, any, nvis, tvis)) return true;
+    if constexpr (N > 1) return trav_steps<COUNT, N - 1>(nodes, tris, st, stk, stride, any, nvis, tvis);
     return false;
 }
 
-// refill_trace with the refill threshold and the steps per check chosen at run
-// time / compile time (STEPS); refill_trace below fixes them.
-template <bool ANY, bool COUNT, int STACK, int STEPS, class Load, class Done>
-__device__ __forceinline__ void refill_trace_tuned(uint32_t n, uint32_t wave, uint32_t nwaves, uint2* stk, int stride,
-                                                   uint32_t refill, Load load, Done done) {
+// Persistent traversal with ray refill (after Aila & Laine 2009, "Understanding
+// the efficiency of ray traversal on GPUs").  The waves of a block take the
+// block's rays (RayShare) in order from one cursor in LDS, whenever at least
+// `refill` of a wave's lanes are idle (or all are), so a wave does not wait for
+// its slowest ray with the other lanes masked off, and the waves of a block end
+// together: with a fixed slice per wave, waves of the same launch were busy for
+// 76 to 257 us (161 on average; 1.24M bounce rays, 1.02M triangles), since a slice
+// of a few chunks does not average out.  Between two such checks a lane takes up
+// to STEPS traversal steps.  load(id, ray, nodes, tris) fetches ray `id` and the
+// BVH it is traced against; done(id, state, nvis, tvis) is called once per ray
+// with its finished state, also for invalid rays (which miss), when the wave
+// hands out rays again: the lanes that finished in between deliver together (a
+// call per finished lane ran the hit's stores and barycentrics at 1-3 of 64
+// lanes).  Every ray's traversal is the one of traverse(), so results are
+// identical.  All threads of the block must call it.
+template <bool ANY, bool COUNT, int STACK, int STEPS, int W, class Load, class Done>
+__device__ __forceinline__ void refill_trace(uint32_t n, TraceLds<STACK, W>& lds, uint32_t refill, Load load, Done done) {
+    const RayShare share(n, blockIdx.x, gridDim.x);
     const uint32_t lane = __lane_id();
     const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-    const uint32_t band = nwaves * 64u;
-    const uint32_t full = n / band;  // whole bands
-    const uint32_t base = full * band, rest = n - base;
-    const uint32_t lo = (uint32_t)(((uint64_t)wave * rest) / nwaves);
-    // this wave's rays, counted in its own order: 64 per whole band, then its slice
-    const uint32_t end = full * 64u + (uint32_t)(((uint64_t)(wave + 1u) * rest) / nwaves) - lo;
-    uint32_t cursor = 0;
-    bool active = false;
+    const uint32_t lanes = share.lanes();
+    const bool usable = lane < lanes;
+    if (lanes < 64u) refill = min(refill, lanes / 4u);
+    uint2* stk = lds.lane_stack();
+    if (threadIdx.x == 0) lds.cursor = 0u;
+    __syncthreads();
+    bool drained = false;
+    bool active = false, pending = false;  // pending: the lane's ray is finished, done() not yet called
     uint32_t id = 0, nv = 0, tv = 0;
     const uint4* nodes = nullptr;
     const float4* tris = nullptr;
     TravState st;
     while (true) {
-        const uint64_t idle = __ballot(!active);
+        const uint64_t idle = __ballot(usable && !active);
         const uint32_t nidle = (uint32_t)__popcll(idle);
-        if (nidle == 64u && cursor >= end) break;
-        if (cursor < end && (nidle >= refill || nidle == 64u)) {
-            if (!active) {
-                const uint32_t k = cursor + (uint32_t)__popcll(idle & below);
-                if (k < end) {
-                    id = k < full * 64u ? (wave + (k >> 6) * nwaves) * 64u + (k & 63u) : base + lo + (k - full * 64u);
+        if (nidle == lanes || (!drained && nidle >= refill)) {
+            if (pending) done(id, st, nv, tv);
+            if (drained) break;
+            uint32_t at = 0;
+            if (lane == 0) at = atomicAdd(&lds.cursor, nidle);
+            at = __builtin_amdgcn_readfirstlane(at);
+            if (usable && !active) {
+                pending = false;
+                const uint32_t k = at + (uint32_t)__popcll(idle & below);
+                if (k < share.end) {
+                    id = share.id(k);
                     Ray ray;
                     load(id, ray, nodes, tris);
                     nv = tv = 0;
                     active = trav_init(ray, st);
-                    if (!active) done(id, st, nv, tv);
+                    pending = !active;
                 }
             }
-            cursor += nidle;
+            drained = at + nidle >= share.end;
         }
-        if (active && trav_steps<ANY, COUNT, STACK, STEPS>(nodes, tris, st, stk, stride, nv, tv)) {
+        if (active && trav_steps<COUNT, STEPS>(nodes, tris, st, stk, 64, ANY, nv, tv)) {
             active = false;
-            done(id, st, nv, tv);
+            pending = true;
         }
     }
 }
 
-template <bool ANY, bool COUNT, int STACK, int REFILL, class Load, class Done>
-__device__ __forceinline__ void refill_trace(uint32_t n, uint32_t wave, uint32_t nwaves, uint2* stk, int stride,
-                                             Load load, Done done) {
-    refill_trace_tuned<ANY, COUNT, STACK, kStepsPerRefill>(n, wave, nwaves, stk, stride, (uint32_t)REFILL, load, done);
-}
+// Traversal steps between two refill checks where they are not tuned: the check
+// (a ballot and the ray hand-out) costs as much as a light step.  C2 incoherent
+// rays, Grays/s: 1 step 3.21, 2: 3.33, 3: 3.37, 4: 3.35, 6: 3.31; the config-5
+// batch frame 15.6, 14.4, 13.9, 13.6, 13.7 ms.
+constexpr int kStepsPerRefill = 4;
 
 // Barycentrics (u, v) of a leaf record hit; bary = (1-u-v, u, v).
-__device__ __forceinline__ void hit_uv(const float4* __restrict__ tris, uint32_t rec, const Ray& ray, float& u,
+__device__ __forceinline__ void hit_uv(const float4* __restrict__ tris, uint32_t rec, const RayPre& p, float& u,
                                        float& v) {
-    RayPre p = ray_setup(ray);
     const float4* tp = tris + (size_t)rec * kTriWords;
     float4 r0 = tp[0], r1 = tp[1], r2 = tp[2];
     float t, U, V, W, det;
     intersect_tri(p, r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w, r2.x, t, U, V, W, det);
     u = V / det;
     v = W / det;
+}
+__device__ __forceinline__ void hit_uv(const float4* __restrict__ tris, uint32_t rec, const Ray& ray, float& u,
+                                       float& v) {
+    hit_uv(tris, rec, ray_setup(ray), u, v);
 }
 
 // Block-level queue append: every thread of the block calls it (convergent:

@@ -19,8 +19,6 @@
 namespace snkpt {
 namespace {
 
-constexpr int kTraceBlock = 128;
-
 __global__ void k_trace_empty(uint32_t n, const uint32_t* __restrict__ count_dev, float* __restrict__ t_out,
                               uint32_t* __restrict__ inst_out, uint32_t* __restrict__ prim_out,
                               float* __restrict__ u_out, float* __restrict__ v_out, uint32_t* __restrict__ nvis_out,
@@ -37,24 +35,17 @@ __global__ void k_trace_empty(uint32_t n, const uint32_t* __restrict__ count_dev
     if (tvis_out) tvis_out[i] = 0;
 }
 
-// Persistent closest / any hit over the ray stream: each wave owns one 64-ray
-// chunk per band of the rays plus an even slice of the last band, and refills
-// its idle lanes from them (see refill_trace).  No atomics: a wave's cursor is
-// uniform and private to it.
+// Persistent closest / any hit over the ray stream (see refill_trace).
 template <bool ANY, bool COUNT, int STACK, int STEPS>
-__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(STACK <= 10 ? 8 : 1, 8))) void k_trace_refill(const float4* __restrict__ org_tmin,
-                                                              const float4* __restrict__ dir_tmax, uint32_t n,
-                                                              const uint32_t* __restrict__ count_dev,
-                                                              const uint4* __restrict__ nodes,
-                                                              const float4* __restrict__ tris,
-                                                              float* __restrict__ t_out, uint32_t* __restrict__ inst_out,
-                                                              uint32_t* __restrict__ prim_out, float* __restrict__ u_out,
-                                                              float* __restrict__ v_out, uint32_t* __restrict__ nvis_out,
-                                                              uint32_t* __restrict__ tvis_out, uint32_t refill) {
-    __shared__ uint2 stk[STACK * kTraceBlock];
+__global__ __launch_bounds__(64 * trace_waves(STACK))
+    __attribute__((amdgpu_waves_per_eu(trace_waves_per_simd(STACK), 8))) void k_trace_refill(
+        const float4* __restrict__ org_tmin, const float4* __restrict__ dir_tmax, uint32_t n,
+        const uint32_t* __restrict__ count_dev, const uint4* __restrict__ nodes, const float4* __restrict__ tris,
+        float* __restrict__ t_out, uint32_t* __restrict__ inst_out, uint32_t* __restrict__ prim_out,
+        float* __restrict__ u_out, float* __restrict__ v_out, uint32_t* __restrict__ nvis_out,
+        uint32_t* __restrict__ tvis_out, uint32_t refill) {
+    __shared__ TraceLds<STACK> lds;
     const uint32_t nn = count_dev ? *count_dev : n;
-    const uint32_t nwaves = gridDim.x * (kTraceBlock / 64);
-    const uint32_t wave = blockIdx.x * (kTraceBlock / 64) + (threadIdx.x >> 6);
     auto load = [&](uint32_t id, Ray& ray, const uint4*& nd, const float4*& tr) {
         float4 a = org_tmin[id], d = dir_tmax[id];
         ray = Ray{a.x, a.y, a.z, a.w, d.x, d.y, d.z, d.w};
@@ -69,10 +60,8 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(STA
             if (inst_out) inst_out[id] = __float_as_uint(r2.y);
             if (prim_out) prim_out[id] = __float_as_uint(r2.z);
             if (u_out || v_out) {
-                float4 a = org_tmin[id], d = dir_tmax[id];
-                Ray ray{a.x, a.y, a.z, a.w, d.x, d.y, d.z, d.w};
                 float u, v;
-                hit_uv(tris, res.rec, ray, u, v);
+                hit_uv(tris, res.rec, st.p, u, v);
                 if (u_out) u_out[id] = u;
                 if (v_out) v_out[id] = v;
             }
@@ -88,7 +77,7 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(STA
             if (tvis_out) tvis_out[id] = tv;
         }
     };
-    refill_trace_tuned<ANY, COUNT, STACK, STEPS>(nn, wave, nwaves, &stk[threadIdx.x], kTraceBlock, refill, load, done);
+    refill_trace<ANY, COUNT, STACK, STEPS>(nn, lds, refill, load, done);
 }
 
 // Hand-swept defaults (C2, 1.02M triangles): refill once 8 lanes are idle (4:
@@ -96,53 +85,31 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(STA
 // 3.15, 32: 3.09; coherent primary rays favour 8: 6.31 against 6.18 at 16), 4
 // steps between refill checks, all resident blocks.
 constexpr uint32_t kRefill = 8;
-// Resident 128-lane blocks per CU allowed by the 160 KB of LDS: a lane's stack
-// takes STACK x 8 B (10: 16 blocks, 12: 13, 16: 10, 32: 5, 64: 2).  The 10-entry
-// variant is held to 64 VGPRs so that 8 waves per SIMD fit (6 waves per SIMD
-// with 80 VGPRs: +3% on incoherent rays, -12% on primary rays).
-inline uint32_t refill_blocks_per_cu(uint32_t need) {
-    return need <= 10 ? 16u : need <= 12 ? 13u : need <= 16 ? 10u : need <= 32 ? 5u : 2u;
-}
-// Blocks per CU that give every SIMD the same number of waves (two waves per
-// block over four SIMDs: an even count): 13 blocks put 7 waves on two SIMDs and
-// 6 on the others, and ran the 12-entry variant 18 % slower than 12 blocks.
-inline uint32_t balanced_blocks(uint32_t b) { return b > 1u ? (b & ~1u) : 1u; }
 constexpr uint32_t kStepsDefault = 4;
-TraceShape default_shape(uint32_t need) {
-    return TraceShape{kRefill, kStepsDefault, balanced_blocks(refill_blocks_per_cu(need)), 0.0f};
+// blocks_per_cu counts pairs of waves per CU.  The most that reside: the LDS of
+// the stacks and the VGPR budget (trace_waves), two blocks of that many waves.
+uint32_t max_pairs(uint32_t need) {
+    uint32_t m = 2u;
+    with_stack(need, [&](auto s) { m = (uint32_t)cu_waves(decltype(s)::value) / 2u; });
+    return m;
 }
+TraceShape default_shape(uint32_t need) { return TraceShape{kRefill, kStepsDefault, max_pairs(need), 0.0f}; }
 
-template <bool ANY, bool COUNT, int STEPS>
-void launch_stack_steps(uint32_t stack, uint32_t g, uint32_t refill, hipStream_t st, const float4* o,
-                        const float4* d, uint32_t n, const uint32_t* cnt, const uint4* nodes, const float4* tris,
-                        const snkpt_hits& h, uint32_t* nv, uint32_t* tv) {
-#define K_LAUNCH(S)                                                                                          \
-    k_trace_refill<ANY, COUNT, S, STEPS><<<g, kTraceBlock, 0, st>>>(o, d, n, cnt, nodes, tris, h.t, h.inst, \
-                                                                     h.prim, h.u, h.v, nv, tv, refill)
-    if (stack <= 10)
-        K_LAUNCH(10);
-    else if (stack <= 12)
-        K_LAUNCH(12);
-    else if (stack <= 16)
-        K_LAUNCH(16);
-    else if (stack <= 32)
-        K_LAUNCH(32);
-    else
-        K_LAUNCH(64);
-#undef K_LAUNCH
-}
-
-// Persistent refill launch of the tuned shape (kind 0 closest hit, 1 any hit),
-// its grid capped by the (maximum) ray count.
+// Persistent refill launch of the tuned shape for at most n rays.
 template <bool ANY, bool COUNT>
-void launch_stack(const TraceShape& sh, uint32_t stack, uint32_t grid, uint32_t cus, hipStream_t st,
-                  const float4* o, const float4* d, uint32_t n, const uint32_t* cnt, const uint4* nodes,
-                  const float4* tris, const snkpt_hits& h, uint32_t* nv, uint32_t* tv) {
-    const uint32_t g = std::min(cus * std::max(1u, sh.blocks_per_cu), grid);
-    if (sh.steps == 3)
-        launch_stack_steps<ANY, COUNT, 3>(stack, g, sh.refill, st, o, d, n, cnt, nodes, tris, h, nv, tv);
-    else
-        launch_stack_steps<ANY, COUNT, 4>(stack, g, sh.refill, st, o, d, n, cnt, nodes, tris, h, nv, tv);
+void launch_stack(const TraceShape& sh, uint32_t need, uint32_t cus, hipStream_t st, const float4* o, const float4* d,
+                  uint32_t n, const uint32_t* cnt, const uint4* nodes, const float4* tris, const snkpt_hits& h,
+                  uint32_t* nv, uint32_t* tv) {
+    with_stack(need, [&](auto s) {
+        constexpr int S = decltype(s)::value;
+        const TraceGrid g = trace_grid(S, trace_waves(S), 2u * std::max(1u, sh.blocks_per_cu), cus, n);
+        if (sh.steps == 3)
+            k_trace_refill<ANY, COUNT, S, 3><<<g.blocks, g.threads, 0, st>>>(
+                o, d, n, cnt, nodes, tris, h.t, h.inst, h.prim, h.u, h.v, nv, tv, sh.refill);
+        else
+            k_trace_refill<ANY, COUNT, S, 4><<<g.blocks, g.threads, 0, st>>>(
+                o, d, n, cnt, nodes, tris, h.t, h.inst, h.prim, h.u, h.v, nv, tv, sh.refill);
+    });
 }
 
 // Rays of the autotuner's sample, like a path tracer's bounce rays: ray i
@@ -195,7 +162,8 @@ snkpt_status autotune_trace(snkpt_ctx* ctx, hipStream_t st) {
     if (!A.built || A.shape_fixed || A.num_tris == 0) return SNKPT_OK;
     const uint32_t need = A.depth > 0 ? A.depth - 1 : 0;
     if (need > 64) return SNKPT_OK;
-    const uint32_t stack = need <= 10 ? 10u : need <= 12 ? 12u : need <= 16 ? 16u : need <= 32 ? 32u : 64u;
+    uint32_t stack = 64u;
+    with_stack(need, [&](auto s) { stack = (uint32_t)decltype(s)::value; });
     uint32_t lg = 0;
     while ((1u << lg) < A.num_tris && lg < 31) ++lg;
     const auto key = std::make_tuple(ctx->device, stack, lg);
@@ -225,7 +193,7 @@ snkpt_status autotune_trace(snkpt_ctx* ctx, hipStream_t st) {
     }
     const snkpt_hits h{t.as<float>(), ids.as<uint32_t>(), ids.as<uint32_t>() + n, nullptr, nullptr};
     const uint32_t cus = ctx->props.multiProcessorCount > 0 ? (uint32_t)ctx->props.multiProcessorCount : 256u;
-    const uint32_t bmax = refill_blocks_per_cu(need);
+    const uint32_t bmax = max_pairs(need);
     TraceShape best[2];
     snkpt_status status = SNKPT_OK;
     for (int kind = 0; kind < 2 && status == SNKPT_OK; ++kind) {
@@ -233,19 +201,19 @@ snkpt_status autotune_trace(snkpt_ctx* ctx, hipStream_t st) {
         best[kind].ms = 1e30f;
         for (uint32_t refill : {4u, 8u, 16u})
             for (uint32_t steps : {3u, 4u})
-                for (uint32_t bpc = balanced_blocks(bmax); bpc >= std::max(1u, bmax / 2) && bpc >= 1u;
+                for (uint32_t bpc = bmax; bpc >= std::max(1u, bmax / 2) && bpc >= 1u;
                      bpc = bpc > 2u ? bpc - 2u : 0u) {
                     const TraceShape sh{refill, steps, bpc, 0.0f};
                     float ms = 1e30f;
                     for (int rep = 0; rep < 4; ++rep) {
                         (void)hipEventRecord(e0, st);
                         if (kind)
-                            launch_stack<true, false>(sh, need, (n + kTraceBlock - 1) / kTraceBlock, cus, st,
+                            launch_stack<true, false>(sh, need, cus, st,
                                                       org.as<float4>(), dir.as<float4>(), n, nullptr,
                                                       A.nodes.as<uint4>(), A.leaf_tris.as<float4>(), h, nullptr,
                                                       nullptr);
                         else
-                            launch_stack<false, false>(sh, need, (n + kTraceBlock - 1) / kTraceBlock, cus, st,
+                            launch_stack<false, false>(sh, need, cus, st,
                                                        org.as<float4>(), dir.as<float4>(), n, nullptr,
                                                        A.nodes.as<uint4>(), A.leaf_tris.as<float4>(), h, nullptr,
                                                        nullptr);
@@ -282,7 +250,6 @@ snkpt_status launch_trace(snkpt_ctx* ctx, const float4* org_tmin, const float4* 
     if (!A.built) return fail(ctx, SNKPT_ERR_NOT_BUILT, "trace: acceleration structure not built");
     if (n == 0) return SNKPT_OK;
     if (!org_tmin || !dir_tmax || !hits.t) return fail(ctx, SNKPT_ERR_INVALID_ARG, "trace: null ray or hit stream");
-    uint32_t grid = (n + kTraceBlock - 1) / kTraceBlock;
     if (A.num_tris == 0) {
         k_trace_empty<<<(n + 255) / 256, 256, 0, st>>>(n, count_dev, hits.t, hits.inst, hits.prim, hits.u, hits.v,
                                                        node_visits, tri_visits);
@@ -296,17 +263,17 @@ snkpt_status launch_trace(snkpt_ctx* ctx, const float4* org_tmin, const float4* 
         const float4* tris = A.leaf_tris.as<float4>();
         if (any_hit) {
             if (count)
-                launch_stack<true, true>(sh, need, grid, cus, st, org_tmin, dir_tmax, n, count_dev, nodes, tris, hits,
+                launch_stack<true, true>(sh, need, cus, st, org_tmin, dir_tmax, n, count_dev, nodes, tris, hits,
                                          node_visits, tri_visits);
             else
-                launch_stack<true, false>(sh, need, grid, cus, st, org_tmin, dir_tmax, n, count_dev, nodes, tris,
+                launch_stack<true, false>(sh, need, cus, st, org_tmin, dir_tmax, n, count_dev, nodes, tris,
                                           hits, nullptr, nullptr);
         } else {
             if (count)
-                launch_stack<false, true>(sh, need, grid, cus, st, org_tmin, dir_tmax, n, count_dev, nodes, tris,
+                launch_stack<false, true>(sh, need, cus, st, org_tmin, dir_tmax, n, count_dev, nodes, tris,
                                           hits, node_visits, tri_visits);
             else
-                launch_stack<false, false>(sh, need, grid, cus, st, org_tmin, dir_tmax, n, count_dev, nodes, tris,
+                launch_stack<false, false>(sh, need, cus, st, org_tmin, dir_tmax, n, count_dev, nodes, tris,
                                            hits, nullptr, nullptr);
         }
     }
