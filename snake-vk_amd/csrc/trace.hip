@@ -15,6 +15,7 @@
 #include "shading.h"
 #include "snkpt_dev.h"
 #include "snkpt_host.h"
+#include "trace_group.h"
 
 namespace snkpt {
 namespace {
@@ -35,6 +36,32 @@ __global__ void k_trace_empty(uint32_t n, const uint32_t* __restrict__ count_dev
     if (tvis_out) tvis_out[i] = 0;
 }
 
+// Writes ray id's hit (or miss) to the caller's arrays.
+__device__ __forceinline__ void write_hit(const TravState& st, const float4* __restrict__ tris, uint32_t id,
+                                          float* __restrict__ t_out, uint32_t* __restrict__ inst_out,
+                                          uint32_t* __restrict__ prim_out, float* __restrict__ u_out,
+                                          float* __restrict__ v_out) {
+    const TraceResult& res = st.res;
+    if (res.rec != 0xFFFFFFFFu) {
+        float4 r2 = tris[(size_t)res.rec * kTriWords + 2];
+        t_out[id] = res.t;
+        if (inst_out) inst_out[id] = __float_as_uint(r2.y);
+        if (prim_out) prim_out[id] = __float_as_uint(r2.z);
+        if (u_out || v_out) {
+            float u, v;
+            hit_uv(tris, res.rec, st.p, u, v);
+            if (u_out) u_out[id] = u;
+            if (v_out) v_out[id] = v;
+        }
+    } else {
+        t_out[id] = -1.0f;
+        if (inst_out) inst_out[id] = 0xFFFFFFFFu;
+        if (prim_out) prim_out[id] = 0xFFFFFFFFu;
+        if (u_out) u_out[id] = 0.0f;
+        if (v_out) v_out[id] = 0.0f;
+    }
+}
+
 // Persistent closest / any hit over the ray stream (see refill_trace).
 template <bool ANY, bool COUNT, int STACK, int STEPS>
 __global__ __launch_bounds__(64 * trace_waves(STACK))
@@ -53,31 +80,33 @@ __global__ __launch_bounds__(64 * trace_waves(STACK))
         tr = tris;
     };
     auto done = [&](uint32_t id, const TravState& st, uint32_t nv, uint32_t tv) {
-        const TraceResult& res = st.res;
-        if (res.rec != 0xFFFFFFFFu) {
-            float4 r2 = tris[(size_t)res.rec * kTriWords + 2];
-            t_out[id] = res.t;
-            if (inst_out) inst_out[id] = __float_as_uint(r2.y);
-            if (prim_out) prim_out[id] = __float_as_uint(r2.z);
-            if (u_out || v_out) {
-                float u, v;
-                hit_uv(tris, res.rec, st.p, u, v);
-                if (u_out) u_out[id] = u;
-                if (v_out) v_out[id] = v;
-            }
-        } else {
-            t_out[id] = -1.0f;
-            if (inst_out) inst_out[id] = 0xFFFFFFFFu;
-            if (prim_out) prim_out[id] = 0xFFFFFFFFu;
-            if (u_out) u_out[id] = 0.0f;
-            if (v_out) v_out[id] = 0.0f;
-        }
+        write_hit(st, tris, id, t_out, inst_out, prim_out, u_out, v_out);
         if (COUNT) {
             if (nvis_out) nvis_out[id] = nv;
             if (tvis_out) tvis_out[id] = tv;
         }
     };
     refill_trace<ANY, COUNT, STACK, STEPS>(nn, lds, refill, load, done);
+}
+
+// The same with eight lanes per ray, for small calls (see group_trace).
+template <bool ANY, int STACK>
+__global__ __launch_bounds__(64 * kGroupWaves) void k_trace_group(
+    const float4* __restrict__ org_tmin, const float4* __restrict__ dir_tmax, uint32_t n,
+    const uint32_t* __restrict__ count_dev, const uint4* __restrict__ nodes, const float4* __restrict__ tris,
+    float* __restrict__ t_out, uint32_t* __restrict__ inst_out, uint32_t* __restrict__ prim_out,
+    float* __restrict__ u_out, float* __restrict__ v_out) {
+    __shared__ GroupLds<STACK> lds;
+    auto load = [&](uint32_t id, Ray& ray, const uint4*& nd, const float4*& tr) {
+        float4 a = org_tmin[id], d = dir_tmax[id];
+        ray = Ray{a.x, a.y, a.z, a.w, d.x, d.y, d.z, d.w};
+        nd = nodes;
+        tr = tris;
+    };
+    auto done = [&](uint32_t id, const TravState& st) {
+        write_hit(st, tris, id, t_out, inst_out, prim_out, u_out, v_out);
+    };
+    group_trace<ANY, STACK>(count_dev ? *count_dev : n, lds, load, done);
 }
 
 // Hand-swept defaults (C2, 1.02M triangles): refill once 8 lanes are idle (4:
@@ -257,6 +286,22 @@ snkpt_status launch_trace(snkpt_ctx* ctx, const float4* org_tmin, const float4* 
         uint32_t need = A.depth > 0 ? A.depth - 1 : 0;
         if (need > 64) return fail(ctx, SNKPT_ERR_CAPACITY, "trace: BVH8 deeper than the 64-entry traversal stack");
         bool count = node_visits || tri_visits;
+        if (!count && n <= kGroupRays) {
+            with_stack(need, [&](auto s) {
+                constexpr int S = decltype(s)::value;
+                const TraceGrid g = group_grid(kGroupCuWaves, ctx->props.multiProcessorCount > 0 ? (uint32_t)ctx->props.multiProcessorCount : 256u, n);
+                if (any_hit)
+                    k_trace_group<true, S><<<g.blocks, g.threads, 0, st>>>(
+                        org_tmin, dir_tmax, n, count_dev, A.nodes.as<uint4>(), A.leaf_tris.as<float4>(), hits.t,
+                        hits.inst, hits.prim, hits.u, hits.v);
+                else
+                    k_trace_group<false, S><<<g.blocks, g.threads, 0, st>>>(
+                        org_tmin, dir_tmax, n, count_dev, A.nodes.as<uint4>(), A.leaf_tris.as<float4>(), hits.t,
+                        hits.inst, hits.prim, hits.u, hits.v);
+            });
+            hipError_t e = hipGetLastError();
+            return e == hipSuccess ? SNKPT_OK : hip_fail(ctx, e, "trace launch");
+        }
         const uint32_t cus = ctx->props.multiProcessorCount > 0 ? (uint32_t)ctx->props.multiProcessorCount : 256u;
         const TraceShape sh = A.shape[any_hit ? 1 : 0].refill ? A.shape[any_hit ? 1 : 0] : default_shape(need);
         const uint4* nodes = A.nodes.as<uint4>();
