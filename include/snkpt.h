@@ -164,8 +164,7 @@ typedef struct snkpt_settings {
     uint32_t tail_bounce;           /* SNKPT_MODE_PT (and the path-traced bounces of ReSTIR and G-buffer frames):
                                        bounce from which the paths still alive run one thread per path instead of one
                                        launch per bounce; same radiance bit for bit.  0 = chosen from the context's
-                                       previous frame (the first bounce whose queue of paths fits twice the resident
-                                       lanes); >= max_depth = never */
+                                       previous frame (the first bounce with at most 2^22 queued paths); >= max_depth = never */
     uint32_t reserved[1];
 } snkpt_settings;
 

@@ -154,17 +154,13 @@ __global__ __launch_bounds__(64 * kBatchWaves)
     refill_trace<false, false, STACK, kStepsPerRefill>(n, lds, kRefillLanes, load, done);
 }
 
-// The late bounces of the batch, one thread per path (tail_paths).
-constexpr int kBTailBlock = 128;
-constexpr uint32_t kBTailBlocksPerCu = 8;
+// The late bounces of the batch (tail_paths).
 template <int STACK>
-__global__ __launch_bounds__(kBTailBlock) void k_btail(SceneMany ss, PtParams P, Queue in,
-                                                       const uint32_t* __restrict__ count, PathState ps,
-                                                       float4* __restrict__ rad,
-                                                       unsigned long long* __restrict__ stats) {
-    __shared__ uint2 stk[STACK * kBTailBlock];
-    __shared__ uint32_t red[2];
-    tail_paths<STACK, kBTailBlock>(ss, P, ShadeHooks{}, in, *count, ps, rad, &stk[threadIdx.x], stats, red);
+__global__ __launch_bounds__(64 * tail_waves(STACK)) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_btail(
+    SceneMany ss, PtParams P, Queue in, const uint32_t* __restrict__ count, PathState ps, float4* __restrict__ rad,
+    unsigned long long* __restrict__ stats) {
+    __shared__ TailLds<STACK> lds;
+    tail_paths<STACK>(ss, P, ShadeHooks{}, in, *count, ps, rad, lds, stats);
 }
 
 template <int KIND>
@@ -553,18 +549,14 @@ void launch_traces(snkpt_batch* B, const SceneMany& ss, int cur, hipStream_t st,
 void launch_btail(snkpt_batch* B, const SceneMany& ss, const PtParams& P, int cur, hipStream_t st) {
     Queue qin{B->q_org[cur].as<float4>(), B->q_dir[cur].as<float4>(), B->q_path[cur].as<uint32_t>()};
     PathState ps{B->p_thr.as<float4>(), B->p_rng.as<uint2>(), B->p_bounce.as<uint32_t>()};
-    const uint32_t grid = (uint32_t)B->cus * kBTailBlocksPerCu;
     const uint32_t* count = B->counts.as<uint32_t>() + cur;
     float4* rad = B->rad.as<float4>();
     unsigned long long* stats = B->stats.as<unsigned long long>();
-    if (B->stack <= 10)
-        k_btail<10><<<grid, kBTailBlock, 0, st>>>(ss, P, qin, count, ps, rad, stats);
-    else if (B->stack <= 16)
-        k_btail<16><<<grid, kBTailBlock, 0, st>>>(ss, P, qin, count, ps, rad, stats);
-    else if (B->stack <= 32)
-        k_btail<32><<<grid, kBTailBlock, 0, st>>>(ss, P, qin, count, ps, rad, stats);
-    else
-        k_btail<64><<<grid, kBTailBlock, 0, st>>>(ss, P, qin, count, ps, rad, stats);
+    with_stack(B->stack, [&](auto s) {
+        constexpr int S = decltype(s)::value;
+        const TraceGrid g = tail_grid(S, (uint32_t)B->cus, B->cap);
+        k_btail<S><<<g.blocks, g.threads, 0, st>>>(ss, P, qin, count, ps, rad, stats);
+    });
 }
 
 // Bounce of the plain batch frame from which the tail runs (0: never).

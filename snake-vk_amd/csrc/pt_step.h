@@ -4,6 +4,7 @@
 
 #include "render_modes.h"
 #include "snkpt_dev.h"
+#include "trace_group.h"
 
 namespace snkpt {
 
@@ -227,41 +228,285 @@ __device__ __forceinline__ float4 path_rest(const SceneDev& S, const PtParams& P
     return L;
 }
 
-// The late bounces, one thread per path: every path queued in `in` (n of them)
-// runs to its end in place, from its stored throughput, random stream and
-// bounce.  After Russian roulette has thinned the queue, a launch per bounce
-// leaves most lanes idle; here a lane that ends its path takes the next one.
-// path_rest adds the contributions in the wavefront's order, so the radiance is
-// bit-identical.  The first ray of each entry was counted when it was queued;
-// stats[1] / stats[2] get the rest (red: two words of LDS).
-template <int STACK, int BLOCK, class SS>
+// The path kernel below: four waves per SIMD (the shading needs up to 128 VGPRs),
+// fewer where the stacks' LDS is short.
+__host__ __device__ constexpr int tail_waves(int stack) { return cu_waves(stack) < 16 ? cu_waves(stack) / 2 : 8; }
+template <int STACK>
+struct TailLds {
+    uint2 stk[STACK * 64 * tail_waves(STACK)];
+    uint32_t cursor, n_ext, n_sh;
+};
+inline TraceGrid tail_grid(int stack, uint32_t cus, uint32_t n) {
+    return TraceGrid{std::min(cus * 2u, std::max(1u, (n + 7) / 8)), (uint32_t)tail_waves(stack) * 64u};
+}
+// Lanes of a wave with a hit to shade at which the wave stops traversing and shades
+// them: it costs about as much as three traversal steps, whatever the number of
+// lanes.  A quarter of the lanes where a lane sees few paths (frames of 1.02M
+// triangles and of the room at 1080p, tail from bounce 1, 16 / 32 lanes: 1.597 /
+// 1.595 and 0.986 / 0.961 ms; room at 256 x 256 and 400 x 300: 356 / 370 and 394 /
+// 409 us).  Lanes that only need their next ray started (a settled shadow ray, a
+// path from the queue) are served from an eighth of the lanes on: waiting for the
+// shading with them took 395 us on the 256 x 256 frame, 0.99 ms on the 1080p room.
+constexpr uint32_t kServeLanes = 32;
+// Groups waiting for any service at which a wave of eight-lane groups serves them.
+constexpr uint32_t kServeGroups = 2;
+
+// The late bounces of every path queued in `in` (n of them), each from its stored
+// throughput, random stream and bounce to its end.  After Russian roulette has
+// thinned the queue, a launch per bounce leaves most lanes idle; here a lane
+// carries one path and all lanes of a wave traverse together, extension rays
+// beside shadow rays.  A lane whose ray is finished waits until enough lanes do;
+// then the wave shades their hits, settles their shadow rays, hands out the
+// next queued paths to lanes whose path ended, and traverses on.  (Running each
+// path's trace, shade and shadow in its own loop had 8.5 of 64 lanes active per
+// VALU instruction: 774 us for the 367k paths of the 1.02M-triangle frame.)
+// What a path holds between rays stays in its queue slot and path state
+// (in.org / in.dir: its next ray; ps: throughput and random stream), so the
+// traversal loop keeps few registers.  Contributions are added to rad[path] in
+// the wavefront's order (emission, then the unoccluded shadow ray, vertex by
+// vertex), so the radiance is bit-identical.  The first ray of each entry was
+// counted when it was queued; stats[1] / stats[2] get the rest.
+template <int STACK, class SS>
 __device__ __forceinline__ void tail_paths(const SS& ss, const PtParams& P, const ShadeHooks& H, const Queue& in,
-                                           uint32_t n, const PathState& ps, float4* __restrict__ rad, uint2* stk,
-                                           unsigned long long* __restrict__ stats, uint32_t* red) {
-    if (threadIdx.x == 0) red[0] = red[1] = 0u;
+                                           uint32_t n, const PathState& ps, float4* __restrict__ rad,
+                                           TailLds<STACK>& lds, unsigned long long* __restrict__ stats) {
+    enum { kNone = 0u, kExt = 1u, kShadow = 2u, kShadowThenExt = 3u };
+    const RayShare share(n, blockIdx.x, gridDim.x);
+    const uint32_t lane = __lane_id();
+    const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    const uint32_t lanes = share.lanes();
+    const bool usable = lane < lanes;
+    const uint32_t serve = share.end > 2u * blockDim.x ? kServeLanes : max(1u, lanes / 4u);
+    const uint32_t restart = max(1u, lanes / 8u);
+    uint2* stk = lds.stk + (threadIdx.x >> 6) * (STACK * 64u) + lane;
+    if (threadIdx.x == 0) lds.cursor = lds.n_ext = lds.n_sh = 0u;
     __syncthreads();
-    uint32_t n_ext = 0, n_sh = 0;
-    for (uint32_t i = blockIdx.x * BLOCK + threadIdx.x; i < n; i += gridDim.x * BLOCK) {
-        const uint32_t path = in.path[i];
-        const float4 o = in.org[i], d = in.dir[i];
-        const uint2 rs = ps.rng[path];
-        const Rng rng{(uint64_t)rs.x | ((uint64_t)rs.y << 32), ((uint64_t)ss.stream(path) << 1u) | 1u};
-        rad[path] = path_rest<0, STACK>(ss.at(path), P, H, path, ps.bounce[path],
-                                        Ray{o.x, o.y, o.z, o.w, d.x, d.y, d.z, d.w}, ps.thr[path], rng, stk, BLOCK,
-                                        rad[path], n_ext, n_sh);
+    uint32_t n_ext = 0, n_sh = 0, nv = 0, tv = 0;
+    uint32_t what = kNone, slot = 0, path = 0, bounce = 0;
+    bool active = false, drained = false;
+    V3 sh_c{0.0f, 0.0f, 0.0f};
+    const uint4* nodes = nullptr;
+    const float4* tris = nullptr;
+    TravState st;
+    while (true) {
+        const bool none = __ballot(active) == 0ull;
+        const bool shade = none || (uint32_t)__popcll(__ballot(!active && what == kExt)) >= serve;
+        const bool light = shade || (uint32_t)__popcll(__ballot(usable && !active && what != kExt &&
+                                                                 !(drained && what == kNone))) >= restart;
+        if (light) {
+            Ray r;
+            bool start = false;
+            if (!active && what >= kShadow) {
+                if (st.res.rec == 0xFFFFFFFFu) {
+                    const float4 L = rad[path];
+                    rad[path] = make_float4(L.x + sh_c.x, L.y + sh_c.y, L.z + sh_c.z, L.w);
+                }
+                start = what == kShadowThenExt;
+                what = start ? kExt : kNone;
+                if (start) {
+                    const float4 o = in.org[slot], d = in.dir[slot];
+                    r = Ray{o.x, o.y, o.z, o.w, d.x, d.y, d.z, d.w};
+                }
+            } else if (shade && !active && what == kExt) {
+                what = kNone;
+                if (st.res.rec != 0xFFFFFFFFu) {
+                    const SceneDev& S = ss.at(path);
+                    const float4 r2 = S.leaf[(size_t)st.res.rec * kTriWords + 2];
+                    float hu, hv;
+                    hit_uv(S.leaf, st.res.rec, st.p, hu, hv);
+                    const float4 d = in.dir[slot];
+                    const uint2 rs = ps.rng[path];
+                    Rng rng{(uint64_t)rs.x | ((uint64_t)rs.y << 32), ((uint64_t)ss.stream(path) << 1u) | 1u};
+                    VertexOut o;
+                    path_vertex<0>(S, P, H, path, bounce, V3{d.x, d.y, d.z}, st.res.t, __float_as_uint(r2.y),
+                                   __float_as_uint(r2.z), hu, hv, ps.thr[path], rng, make_float4(0.0f, 0.0f, 0.0f, 0.0f),
+                                   o);
+                    if (o.emit) {
+                        const float4 L = rad[path];
+                        rad[path] = make_float4(L.x + o.c_emit.x, L.y + o.c_emit.y, L.z + o.c_emit.z, L.w);
+                    }
+                    if (o.ext) {
+                        ++n_ext;
+                        ++bounce;
+                        in.org[slot] = make_float4(o.ext_o.x, o.ext_o.y, o.ext_o.z, 0.0f);
+                        in.dir[slot] = make_float4(o.ext_d.x, o.ext_d.y, o.ext_d.z, 1e30f);
+                        ps.thr[path] = o.thr4;
+                        ps.rng[path] = make_uint2((uint32_t)rng.state, (uint32_t)(rng.state >> 32));
+                        r = Ray{o.ext_o.x, o.ext_o.y, o.ext_o.z, 0.0f, o.ext_d.x, o.ext_d.y, o.ext_d.z, 1e30f};
+                        what = kExt;
+                    }
+                    if (o.sh) {
+                        ++n_sh;
+                        sh_c = o.sh_c;
+                        r = Ray{o.sh_o.x, o.sh_o.y, o.sh_o.z, 0.0f, o.sh_d.x, o.sh_d.y, o.sh_d.z, o.sh_t};
+                        what = o.ext ? kShadowThenExt : kShadow;
+                    }
+                    start = what != kNone;
+                }
+            }
+            if (!drained) {
+                const uint64_t free = __ballot(usable && !active && what == kNone);
+                const uint32_t nfree = (uint32_t)__popcll(free);
+                uint32_t at = 0;
+                if (lane == 0) at = atomicAdd(&lds.cursor, nfree);
+                at = __builtin_amdgcn_readfirstlane(at);
+                const uint32_t k = at + (uint32_t)__popcll(free & below);
+                if (usable && !active && what == kNone && k < share.end) {
+                    slot = share.id(k);
+                    path = in.path[slot];
+                    bounce = ps.bounce[path];
+                    const float4 o = in.org[slot], d = in.dir[slot];
+                    r = Ray{o.x, o.y, o.z, o.w, d.x, d.y, d.z, d.w};
+                    const SceneDev& S = ss.at(path);
+                    nodes = S.nodes;
+                    tris = S.leaf;
+                    what = kExt;
+                    start = true;
+                }
+                drained = at + nfree >= share.end;
+            }
+            if (start) active = trav_init(r, st);
+            if (drained && __ballot(what != kNone) == 0ull) break;
+        }
+        if (active && trav_steps<false, kStepsPerRefill>(nodes, tris, st, stk, 64, what >= kShadow, nv, tv))
+            active = false;
     }
     for (int o = 32; o > 0; o >>= 1) {
         n_ext += __shfl_xor(n_ext, o, 64);
         n_sh += __shfl_xor(n_sh, o, 64);
     }
-    if ((threadIdx.x & 63) == 0) {
-        atomicAdd(&red[0], n_ext);
-        atomicAdd(&red[1], n_sh);
+    if (lane == 0) {
+        atomicAdd(&lds.n_ext, n_ext);
+        atomicAdd(&lds.n_sh, n_sh);
     }
     __syncthreads();
-    if (threadIdx.x == 0 && (red[0] | red[1])) {
-        atomicAdd(&stats[1], (unsigned long long)red[0]);
-        atomicAdd(&stats[2], (unsigned long long)red[1]);
+    if (threadIdx.x == 0 && (lds.n_ext | lds.n_sh)) {
+        atomicAdd(&stats[1], (unsigned long long)lds.n_ext);
+        atomicAdd(&stats[2], (unsigned long long)lds.n_sh);
+    }
+}
+
+// tail_paths with eight lanes per path (trace_group.h), for small queues: a path's
+// rays are traced by its group, its vertices shaded by every lane of the group
+// alike; one lane adds to the radiance and counts.  Same order of contributions.
+template <int STACK, class SS>
+__device__ __forceinline__ void tail_paths_group(const SS& ss, const PtParams& P, const ShadeHooks& H, const Queue& in,
+                                                 uint32_t n, const PathState& ps, float4* __restrict__ rad,
+                                                 GroupLds<STACK>& lds, unsigned long long* __restrict__ stats) {
+    enum { kNone = 0u, kExt = 1u, kShadow = 2u, kShadowThenExt = 3u };
+    const RayShare share(n, blockIdx.x, gridDim.x);
+    const uint32_t lane = __lane_id(), group = lane >> 3;
+    const bool first = (lane & 7u) == 0u;
+    const uint32_t groups = min(8u, max(1u, (share.end + kGroupWaves - 1u) / kGroupWaves));
+    const bool usable = group < groups;
+    const uint64_t below = (1ull << (group * 8u)) - 1ull;
+    uint2* stk = lds.group_stack();
+    if (threadIdx.x == 0) lds.cursor = lds.n_ext = lds.n_sh = 0u;
+    __syncthreads();
+    uint32_t n_ext = 0, n_sh = 0;
+    uint32_t what = kNone, slot = 0, path = 0, bounce = 0;
+    bool active = false, drained = false;
+    V3 sh_c{0.0f, 0.0f, 0.0f};
+    const uint4* nodes = nullptr;
+    const float4* tris = nullptr;
+    TravState st;
+    while (true) {
+        const uint32_t waiting = (uint32_t)__popcll(__ballot(usable && !active && !(drained && what == kNone))) >> 3;
+        const bool none = __ballot(active) == 0ull;
+        if (none || waiting >= kServeGroups) {
+            Ray r;
+            bool start = false;
+            if (!active && what >= kShadow) {
+                if (first && st.res.rec == 0xFFFFFFFFu) {
+                    const float4 L = rad[path];
+                    rad[path] = make_float4(L.x + sh_c.x, L.y + sh_c.y, L.z + sh_c.z, L.w);
+                }
+                start = what == kShadowThenExt;
+                what = start ? kExt : kNone;
+                if (start) {
+                    const float4 o = in.org[slot], d = in.dir[slot];
+                    r = Ray{o.x, o.y, o.z, o.w, d.x, d.y, d.z, d.w};
+                }
+            } else if (!active && what == kExt) {
+                what = kNone;
+                if (st.res.rec != 0xFFFFFFFFu) {
+                    const SceneDev& S = ss.at(path);
+                    const float4 r2 = S.leaf[(size_t)st.res.rec * kTriWords + 2];
+                    float hu, hv;
+                    hit_uv(S.leaf, st.res.rec, st.p, hu, hv);
+                    const float4 d = in.dir[slot];
+                    const uint2 rs = ps.rng[path];
+                    Rng rng{(uint64_t)rs.x | ((uint64_t)rs.y << 32), ((uint64_t)ss.stream(path) << 1u) | 1u};
+                    VertexOut o;
+                    path_vertex<0>(S, P, H, path, bounce, V3{d.x, d.y, d.z}, st.res.t, __float_as_uint(r2.y),
+                                   __float_as_uint(r2.z), hu, hv, ps.thr[path], rng, make_float4(0.0f, 0.0f, 0.0f, 0.0f),
+                                   o);
+                    if (first && o.emit) {
+                        const float4 L = rad[path];
+                        rad[path] = make_float4(L.x + o.c_emit.x, L.y + o.c_emit.y, L.z + o.c_emit.z, L.w);
+                    }
+                    if (o.ext) {  // every lane stores the same values, so each reads back its own
+                        if (first) ++n_ext;
+                        ++bounce;
+                        in.org[slot] = make_float4(o.ext_o.x, o.ext_o.y, o.ext_o.z, 0.0f);
+                        in.dir[slot] = make_float4(o.ext_d.x, o.ext_d.y, o.ext_d.z, 1e30f);
+                        ps.thr[path] = o.thr4;
+                        ps.rng[path] = make_uint2((uint32_t)rng.state, (uint32_t)(rng.state >> 32));
+                        r = Ray{o.ext_o.x, o.ext_o.y, o.ext_o.z, 0.0f, o.ext_d.x, o.ext_d.y, o.ext_d.z, 1e30f};
+                        what = kExt;
+                    }
+                    if (o.sh) {
+                        if (first) ++n_sh;
+                        sh_c = o.sh_c;
+                        r = Ray{o.sh_o.x, o.sh_o.y, o.sh_o.z, 0.0f, o.sh_d.x, o.sh_d.y, o.sh_d.z, o.sh_t};
+                        what = o.ext ? kShadowThenExt : kShadow;
+                    }
+                    start = what != kNone;
+                }
+            }
+            if (!drained) {
+                const uint64_t free = __ballot(usable && !active && what == kNone);
+                const uint32_t nfree = (uint32_t)__popcll(free) >> 3;
+                uint32_t at = 0;
+                if (lane == 0) at = atomicAdd(&lds.cursor, nfree);
+                at = __builtin_amdgcn_readfirstlane(at);
+                const uint32_t j = at + ((uint32_t)__popcll(free & below) >> 3);
+                if (usable && !active && what == kNone && j < share.end) {
+                    slot = share.id(j);
+                    path = in.path[slot];
+                    bounce = ps.bounce[path];
+                    const float4 o = in.org[slot], d = in.dir[slot];
+                    r = Ray{o.x, o.y, o.z, o.w, d.x, d.y, d.z, d.w};
+                    const SceneDev& S = ss.at(path);
+                    nodes = S.nodes;
+                    tris = S.leaf;
+                    what = kExt;
+                    start = true;
+                }
+                drained = at + nfree >= share.end;
+            }
+            if (start) active = trav_init(r, st);
+            if (drained && __ballot(what != kNone) == 0ull) break;
+        }
+        if (active) {
+            const bool any = what >= kShadow;
+            bool fin = group_step(nodes, tris, st, stk, any);
+            if (!fin) fin = group_step(nodes, tris, st, stk, any);
+            if (fin) active = false;
+        }
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        n_ext += __shfl_xor(n_ext, o, 64);
+        n_sh += __shfl_xor(n_sh, o, 64);
+    }
+    if (lane == 0) {
+        atomicAdd(&lds.n_ext, n_ext);
+        atomicAdd(&lds.n_sh, n_sh);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && (lds.n_ext | lds.n_sh)) {
+        atomicAdd(&stats[1], (unsigned long long)lds.n_ext);
+        atomicAdd(&stats[2], (unsigned long long)lds.n_sh);
     }
 }
 

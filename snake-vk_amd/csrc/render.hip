@@ -24,6 +24,7 @@
 #include "render_common.h"
 #include "pt_step.h"
 #include "render_modes.h"
+#include "trace_group.h"
 
 namespace snkpt {
 
@@ -173,6 +174,24 @@ __global__ __launch_bounds__(64 * trace_waves(STACK))
     refill_trace<true, false, STACK, kStepsPerRefill>(nn, lds, kRefillLanes, load, done);
 }
 
+// The same with eight lanes per ray, for small queues (see group_trace).
+template <int STACK>
+__global__ __launch_bounds__(64 * kGroupWaves) void k_shadow_group(const uint4* __restrict__ nodes,
+                                                                   const float4* __restrict__ tris, ShadowQueue sq,
+                                                                   const uint32_t* __restrict__ counts,
+                                                                   float4* __restrict__ rad) {
+    __shared__ GroupLds<STACK> lds;
+    auto load = [&](uint32_t i, Ray& ray, const uint4*& nd, const float4*& tr) {
+        ray = shadow_ray(sq, i);
+        nd = nodes;
+        tr = tris;
+    };
+    auto done = [&](uint32_t i, const TravState& st) {
+        if ((__lane_id() & 7u) == 0u) shadow_done(sq, i, st.res, rad);
+    };
+    group_trace<true, STACK>(counts[2], lds, load, done);
+}
+
 // Whole paths, one per thread (KIND 0: radiance into rad[i]; KIND 2: training
 // records as the wavefront's kind-2 shade).  Ray counts: one atomic per block.
 constexpr int kMegaBlock = 128;
@@ -210,15 +229,21 @@ __global__ __launch_bounds__(kMegaBlock) void k_pt_mega(SceneDev S, CamDev cam, 
     }
 }
 
-// The late bounces of the plain path tracer, one thread per path (tail_paths).
+// The late bounces of the plain path tracer (tail_paths).
 template <int STACK>
-__global__ __launch_bounds__(kMegaBlock) void k_pt_tail(SceneDev S, PtParams P, ShadeHooks H, Queue in,
-                                                        const uint32_t* __restrict__ count, PathState ps,
-                                                        float4* __restrict__ rad,
-                                                        unsigned long long* __restrict__ stats) {
-    __shared__ uint2 stk[STACK * kMegaBlock];
-    __shared__ uint32_t red[2];
-    tail_paths<STACK, kMegaBlock>(SceneOne{S}, P, H, in, *count, ps, rad, &stk[threadIdx.x], stats, red);
+__global__ __launch_bounds__(64 * tail_waves(STACK)) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_pt_tail(
+    SceneDev S, PtParams P, ShadeHooks H, Queue in, const uint32_t* __restrict__ count, PathState ps,
+    float4* __restrict__ rad, unsigned long long* __restrict__ stats) {
+    __shared__ TailLds<STACK> lds;
+    tail_paths<STACK>(SceneOne{S}, P, H, in, *count, ps, rad, lds, stats);
+}
+
+template <int STACK>
+__global__ __launch_bounds__(64 * kGroupWaves) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_pt_tail_group(
+    SceneDev S, PtParams P, ShadeHooks H, Queue in, const uint32_t* __restrict__ count, PathState ps,
+    float4* __restrict__ rad, unsigned long long* __restrict__ stats) {
+    __shared__ GroupLds<STACK> lds;
+    tail_paths_group<STACK>(SceneOne{S}, P, H, in, *count, ps, rad, lds, stats);
 }
 
 // Output of the frame: its mean radiance, or with `accumulate` the weighted
@@ -260,9 +285,13 @@ __global__ void k_add_f64(const float4* __restrict__ rad, double* __restrict__ a
 }
 
 inline uint32_t nblk(uint32_t n, uint32_t b) { return n == 0 ? 1 : (n + b - 1) / b; }
-// Resident blocks per CU of the per-thread tail (119 VGPRs: 4 waves per SIMD).
-constexpr uint32_t kTailBlocksPerCu = 8;
 constexpr uint32_t kTailNever = 0xFFFFFFFFu;
+// Longest queue the path kernel takes from the wavefront.  From bounce 1 on it
+// beats a launch per bounce at 65k, 1.3M and 1.9M paths (1.02M-triangle frame at
+// 1080p 1.60 ms from bounce 1, 1.77 from 2, 1.94 from 3; room 1.00, 1.13, 1.26),
+// while the wavefront's 6 waves per SIMD are ahead on the 15M paths of 64 batched
+// views (11.94 ms from bounce 1, 11.66 from 2, 11.27 from 3): the line lies between.
+constexpr unsigned long long kTailFit = 1ull << 22;
 
 // inverse of a 4x4 (row-major) by cofactors, in double
 bool inverse4(const double m[16], double inv[16]) {
@@ -417,22 +446,20 @@ snkpt_status launch_tail(snkpt_ctx* ctx, RenderState& R, const SceneDev& S, cons
     if (A.num_tris == 0) return SNKPT_OK;  // no hits, so nothing was queued
     const uint32_t need = A.depth > 0 ? A.depth - 1 : 0;
     const uint32_t cus = ctx->props.multiProcessorCount > 0 ? (uint32_t)ctx->props.multiProcessorCount : 256u;
-    const uint32_t grid = std::min(nblk(n_max, kMegaBlock), cus * kTailBlocksPerCu);
     const uint32_t* count = R.counts.as<uint32_t>() + cur;
     unsigned long long* stats = R.stats.as<unsigned long long>();
-#define SNKPT_TAIL(STK) \
-    k_pt_tail<STK><<<grid, kMegaBlock, 0, st>>>(S, P, H, queue_of(R, cur), count, paths_of(R), rad, stats)
-    if (need <= 10)
-        SNKPT_TAIL(10);
-    else if (need <= 16)
-        SNKPT_TAIL(16);
-    else if (need <= 32)
-        SNKPT_TAIL(32);
-    else if (need <= 64)
-        SNKPT_TAIL(64);
-    else
-        return fail(ctx, SNKPT_ERR_CAPACITY, "path tail: BVH8 deeper than the 64-entry traversal stack");
-#undef SNKPT_TAIL
+    const bool ok = with_stack(need, [&](auto s) {
+        constexpr int SK = decltype(s)::value;
+        if (n_max <= group_paths(std::min(A.depth, 64u))) {
+            const TraceGrid g = group_grid(16u, cus, n_max);
+            k_pt_tail_group<SK><<<g.blocks, g.threads, 0, st>>>(S, P, H, queue_of(R, cur), count, paths_of(R), rad,
+                                                                stats);
+            return;
+        }
+        const TraceGrid g = tail_grid(SK, cus, n_max);
+        k_pt_tail<SK><<<g.blocks, g.threads, 0, st>>>(S, P, H, queue_of(R, cur), count, paths_of(R), rad, stats);
+    });
+    if (!ok) return fail(ctx, SNKPT_ERR_CAPACITY, "path tail: BVH8 deeper than the 64-entry traversal stack");
     return SNKPT_OK;
 }
 
@@ -441,9 +468,16 @@ snkpt_status launch_shadow(snkpt_ctx* ctx, RenderState& R, float4* rad, hipStrea
     if (A.num_tris == 0) return SNKPT_OK;  // no hits, so no shadow rays were queued
     uint32_t need = A.depth > 0 ? A.depth - 1 : 0;
     const uint32_t cus = ctx->props.multiProcessorCount > 0 ? (uint32_t)ctx->props.multiProcessorCount : 256u;
+    const uint32_t most = n_max ? n_max : R.w * R.h;
     const bool ok = with_stack(need, [&](auto s) {
         constexpr int S = decltype(s)::value;
-        const TraceGrid g = trace_grid(S, trace_waves(S), (uint32_t)cu_waves(S), cus, n_max ? n_max : R.w * R.h);
+        if (most <= kGroupRays) {
+            const TraceGrid g = group_grid(kGroupCuWaves, cus, most);
+            k_shadow_group<S><<<g.blocks, g.threads, 0, st>>>(A.nodes.as<uint4>(), A.leaf_tris.as<float4>(),
+                                                              shadow_of(R), R.counts.as<uint32_t>(), rad);
+            return;
+        }
+        const TraceGrid g = trace_grid(S, trace_waves(S), (uint32_t)cu_waves(S), cus, most);
         k_shadow<S><<<g.blocks, g.threads, 0, st>>>(A.nodes.as<uint4>(), A.leaf_tris.as<float4>(), shadow_of(R),
                                                     R.counts.as<uint32_t>(), rad);
     });
@@ -468,7 +502,8 @@ snkpt_status pt_bounces(snkpt_ctx* ctx, const snkpt_settings* s, int cur, uint32
     if (H.kind == 0) {
         const uint32_t t = s->tail_bounce ? s->tail_bounce
                            : R.tail_auto  ? R.tail_auto
-                                          : std::max(1u, P.rr_start);
+                           : n <= kTailFit ? 1u
+                                           : std::max(1u, P.rr_start);
         tail_from = t < P.max_depth ? std::max(t, 1u) : 0u;
     }
     R.hist_first = first;
@@ -606,19 +641,17 @@ snkpt_status begin_frame(snkpt_ctx* ctx, uint32_t w, uint32_t h, hipStream_t st)
     return SNKPT_OK;
 }
 
-// The per-thread tail's bounce for the next frame: the first bounce (>= 1) whose
-// queue of paths fits twice the tail's resident lanes.  q: this frame's queue
+// The path kernel's bounce for the next frame: the first bounce (>= 1) whose
+// queue holds at most kTailFit paths.  q: this frame's queue
 // lengths, known for the bounces the wavefront began (up to the tail's start);
 // when the tail started on a longer queue, the next frame tries one bounce later.
 static void tail_feedback(snkpt_ctx* ctx, const unsigned long long* q) {
     RenderState& R = *ctx->render;
     if (R.hist_depth == 0) return;  // no path-traced bounces this frame
-    const uint32_t cus = ctx->props.multiProcessorCount > 0 ? (uint32_t)ctx->props.multiProcessorCount : 256u;
-    const unsigned long long fit = 2ull * cus * kTailBlocksPerCu * kMegaBlock;
     const uint32_t last = std::min(R.tail_used ? R.tail_used : R.hist_depth - 1, kQueueHist - 1);
     uint32_t pick = R.tail_used && R.tail_used + 1 < R.hist_depth ? R.tail_used + 1 : kTailNever;
     for (uint32_t b = std::max(R.hist_first, 1u); b <= last; ++b)
-        if (q[b] <= fit) {
+        if (q[b] <= kTailFit) {
             pick = b;
             break;
         }
