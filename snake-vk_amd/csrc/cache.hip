@@ -31,7 +31,7 @@ struct CacheState {
     DeviceBuffer mlp32, mlp16, mlp16t, mlp_m, mlp_v, mlp_gradf, grid_gradf;
     // exponential moving averages of the weights (fp32 and the fp16 copies queries read)
     DeviceBuffer grid_e32, grid_e16, mlp_e32, mlp_e16;
-    DeviceBuffer partial, loss_part, x0, dx0, y, mlp_red, grid_priv;
+    DeviceBuffer partial, loss_part, x0, pos, rows, dx0, y, mlp_red, grid_priv;
     uint32_t cap = 0;         // samples the inference work buffers hold
     uint32_t tcap = 0;        // samples the training work buffers hold
     uint32_t last_n = 0;
@@ -211,6 +211,134 @@ __device__ __forceinline__ void encode_block(const float* __restrict__ samples, 
     }
 }
 
+// ---- encoding of one network's queries, level by level ----
+// The 64 inputs of query i are 32 half pairs, x0t[row * stride + i]: rows 0-15 the
+// grid levels, rows 16-31 the other features, so that one level's features of
+// neighbouring queries are neighbours in memory and a level can be encoded by
+// itself.  A hashed level's table is 2 MiB: with all levels of a query in one
+// block the 32 MiB of tables pass through every die's 4 MB L2 and each gather misses
+// it; level by level (the blocks of a level are launched before the next level's)
+// a die holds the one table it reads.  1M random points: 805 us with 16 levels per
+// block.
+
+// The 8 corner entries of level l: corners k and k + 1 of an x pair lie in one
+// aligned pair of entries when x (hashed: e and e ^ 1; dense: the first entry) is
+// even, and then come with one 8 B load: 6 loads instead of 8 on average.
+__device__ __forceinline__ float2 encode_level_pairs(const float p[3], const GridGeom& G, int l,
+                                                     const __half2* __restrict__ grid) {
+    const Cell c = cell_of(p, (float)G.res[l]);
+    const uint32_t* g = (const uint32_t*)(grid + (size_t)l * kGridT);
+    uint32_t e0[4], e1[4];
+    const bool dense = G.dense[l] != 0u;
+    if (dense) {
+        const uint32_t n = G.res[l] + 1u, e = c.ix + c.iy * n + c.iz * n * n;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            e0[j] = e + (j & 1) * n + (j >> 1) * n * n;
+            e1[j] = e0[j] + 1u;
+        }
+    } else {
+        const uint32_t hy = c.iy * 2654435761u, hz = c.iz * 805459861u;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t h = (hy + (j & 1) * 2654435761u) ^ (hz + (j >> 1) * 805459861u);
+            e0[j] = (c.ix ^ h) & (kGridT - 1u);
+            e1[j] = ((c.ix + 1u) ^ h) & (kGridT - 1u);
+        }
+    }
+    uint2 pr[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) pr[j] = *(const uint2*)(g + (e0[j] & ~1u));
+    uint32_t v[8];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        v[2 * j] = (e0[j] & 1u) ? pr[j].y : pr[j].x;
+        v[2 * j + 1] = (e0[j] & 1u) ? pr[j].x : pr[j].y;
+    }
+    if (dense) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (e0[j] & 1u) v[2 * j + 1] = g[e1[j]];
+    } else if (c.ix & 1u) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[2 * j + 1] = g[e1[j]];
+    }
+    float f0 = 0.0f, f1 = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const float2 f = __half22float2(__builtin_bit_cast(__half2, v[k]));
+        const float w = corner_weight(c, k);
+        f0 += w * f.x;
+        f1 += w * f.y;
+    }
+    return make_float2(f0, f1);
+}
+__device__ __forceinline__ half2v_t to_half2v(float a, float b) {
+    half2v_t v;
+    v[0] = (_Float16)a;
+    v[1] = (_Float16)b;
+    return v;
+}
+
+struct EncLevels {
+    uint32_t n, l[kGridLevels];
+};
+
+// The dense levels (1.2 MB of tables together) and the features that need no grid;
+// the normalised positions go to `pos` (three arrays of `stride`) for the levels' pass.
+constexpr int kEncTBlock = 256;
+__global__ __launch_bounds__(kEncTBlock) void k_encode_dense(const float* __restrict__ samples, uint32_t n,
+                                                             const uint32_t* __restrict__ n_dev, uint32_t stride,
+                                                             GridGeom G, EncLevels L, const __half2* __restrict__ grid,
+                                                             half2v_t* __restrict__ x0t, float* __restrict__ pos) {
+    if (n_dev) n = min(n, *n_dev);
+    const uint32_t i = blockIdx.x * kEncTBlock + threadIdx.x;
+    if (i >= n) return;
+    float s[kSampleFloats];
+    const float4* q = (const float4*)(samples + (size_t)kSampleFloats * i);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const float4 v = q[j];
+        s[4 * j] = v.x, s[4 * j + 1] = v.y, s[4 * j + 2] = v.z, s[4 * j + 3] = v.w;
+    }
+    float p[3];
+    norm_pos(s, G, p);
+    if (pos) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) pos[(size_t)a * stride + i] = p[a];
+    }
+    for (uint32_t k = 0; k < L.n; ++k) {
+        const float2 f = encode_level_pairs(p, G, (int)L.l[k], grid);
+        x0t[(size_t)L.l[k] * stride + i] = to_half2v(f.x, f.y);
+    }
+#pragma unroll
+    for (int l = 0; l < kGridLevels; ++l)
+        x0t[(size_t)(16 + l) * stride + i] = to_half2v(extra_feature(s, 2 * l), extra_feature(s, 2 * l + 1));
+}
+
+// One hashed level per blockIdx.y, a query per thread.
+__global__ __launch_bounds__(kEncTBlock) void k_encode_hashed(const float* __restrict__ samples,
+                                                              const float* __restrict__ pos, uint32_t n,
+                                                              const uint32_t* __restrict__ n_dev, uint32_t stride,
+                                                              GridGeom G, EncLevels L,
+                                                              const __half2* __restrict__ grid,
+                                                              half2v_t* __restrict__ x0t) {
+    if (n_dev) n = min(n, *n_dev);
+    const uint32_t i = blockIdx.x * kEncTBlock + threadIdx.x;
+    if (i >= n) return;
+    const int l = (int)L.l[blockIdx.y];
+    float p[3];
+    if (pos) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) p[a] = pos[(size_t)a * stride + i];
+    } else {
+        norm_pos(samples + (size_t)kSampleFloats * i, G, p);
+    }
+    const float2 f = encode_level_pairs(p, G, l, grid);
+    x0t[(size_t)l * stride + i] = to_half2v(f.x, f.y);
+}
+
+// A small call in one launch, into rows of 64 inputs.
 __global__ __launch_bounds__(kEncBlock) void k_encode(const float* __restrict__ samples, uint32_t n,
                                                      const uint32_t* __restrict__ n_dev, GridGeom G,
                                                      const __half2* __restrict__ grid, _Float16* __restrict__ x0) {
@@ -218,6 +346,41 @@ __global__ __launch_bounds__(kEncBlock) void k_encode(const float* __restrict__ 
     if (blockIdx.x * 64 >= n) return;  // the whole block is past the end
     encode_block(samples, n, G, grid, x0);
 }
+
+// Largest call encoded in one launch: queries of random points take 25 / 39 / 65 /
+// 121 us at 16k / 32k / 65k / 131k in one launch, 37 / 46 / 53 / 77 in two.
+constexpr uint32_t kEncSmall = 1u << 15;
+
+// Stride of the level-major encoding of a call for n queries; 0: rows of 64 inputs.
+inline uint32_t enc_stride(uint32_t n) { return n <= kEncSmall ? 0u : (n + 63u) & ~63u; }
+// Encodes n queries (min(n, *n_dev) with n_dev) into x0t in the layout of
+// enc_stride(n); pos: 3 x stride floats, or null (the samples' positions are then
+// read per level).
+void encode_queries(const float* samples, uint32_t n, const uint32_t* n_dev, const GridGeom& G, const __half2* grid,
+                    _Float16* x0t, float* pos, hipStream_t st) {
+    if (n == 0) return;
+    EncLevels d{0, {}}, h{0, {}};
+    for (int l = 0; l < kGridLevels; ++l) {
+        EncLevels& e = G.dense[l] ? d : h;
+        e.l[e.n++] = (uint32_t)l;
+    }
+    const uint32_t blocks = (n + kEncTBlock - 1) / kEncTBlock, stride = enc_stride(n);
+    if (!stride) {
+        k_encode<<<(n + 63) / 64, kEncBlock, 0, st>>>(samples, n, n_dev, G, grid, x0t);
+        return;
+    }
+    k_encode_dense<<<blocks, kEncTBlock, 0, st>>>(samples, n, n_dev, stride, G, d, grid, (half2v_t*)x0t, pos);
+    if (h.n)
+        k_encode_hashed<<<dim3(blocks, h.n), kEncTBlock, 0, st>>>(samples, pos, n, n_dev, stride, G, h, grid,
+                                                                  (half2v_t*)x0t);
+}
+
+// Rows of 64 inputs per query from the encoded queries (for reading them back).
+__global__ void k_rows_of(const half2v_t* __restrict__ x0t, uint32_t n, uint32_t stride, half2v_t* __restrict__ rows) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, r = blockIdx.y;
+    if (i < n) rows[(size_t)32 * i + r] = x0t[(size_t)r * stride + i];
+}
+
 inline uint32_t enc_blocks(uint32_t n) { return n == 0 ? 1u : (n + 63) / 64; }
 
 // Network of the 64-row-aligned segment holding `row`: segments [off[k], off[k+1])
@@ -281,6 +444,22 @@ __device__ __forceinline__ void load_x0_tile(const _Float16* __restrict__ x0, ui
     }
 }
 
+// The same from the level-major encoding.
+__device__ __forceinline__ void load_x0t_tile(const _Float16* __restrict__ x0t, uint32_t base, uint32_t n,
+                                              uint32_t stride, _Float16* act, int lane) {
+    const uint32_t q = base + lane;
+    const uint32_t* src = (const uint32_t*)x0t + q;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        uint4 v = make_uint4(0u, 0u, 0u, 0u);
+        if (q < n) {
+            const uint32_t* r = src + (size_t)(4 * j) * stride;
+            v = make_uint4(r[0], r[stride], r[2 * (size_t)stride], r[3 * (size_t)stride]);
+        }
+        *(uint4*)(act + lane * kRow + 8 * j) = v;
+    }
+}
+
 constexpr int kInferWaves = 4;
 
 // ReLU of FP16 values as a signed 16-bit max with 0 (a negative half has its
@@ -333,12 +512,16 @@ __device__ __forceinline__ void layer_hidden(const _Float16* in, const _Float16*
 }
 
 // 64 rows per wave from `base` through the network W (rows at or past n read as zero).
-__device__ __forceinline__ void infer_block(const _Float16* __restrict__ x0, uint32_t n, uint32_t base,
-                                            const _Float16* __restrict__ W, float4* __restrict__ y) {
+// x0: rows of 64 inputs (stride 0), or the level-major encoding of this stride.
+__device__ __forceinline__ void infer_block(const _Float16* __restrict__ x0, uint32_t stride, uint32_t n,
+                                            uint32_t base, const _Float16* __restrict__ W, float4* __restrict__ y) {
     __shared__ __attribute__((aligned(16))) _Float16 buf[kInferWaves][64 * kRow];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     _Float16* a0 = buf[wv];
-    load_x0_tile(x0, base, n, a0, lane);
+    if (stride)
+        load_x0t_tile(x0, base, n, stride, a0, lane);
+    else
+        load_x0_tile(x0, base, n, a0, lane);
     __syncthreads();
 #pragma unroll
     for (int l = 0; l < kHidden; ++l) {
@@ -365,15 +548,16 @@ __device__ __forceinline__ void infer_block(const _Float16* __restrict__ x0, uin
     }
 }
 
-// Inference: y[q] = MLP(x0[q]) for 64 samples per wave.
-__global__ __launch_bounds__(64 * kInferWaves) void k_mlp_infer(const _Float16* __restrict__ x0, uint32_t n,
+// Inference: y[q] = MLP of the encoded query q, 64 queries per wave.
+__global__ __launch_bounds__(64 * kInferWaves) void k_mlp_infer(const _Float16* __restrict__ x0t, uint32_t stride,
+                                                                uint32_t n,
                                                                 const uint32_t* __restrict__ n_dev,
                                                                 const _Float16* __restrict__ W,
                                                                 float4* __restrict__ y) {
     if (n_dev) n = min(n, *n_dev);
     if (blockIdx.x * kInferWaves * 64 >= n) return;  // the whole block is past the end
     // waves past n run on zero rows
-    infer_block(x0, n, (blockIdx.x * kInferWaves + (threadIdx.x >> 6)) * 64, W, y);
+    infer_block(x0t, stride, n, (blockIdx.x * kInferWaves + (threadIdx.x >> 6)) * 64, W, y);
 }
 
 // Inference of queries grouped by network (segments as for k_encode_many): each
@@ -387,7 +571,7 @@ __global__ __launch_bounds__(64 * kInferWaves) void k_mlp_infer_many(const _Floa
     const uint32_t base = (blockIdx.x * kInferWaves + (threadIdx.x >> 6)) * 64;
     // a wave past the rows runs on zero rows through network 0 and stores nothing
     const uint32_t k = base < n ? segment_of(off, nseg, base) : 0u;
-    infer_block(x0, n, base, refs[k].mlp, y);
+    infer_block(x0, 0u, n, base, refs[k].mlp, y);
 }
 
 // dX tile (64 samples x 64 inputs) = dZ (64 x K) * W (K x 64), via W^T rows.
@@ -452,8 +636,8 @@ __device__ __forceinline__ void back_dw(const _Float16* g, const _Float16* x, fl
 // The batch holds min(n, *n_dev) samples (n alone without n_dev); the loss is
 // the mean over them of the three channels' relative squared errors, scaled by
 // kLossScale for the FP16 backward.
-__global__ __launch_bounds__(64) void k_mlp_train(const _Float16* __restrict__ x0, const float* __restrict__ samples,
-                                                  uint32_t n, const uint32_t* __restrict__ n_dev,
+__global__ __launch_bounds__(64) void k_mlp_train(const _Float16* __restrict__ x0t, uint32_t stride,
+                                                  const float* __restrict__ samples, uint32_t n, const uint32_t* __restrict__ n_dev,
                                                   const _Float16* __restrict__ W, const _Float16* __restrict__ WT,
                                                   float* __restrict__ partial, float* __restrict__ dx0,
                                                   float* __restrict__ loss_part, uint32_t hashed_levels,
@@ -465,7 +649,10 @@ __global__ __launch_bounds__(64) void k_mlp_train(const _Float16* __restrict__ x
     if (n_dev) n = min(n, *n_dev);
     if (base >= n) return;  // the whole wave is past the batch
     const float grad_scale = kLossScale / (3.0f * (float)n);
-    load_x0_tile(x0, base, n, act[0], lane);
+    if (stride)
+        load_x0t_tile(x0t, base, n, stride, act[0], lane);
+    else
+        load_x0_tile(x0t, base, n, act[0], lane);
     __syncthreads();
     for (int l = 0; l < kHidden; ++l) {
         layer_hidden(act[l], W + l * kLayerParams, act[l + 1], lane);
@@ -915,6 +1102,7 @@ static snkpt_status ensure_work(snkpt_ctx* ctx, CacheState& C, uint32_t n, bool 
     const uint32_t cap = ((n + 63) / 64) * 64;
     if (cap > C.cap) {
         HIPC(C.x0.reserve((size_t)cap * 128));
+        HIPC(C.pos.reserve((size_t)cap * 12));
         HIPC(C.y.reserve((size_t)cap * 16));
         C.cap = cap;
     }
@@ -934,11 +1122,10 @@ snkpt_status cache_infer(snkpt_ctx* ctx, const float* samples, uint32_t n, float
     if (n == 0) return SNKPT_OK;
     snkpt_status e = ensure_work(ctx, C, n, false);
     if (e != SNKPT_OK) return e;
-    k_encode<<<enc_blocks(n), kEncBlock, 0, st>>>(samples, n, nullptr, C.geom, C.grid16.as<__half2>(),
-                                               C.x0.as<_Float16>());
+    encode_queries(samples, n, nullptr, C.geom, C.grid16.as<__half2>(), C.x0.as<_Float16>(), C.pos.as<float>(), st);
     const uint32_t waves = (n + 63) / 64;
     k_mlp_infer<<<(waves + kInferWaves - 1) / kInferWaves, 64 * kInferWaves, 0, st>>>(
-        C.x0.as<_Float16>(), n, nullptr, C.mlp16.as<_Float16>(), (float4*)out);
+        C.x0.as<_Float16>(), enc_stride(n), n, nullptr, C.mlp16.as<_Float16>(), (float4*)out);
     C.last_n = n;
     hipError_t le = hipGetLastError();
     if (le != hipSuccess) return hip_fail(ctx, le, "cache_infer launch");
@@ -987,11 +1174,10 @@ snkpt_status cache_infer_noalloc(snkpt_ctx* ctx, const float* samples, uint32_t 
     }
     if (!x0) return fail(ctx, SNKPT_ERR_HIP, "cache_infer_noalloc: workspace address not set up for this device");
     CacheState& C = *Cp;
-    k_encode<<<enc_blocks(n), kEncBlock, 0, st>>>(samples, n, nullptr, C.geom, C.grid16.as<__half2>(), x0);
+    encode_queries(samples, n, nullptr, C.geom, C.grid16.as<__half2>(), x0, nullptr, st);
     const uint32_t waves = (n + 63) / 64;
-    k_mlp_infer<<<(waves + kInferWaves - 1) / kInferWaves, 64 * kInferWaves, 0, st>>>(x0, n, nullptr,
-                                                                                      C.mlp16.as<_Float16>(),
-                                                                                      (float4*)out);
+    k_mlp_infer<<<(waves + kInferWaves - 1) / kInferWaves, 64 * kInferWaves, 0, st>>>(
+        x0, enc_stride(n), n, nullptr, C.mlp16.as<_Float16>(), (float4*)out);
     hipError_t le = hipGetLastError();
     if (le != hipSuccess) return hip_fail(ctx, le, "cache_infer_noalloc launch");
     return SNKPT_OK;
@@ -1019,12 +1205,11 @@ snkpt_status cache_train_run(snkpt_ctx* ctx, const float* samples, uint32_t n, c
     AdamDev* ad = C.adam.as<AdamDev>();
     k_adam_advance<<<1, 64, 0, st>>>(ad, n, n_dev, lr, ema, b1, b2, apply);
     const uint32_t chunks = (n + 63) / 64;
-    k_encode<<<enc_blocks(n), kEncBlock, 0, st>>>(samples, n, n_dev, C.geom, C.grid16.as<__half2>(),
-                                               C.x0.as<_Float16>());
+    encode_queries(samples, n, n_dev, C.geom, C.grid16.as<__half2>(), C.x0.as<_Float16>(), C.pos.as<float>(), st);
     uint32_t hashed = 0;
     for (int l = 0; l < kGridLevels; ++l)
         if (!C.geom.dense[l]) hashed |= 1u << l;
-    k_mlp_train<<<chunks, 64, 0, st>>>(C.x0.as<_Float16>(), samples, n, n_dev, C.mlp16.as<_Float16>(),
+    k_mlp_train<<<chunks, 64, 0, st>>>(C.x0.as<_Float16>(), enc_stride(n), samples, n, n_dev, C.mlp16.as<_Float16>(),
                                        C.mlp16t.as<_Float16>(), C.partial.as<float>(), C.dx0.as<float>(),
                                        C.loss_part.as<float>(), hashed, ad);
     k_grid_bwd<<<grid_for(n, 128), 128, 0, st>>>(samples, C.dx0.as<float>(), n, n_dev, C.geom,
@@ -1112,6 +1297,12 @@ snkpt_status cache_params(snkpt_ctx* ctx, uint32_t which, void* dst, size_t byte
                       : which == 6 ? C.q_meta.ptr
                                    : C.t_samples.ptr;
     if (sz == 0) return SNKPT_OK;
+    if (which == 4 && enc_stride(C.last_n)) {
+        HIPC(C.rows.reserve(sz));
+        k_rows_of<<<dim3((C.last_n + 255) / 256, 32), 256, 0, st>>>(C.x0.as<half2v_t>(), C.last_n,
+                                                                   enc_stride(C.last_n), C.rows.as<half2v_t>());
+        src = C.rows.ptr;
+    }
     HIPC(hipMemcpyAsync(dst, src, sz, hipMemcpyDeviceToHost, st));
     HIPC(hipStreamSynchronize(st));
     return SNKPT_OK;
@@ -1295,12 +1486,11 @@ snkpt_status cache_query(snkpt_ctx* ctx, const float* samples, uint32_t n, float
     if (n == 0) return SNKPT_OK;
     snkpt_status e = ensure_work(ctx, C, n, false);
     if (e != SNKPT_OK) return e;
-    k_encode<<<enc_blocks(n), kEncBlock, 0, st>>>(samples, n, nullptr, C.geom,
-                                                  (averaged ? C.grid_e16 : C.grid16).as<__half2>(),
-                                                  C.x0.as<_Float16>());
+    encode_queries(samples, n, nullptr, C.geom, (averaged ? C.grid_e16 : C.grid16).as<__half2>(),
+                   C.x0.as<_Float16>(), C.pos.as<float>(), st);
     const uint32_t waves = (n + 63) / 64;
     k_mlp_infer<<<(waves + kInferWaves - 1) / kInferWaves, 64 * kInferWaves, 0, st>>>(
-        C.x0.as<_Float16>(), n, nullptr, (averaged ? C.mlp_e16 : C.mlp16).as<_Float16>(), y);
+        C.x0.as<_Float16>(), enc_stride(n), n, nullptr, (averaged ? C.mlp_e16 : C.mlp16).as<_Float16>(), y);
     return SNKPT_OK;
 }
 
@@ -1535,11 +1725,11 @@ snkpt_status cache_pass(snkpt_ctx* ctx, const CamDev& cd, const snkpt_settings* 
     if ((e = primary_bounces(ctx, cd, s, initstate, st, &H, bounces)) != SNKPT_OK) return e;
     // 2. query the cache
     const bool avg = s->cache_ema > 0.0f;  // query the weight averages
-    k_encode<<<enc_blocks(n), kEncBlock, 0, st>>>(C.q_samples.as<float>(), n, qc, C.geom,
-                                                  (avg ? C.grid_e16 : C.grid16).as<__half2>(), C.x0.as<_Float16>());
+    encode_queries(C.q_samples.as<float>(), n, qc, C.geom, (avg ? C.grid_e16 : C.grid16).as<__half2>(),
+                   C.x0.as<_Float16>(), C.pos.as<float>(), st);
     const uint32_t waves = (n + 63) / 64;
     k_mlp_infer<<<(waves + kInferWaves - 1) / kInferWaves, 64 * kInferWaves, 0, st>>>(
-        C.x0.as<_Float16>(), n, qc, (avg ? C.mlp_e16 : C.mlp16).as<_Float16>(), C.y.as<float4>());
+        C.x0.as<_Float16>(), enc_stride(n), n, qc, (avg ? C.mlp_e16 : C.mlp16).as<_Float16>(), C.y.as<float4>());
     k_cache_apply<<<grid_for(n, 256), 256, 0, st>>>(C.q_meta.as<float4>(), C.y.as<float4>(), qc, R.rad.as<float4>(),
                                                       stats + 3);
     (void)pass;

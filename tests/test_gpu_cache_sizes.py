@@ -1,0 +1,49 @@
+"""GPU: the cache's queries give the same bits whatever the call's size (rows of
+inputs up to 32,768 queries, level by level above), against the FP64 oracle's
+encoding at the line between the two and at ragged sizes."""
+import numpy as np
+import pytest
+
+from oracle import binding as O
+
+pytestmark = pytest.mark.gpu
+LO, HI = [-1.0, 0.0, -1.0], [1.0, 2.0, 1.0]
+
+
+@pytest.fixture(scope="module")
+def net(gpu):
+    import snkpt
+    import torch
+    ctx = snkpt.Context(0)
+    ctx.cache_reset(3, LO, HI)
+    rng = np.random.default_rng(4)
+    grid = (rng.uniform(-1, 1, O.GRID_PARAMS) * 0.3).astype(np.float32)
+    ctx.cache_set_params(1, grid)
+    n = 70001
+    s = np.zeros((n, 16), np.float32)
+    s[:, 0:3] = rng.uniform([-1.1, -0.1, -1.1], [1.1, 2.1, 1.1], (n, 3))  # some outside the box
+    s[:8, 0:3] = [[a, b, c] for a in (-1, 1) for b in (0, 2) for c in (-1, 1)]  # its corners
+    d = rng.normal(size=(n, 6))
+    s[:, 3:6] = d[:, :3] / np.linalg.norm(d[:, :3], axis=1, keepdims=True)
+    s[:, 6:9] = d[:, 3:] / np.linalg.norm(d[:, 3:], axis=1, keepdims=True)
+    s[:, 9:13] = rng.uniform(0.05, 1, (n, 4))
+    t = torch.from_numpy(s).cuda()
+    full = ctx.cache_infer(t).cpu().numpy()
+    enc = ctx.cache_params(4).reshape(n, 64).copy()
+    return ctx, s, t, full, enc, grid
+
+
+@pytest.mark.parametrize("n", [1, 65, 32767, 32768, 32769, 65535, 70001])
+def test_same_bits_at_every_size(net, n):
+    ctx, _, t, full, enc, _ = net
+    y = ctx.cache_infer(t[:n].contiguous()).cpu().numpy()
+    assert np.array_equal(y.view(np.uint32), full[:n].view(np.uint32))
+    assert np.array_equal(ctx.cache_params(4).view(np.uint16), enc[:n].reshape(-1).view(np.uint16))
+
+
+def test_encoding_matches_oracle(net):
+    _, s, _, _, enc, grid = net
+    pick = np.r_[0:64, 32700:32800, 69900:70001]
+    want = O.cache_encode(O.CacheGeom(LO, HI), grid, s[pick])
+    # FP16 grid entries and an FP16 result: the tolerance of the row-wise encoding's test
+    assert np.allclose(enc[pick].astype(np.float64), want, rtol=4e-3, atol=2e-3)
