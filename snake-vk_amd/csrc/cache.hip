@@ -27,11 +27,11 @@ struct CacheState {
     bool ready = false;
     GridGeom geom{};
     DeviceBuffer adam;        // AdamDev: the optimiser's step counter and the step's factors
-    DeviceBuffer grid32, grid16, grid_m, grid_v, grid_grad;  // grid_grad: int64 fixed point
+    DeviceBuffer grid32, grid16, grid_m, grid_v, grid_grad;  // grid_grad: fixed point, hashed levels
     DeviceBuffer mlp32, mlp16, mlp16t, mlp_m, mlp_v, mlp_gradf, grid_gradf;
     // exponential moving averages of the weights (fp32 and the fp16 copies queries read)
     DeviceBuffer grid_e32, grid_e16, mlp_e32, mlp_e16;
-    DeviceBuffer partial, loss_part, x0, pos, rows, dx0, y, mlp_red, grid_priv;
+    DeviceBuffer partial, loss_part, x0, pos, rows, dx0, y, mlp_red, grid_priv;  // grid_priv: dense levels' gradient copies
     uint32_t cap = 0;         // samples the inference work buffers hold
     uint32_t tcap = 0;        // samples the training work buffers hold
     uint32_t last_n = 0;
@@ -182,7 +182,8 @@ __device__ __forceinline__ float extra_feature(const float* s, int k) {
 constexpr int kEncBlock = 64 * kGridLevels;
 // Rows [64 blk, 64 blk + 64) of x0, for blocks of kEncBlock threads.
 __device__ __forceinline__ void encode_block(const float* __restrict__ samples, uint32_t n, const GridGeom& G,
-                                             const __half2* __restrict__ grid, _Float16* __restrict__ x0) {
+                                             const __half2* __restrict__ grid, _Float16* __restrict__ x0,
+                                             float* __restrict__ pos = nullptr, uint32_t pos_stride = 0) {
     // the 64 input rows of the block are assembled in LDS and written out as
     // whole 128 B rows (4 B stores at a 128 B stride would be 64 partial lines)
     __shared__ half2v_t tile[64][33];
@@ -192,6 +193,7 @@ __device__ __forceinline__ void encode_block(const float* __restrict__ samples, 
         const float* s = samples + (size_t)kSampleFloats * i;
         float p[3];
         norm_pos(s, G, p);
+        if (pos && l < 3) pos[(size_t)l * pos_stride + i] = p[l];
         float2 f = encode_level(p, G, l, grid);
         half2v_t v, e;
         v[0] = (_Float16)f.x;
@@ -341,10 +343,11 @@ __global__ __launch_bounds__(kEncTBlock) void k_encode_hashed(const float* __res
 // A small call in one launch, into rows of 64 inputs.
 __global__ __launch_bounds__(kEncBlock) void k_encode(const float* __restrict__ samples, uint32_t n,
                                                      const uint32_t* __restrict__ n_dev, GridGeom G,
-                                                     const __half2* __restrict__ grid, _Float16* __restrict__ x0) {
+                                                     const __half2* __restrict__ grid, _Float16* __restrict__ x0,
+                                                     float* __restrict__ pos, uint32_t pos_stride) {
     if (n_dev) n = min(n, *n_dev);
     if (blockIdx.x * 64 >= n) return;  // the whole block is past the end
-    encode_block(samples, n, G, grid, x0);
+    encode_block(samples, n, G, grid, x0, pos, pos_stride);
 }
 
 // Largest call encoded in one launch: queries of random points take 25 / 39 / 65 /
@@ -354,8 +357,8 @@ constexpr uint32_t kEncSmall = 1u << 15;
 // Stride of the level-major encoding of a call for n queries; 0: rows of 64 inputs.
 inline uint32_t enc_stride(uint32_t n) { return n <= kEncSmall ? 0u : (n + 63u) & ~63u; }
 // Encodes n queries (min(n, *n_dev) with n_dev) into x0t in the layout of
-// enc_stride(n); pos: 3 x stride floats, or null (the samples' positions are then
-// read per level).
+// enc_stride(n).  pos: receives the normalised positions, three arrays of n rounded up
+// to 64 (null: a large call reads the samples' positions once per level instead).
 void encode_queries(const float* samples, uint32_t n, const uint32_t* n_dev, const GridGeom& G, const __half2* grid,
                     _Float16* x0t, float* pos, hipStream_t st) {
     if (n == 0) return;
@@ -366,7 +369,7 @@ void encode_queries(const float* samples, uint32_t n, const uint32_t* n_dev, con
     }
     const uint32_t blocks = (n + kEncTBlock - 1) / kEncTBlock, stride = enc_stride(n);
     if (!stride) {
-        k_encode<<<(n + 63) / 64, kEncBlock, 0, st>>>(samples, n, n_dev, G, grid, x0t);
+        k_encode<<<(n + 63) / 64, kEncBlock, 0, st>>>(samples, n, n_dev, G, grid, x0t, pos, (n + 63u) & ~63u);
         return;
     }
     k_encode_dense<<<blocks, kEncTBlock, 0, st>>>(samples, n, n_dev, stride, G, d, grid, (half2v_t*)x0t, pos);
@@ -748,78 +751,149 @@ __global__ __launch_bounds__(64) void k_mlp_train(const _Float16* __restrict__ x
     }
 }
 
-// Gradient privatisation of the coarsest levels: their few entries (17^3,
-// 23^3, 31^3 dense cells) take most same-address atomics, so blocks spread
-// them over kPrivCopies copies (copy = block index mod kPrivCopies) that a
-// second pass sums back in a fixed order.  Integer sums: the result does not
-// depend on the split.
-constexpr int kPrivLevels = 3;
-constexpr int kPrivCopies = 8;
-__host__ __device__ constexpr uint32_t priv_cells(int l) {
-    return l == 0 ? 17u * 17u * 17u : l == 1 ? 23u * 23u * 23u : 31u * 31u * 31u;
-}
-__host__ __device__ constexpr uint32_t priv_base(int l) {
-    return l == 0 ? 0u : l == 1 ? priv_cells(0) : priv_cells(0) + priv_cells(1);
-}
-constexpr uint32_t kPrivEntries = priv_base(kPrivLevels - 1) + priv_cells(kPrivLevels - 1);  // cells per copy
-
-// Scatter dL/dfeature to the 8 corners of each level (64-bit fixed point, so
-// the sums do not depend on the order of the atomics).  One thread per sample
-// walks the levels in turn: at any moment the threads of the grid spread
-// their atomics over several levels.
-__global__ void k_grid_bwd(const float* __restrict__ samples, const float* __restrict__ dx0, uint32_t n,
-                           const uint32_t* __restrict__ n_dev, GridGeom G, unsigned long long* __restrict__ grad,
-                           unsigned long long* __restrict__ priv, const AdamDev* __restrict__ ad) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n_dev) n = min(n, *n_dev);
-    if (i >= n) return;
-    unsigned long long* mine = priv + (size_t)(blockIdx.x % kPrivCopies) * kPrivEntries * 2;
-    const float ps = packed_scale(ad->gmax);
-    float p[3];
-    norm_pos(samples + (size_t)kSampleFloats * i, G, p);
-    for (int l = 0; l < kGridLevels; ++l) {
-        const float g0 = dx0[(size_t)32 * i + 2 * l], g1 = dx0[(size_t)32 * i + 2 * l + 1];
-        if (g0 == 0.0f && g1 == 0.0f) continue;
-        const Cell c = cell_of(p, (float)G.res[l]);
-        if (G.dense[l]) {
-            // dense levels: many samples share an entry; one 64-bit word per feature
-            for (int k = 0; k < 8; ++k) {
-                float w = corner_weight(c, k);
-                const uint32_t idx = corner_index(c, k, G, l);
-                unsigned long long* dst = l < kPrivLevels ? mine + (size_t)(priv_base(l) + idx) * 2
-                                                          : grad + ((size_t)l * kGridT + idx) * 2;
-                long long v0 = (long long)llrint((double)(w * g0) * kFixScale);
-                long long v1 = (long long)llrint((double)(w * g1) * kFixScale);
-                if (v0) atomicAdd(&dst[0], (unsigned long long)v0);
-                if (v1) atomicAdd(&dst[1], (unsigned long long)v1);
+// ---- gradient of the grid ----
+// dL/dfeature of every sample goes to the 8 corners of each level as fixed point
+// (64-bit sums, so they do not depend on the order).  The sums are made in LDS: a
+// task owns 128 KiB of one level's entries (2^14 hashed entries of one packed word,
+// or 2^13 dense entries of a word per feature), looks at all samples for corners in
+// its range, and writes its words out once, so no word is added to in memory, none
+// has to be cleared, and a line leaves whole.  Device-scope 64-bit atomics, one or
+// two per corner, ran at about 35 G/s: 483 us for 65k random samples (11M of them).
+// Looking costs little: an x pair of hashed corners shares the high bits of its
+// index (x < 2^12), so a sample is four hashes and compares per level; what lies in
+// the range is queued per wave and added 64 at a time.  Coarse dense levels have few
+// entries that take many corners: their tasks split the samples, each part writing a
+// copy of its own, and the optimiser adds the copies up.
+constexpr int kBwdBlock = 1024;
+constexpr uint32_t kHashSlice = 1u << 14;   // entries per hashed task, 8 B each
+constexpr uint32_t kDenseSlice = 1u << 13;  // entries per dense task, 16 B each
+constexpr uint32_t kDenseTasks = 24;        // tasks per dense level: slices x parts is about this
+struct BwdPlan {
+    uint32_t first[kGridLevels + 1];  // first task of a level's
+    uint32_t slices[kGridLevels], parts[kGridLevels];
+    uint32_t cells[kGridLevels];      // entries in use
+    uint32_t copy[kGridLevels];       // dense: first word of the level's copies
+    uint32_t words;                   // words of all copies
+};
+BwdPlan bwd_plan(const GridGeom& G) {
+    BwdPlan p{};
+    uint32_t t = 0;
+    // hashed levels first: their tasks take longest
+    for (int pass = 0; pass < 2; ++pass)
+        for (int l = 0; l < kGridLevels; ++l) {
+            if ((G.dense[l] != 0u) != (pass == 1)) continue;
+            const uint32_t side = G.res[l] + 1u;
+            p.cells[l] = pass ? side * side * side : kGridT;
+            p.slices[l] = pass ? (p.cells[l] + kDenseSlice - 1) / kDenseSlice : kGridT / kHashSlice;
+            p.parts[l] = pass ? std::max(1u, kDenseTasks / p.slices[l]) : 1u;
+            p.first[l] = t;
+            t += p.slices[l] * p.parts[l];
+            if (pass) {
+                p.copy[l] = p.words;
+                p.words += p.parts[l] * p.cells[l] * 2u;
             }
-        } else {
-            for (int k = 0; k < 8; ++k) {
-                float w = corner_weight(c, k);
-                const uint32_t idx = corner_index(c, k, G, l);
-                const long long h = llrintf(w * g0 * ps), lo = llrintf(w * g1 * ps);
+        }
+    p.first[kGridLevels] = t;
+    return p;
+}
+
+__global__ __launch_bounds__(kBwdBlock) void k_grid_bwd(const float* __restrict__ pos, uint32_t stride,
+                                                        const float* __restrict__ dx0, uint32_t n,
+                                                        const uint32_t* __restrict__ n_dev, GridGeom G, BwdPlan P,
+                                                        unsigned long long* __restrict__ hashed,
+                                                        unsigned long long* __restrict__ copies,
+                                                        const AdamDev* __restrict__ ad) {
+    constexpr uint32_t kWords = kHashSlice;  // == 2 x kDenseSlice
+    __shared__ unsigned long long word[kWords];
+    __shared__ uint32_t queue[kBwdBlock / 64][128];
+    if (n_dev) n = min(n, *n_dev);
+    const uint32_t task = blockIdx.x;
+    int l = 0;
+    for (int k = 0; k < kGridLevels; ++k)
+        if (task >= P.first[k] && task - P.first[k] < P.slices[k] * P.parts[k]) l = k;
+    const uint32_t rel = task - P.first[l], slice = rel % P.slices[l], part = rel / P.slices[l];
+    const bool dense = G.dense[l] != 0u;
+    for (uint32_t w = threadIdx.x; w < kWords; w += kBwdBlock) word[w] = 0ull;
+    __syncthreads();
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    uint32_t* q = queue[wave];
+    uint32_t queued = 0;
+    const float r = (float)G.res[l];
+    const uint32_t side = G.res[l] + 1u;
+    const float ps = packed_scale(ad->gmax);
+    // adds the x pair j of sample i (entry i * 4 + j)
+    auto add = [&](uint32_t entry) {
+        const uint32_t i = entry >> 2;
+        const int j = (int)(entry & 3u);
+        const float2 g = *(const float2*)(dx0 + (size_t)32 * i + 2 * l);
+        if (g.x == 0.0f && g.y == 0.0f) return;
+        float p[3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) p[a] = pos[(size_t)a * stride + i];
+        const Cell c = cell_of(p, r);
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            const int k = 2 * j + x;
+            const float w = corner_weight(c, k);
+            const uint32_t e = corner_index(c, k, G, l);
+            if (dense) {
+                const uint32_t at = e - slice * kDenseSlice;
+                if (at >= kDenseSlice) continue;  // the other corner of the pair lies in this slice
+                const long long v0 = (long long)llrint((double)(w * g.x) * kFixScale);
+                const long long v1 = (long long)llrint((double)(w * g.y) * kFixScale);
+                if (v0) atomicAdd(&word[2 * at], (unsigned long long)v0);
+                if (v1) atomicAdd(&word[2 * at + 1], (unsigned long long)v1);
+            } else {
+                const long long h = llrintf(w * g.x * ps), lo = llrintf(w * g.y * ps);
                 const long long v = h * 4294967296ll + lo;
-                if (v) atomicAdd(&grad[((size_t)l * kGridT + idx) * 2], (unsigned long long)v);
+                if (v) atomicAdd(&word[e & (kHashSlice - 1u)], (unsigned long long)v);
+            }
+        }
+    };
+    const uint32_t i0 = (uint32_t)(((uint64_t)n * part) / P.parts[l]);
+    const uint32_t i1 = (uint32_t)(((uint64_t)n * (part + 1u)) / P.parts[l]);
+    for (uint32_t at = i0 + wave * 64u; at < i1; at += kBwdBlock) {
+        const uint32_t i = at + lane;
+        const bool in = i < i1;
+        Cell c{0u, 0u, 0u, 0.0f, 0.0f, 0.0f};
+        if (in) {
+            float p[3];
+#pragma unroll
+            for (int a = 0; a < 3; ++a) p[a] = pos[(size_t)a * stride + i];
+            c = cell_of(p, r);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            bool mine;
+            if (dense) {
+                const uint32_t e = c.ix + (c.iy + (j & 1)) * side + (c.iz + (j >> 1)) * side * side;
+                mine = e / kDenseSlice == slice || (e + 1u) / kDenseSlice == slice;
+            } else {
+                const uint32_t h = (c.iy + (j & 1)) * 2654435761u ^ (c.iz + (j >> 1)) * 805459861u;
+                mine = (h & (kGridT - 1u)) / kHashSlice == slice;
+            }
+            mine = mine && in;
+            const uint64_t m = __ballot(mine);
+            if (mine) q[queued + (uint32_t)__popcll(m & below)] = i * 4u + (uint32_t)j;
+            __builtin_amdgcn_wave_barrier();
+            queued += (uint32_t)__popcll(m);
+            if (queued >= 64u) {  // at most 127 queued before this
+                queued -= 64u;
+                add(q[queued + lane]);
             }
         }
     }
-}
-
-// Folds the private copies into the gradient (copies in a fixed order) and clears them.
-__global__ void k_grid_priv_fold(unsigned long long* __restrict__ priv, unsigned long long* __restrict__ grad) {
-    const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;  // entry * 2 + feature
-    if (e >= kPrivEntries * 2) return;
-    const uint32_t cell = e >> 1, f = e & 1u;
-    const int l = cell < priv_base(1) ? 0 : cell < priv_base(2) ? 1 : 2;
-    unsigned long long s = 0;
-#pragma unroll
-    for (int c = 0; c < kPrivCopies; ++c) {
-        unsigned long long* q = priv + (size_t)c * kPrivEntries * 2 + e;
-        s += *q;
-        *q = 0ull;
+    if (lane < queued) add(q[lane]);
+    __syncthreads();
+    if (dense) {
+        const uint32_t first = slice * kDenseSlice, cells = min(kDenseSlice, P.cells[l] - first);
+        unsigned long long* o = copies + P.copy[l] + ((size_t)part * P.cells[l] + first) * 2u;
+        for (uint32_t w = threadIdx.x; w < 2u * cells; w += kBwdBlock) o[w] = word[w];
+    } else {
+        unsigned long long* o = hashed + (size_t)l * kGridT + (size_t)slice * kHashSlice;
+        for (uint32_t w = threadIdx.x; w < kHashSlice; w += kBwdBlock) o[w] = word[w];
     }
-    const size_t g = ((size_t)l * kGridT + (cell - priv_base(l))) * 2 + f;
-    grad[g] += s;
 }
 
 struct AdamP {
@@ -848,6 +922,8 @@ __global__ void k_mlp_reduce(const float* __restrict__ partial, uint32_t n, cons
     if (blockIdx.y >= groups) return;
     uint32_t c0 = blockIdx.y * per, c1 = min(nchunks, c0 + per);
     float g = 0.0f;
+    // (16 loads in flight; the sum keeps its order)
+#pragma unroll 16
     for (uint32_t c = c0; c < c1; ++c) g += partial[(size_t)c * kMlpParams + p];
     red[(size_t)blockIdx.y * kMlpParams + p] = g;
 }
@@ -865,6 +941,7 @@ __global__ void k_mlp_adam(const float* __restrict__ red, uint32_t n, const uint
     uint32_t nchunks, ngroups, per;
     red_shape(n, nchunks, ngroups, per);
     float g = 0.0f;
+#pragma unroll 16
     for (uint32_t c = 0; c < ngroups; ++c) g += red[(size_t)c * kMlpParams + p];
     g *= A.inv_scale;
     gout[p] = g;
@@ -888,36 +965,39 @@ __global__ void k_mlp_adam(const float* __restrict__ red, uint32_t n, const uint
         wt16[kHidden * kLayerParams + i * kWTRow4 + o] = (_Float16)w;
 }
 
-// Adam on the grid, one thread per entry (both features): decodes the
-// entry's fixed-point gradient (a 64-bit word per feature on dense levels, one
-// packed word on hashed levels), clears it, and steps the entry.  Entries
-// without gradient this step are left as they are (lazy / sparse Adam: their
-// moments are not decayed), so a step reads 8-16 B for most untouched entries.
-__global__ void k_grid_adam(unsigned long long* __restrict__ grad, float2* __restrict__ w32, float2* __restrict__ m,
-                            float2* __restrict__ v, __half2* __restrict__ w16, float2* __restrict__ gout,
-                            float2* __restrict__ e32, __half2* __restrict__ e16, GridGeom G, AdamP A,
-                            const AdamDev* __restrict__ ad) {
+// Adam on the grid, one thread per entry (both features): decodes the entry's
+// fixed-point gradient (the sum of the copies' word per feature on dense levels, one
+// packed word on hashed levels) and steps the entry.  Entries without gradient this
+// step are left as they are (lazy / sparse Adam: their moments are not decayed), so a
+// step reads 8 B for an untouched hashed entry.
+__global__ void k_grid_adam(const unsigned long long* __restrict__ hashed,
+                            const unsigned long long* __restrict__ copies, float2* __restrict__ w32,
+                            float2* __restrict__ m, float2* __restrict__ v, __half2* __restrict__ w16,
+                            float2* __restrict__ gout, float2* __restrict__ e32, __half2* __restrict__ e16,
+                            GridGeom G, BwdPlan P, AdamP A, const AdamDev* __restrict__ ad) {
     const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= (size_t)kGridLevels * kGridT || !ad->live) return;
     const uint32_t l = (uint32_t)(e >> kGridLog2T);
     float g0, g1;
     if (G.dense[l]) {
         // a dense level uses its first (res + 1)^3 slots only
-        const uint32_t side = G.res[l] + 1u;
-        if ((uint32_t)(e & (kGridT - 1u)) >= side * side * side) {
+        const uint32_t cell = (uint32_t)(e & (kGridT - 1u)), cells = P.cells[l];
+        if (cell >= cells) {
             if (gout) gout[e] = make_float2(0.0f, 0.0f);
             return;
         }
-        const long long a = (long long)grad[2 * e], b = (long long)grad[2 * e + 1];
+        long long a = 0, b = 0;
+        for (uint32_t c = 0; c < P.parts[l]; ++c) {
+            const ulonglong2 w = *(const ulonglong2*)(copies + P.copy[l] + ((size_t)c * cells + cell) * 2u);
+            a += (long long)w.x;
+            b += (long long)w.y;
+        }
         if ((a | b) == 0 && !gout) return;
-        if (a) grad[2 * e] = 0ull;
-        if (b) grad[2 * e + 1] = 0ull;
         g0 = (float)((double)a / kFixScale);
         g1 = (float)((double)b / kFixScale);
     } else {
-        const long long w = (long long)grad[2 * e];
+        const long long w = (long long)hashed[e];
         if (w == 0 && !gout) return;
-        if (w) grad[2 * e] = 0ull;
         const long long lo = (long long)(int32_t)(uint32_t)((unsigned long long)w & 0xFFFFFFFFull);
         const long long hi = (w - lo) >> 32;
         const float inv = 1.0f / packed_scale(ad->gmax);  // a power of two: exact
@@ -947,7 +1027,7 @@ __global__ void k_grid_adam(unsigned long long* __restrict__ grad, float2* __res
 }
 
 __global__ void k_grid_init(float* __restrict__ w32, __half* __restrict__ w16, float* __restrict__ m,
-                            float* __restrict__ v, unsigned long long* __restrict__ grad, size_t n, uint64_t seed) {
+                            float* __restrict__ v, size_t n, uint64_t seed) {
     size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= n) return;
     Rng r = rng_seed(seed, p);
@@ -956,7 +1036,6 @@ __global__ void k_grid_init(float* __restrict__ w32, __half* __restrict__ w16, f
     w16[p] = __float2half(w);
     m[p] = 0.0f;
     v[p] = 0.0f;
-    grad[p] = 0ull;
 }
 
 __global__ void k_sync_grid16(const float* __restrict__ w32, __half* __restrict__ w16, size_t n) {
@@ -1049,16 +1128,11 @@ snkpt_status cache_reset(snkpt_ctx* ctx, uint32_t seed, const float* lo, const f
         std::memcpy(h3, ctx->accel.hi, 12);
     }
     make_geom(C.geom, l3, h3);
-    for (int l = 0; l < kPrivLevels; ++l) {
-        const uint64_t cells = (uint64_t)(C.geom.res[l] + 1) * (C.geom.res[l] + 1) * (C.geom.res[l] + 1);
-        if (!C.geom.dense[l] || cells != priv_cells(l))
-            return fail(ctx, SNKPT_ERR_INVALID_ARG, "cache_reset: unexpected coarse-level resolution");
-    }
     HIPC(C.grid32.reserve(kGridParams * 4));
     HIPC(C.grid16.reserve(kGridParams * 2));
     HIPC(C.grid_m.reserve(kGridParams * 4));
     HIPC(C.grid_v.reserve(kGridParams * 4));
-    HIPC(C.grid_grad.reserve(kGridParams * 8));
+    HIPC(C.grid_grad.reserve((size_t)kGridLevels * kGridT * 8));
     HIPC(C.mlp32.reserve(kMlpParams * 4));
     HIPC(C.mlp16.reserve(kMlpParams * 2));
     HIPC(C.mlp16t.reserve(kMlpTParams * 2));
@@ -1066,11 +1140,9 @@ snkpt_status cache_reset(snkpt_ctx* ctx, uint32_t seed, const float* lo, const f
     HIPC(C.mlp_v.reserve(kMlpParams * 4));
     HIPC(C.mlp_gradf.reserve(kMlpParams * 4));
     HIPC(C.mlp_red.reserve((size_t)kRedGroups * kMlpParams * 4));
-    HIPC(C.grid_priv.reserve((size_t)kPrivCopies * kPrivEntries * 2 * 8));
-    HIPC(hipMemsetAsync(C.grid_priv.ptr, 0, (size_t)kPrivCopies * kPrivEntries * 2 * 8, st));
+    HIPC(C.grid_priv.reserve((size_t)bwd_plan(C.geom).words * 8));
     k_grid_init<<<(uint32_t)((kGridParams + 255) / 256), 256, 0, st>>>(
-        C.grid32.as<float>(), C.grid16.as<__half>(), C.grid_m.as<float>(), C.grid_v.as<float>(),
-        C.grid_grad.as<unsigned long long>(), kGridParams, 0x6772696400000000ull ^ seed);
+        C.grid32.as<float>(), C.grid16.as<__half>(), C.grid_m.as<float>(), C.grid_v.as<float>(), kGridParams, 0x6772696400000000ull ^ seed);
     std::vector<float> w;
     init_mlp(w, seed);
     std::vector<float> zeros(kMlpParams, 0.0f);
@@ -1212,11 +1284,10 @@ snkpt_status cache_train_run(snkpt_ctx* ctx, const float* samples, uint32_t n, c
     k_mlp_train<<<chunks, 64, 0, st>>>(C.x0.as<_Float16>(), enc_stride(n), samples, n, n_dev, C.mlp16.as<_Float16>(),
                                        C.mlp16t.as<_Float16>(), C.partial.as<float>(), C.dx0.as<float>(),
                                        C.loss_part.as<float>(), hashed, ad);
-    k_grid_bwd<<<grid_for(n, 128), 128, 0, st>>>(samples, C.dx0.as<float>(), n, n_dev, C.geom,
-                                                 C.grid_grad.as<unsigned long long>(),
-                                                 C.grid_priv.as<unsigned long long>(), ad);
-    k_grid_priv_fold<<<grid_for(kPrivEntries * 2, 256), 256, 0, st>>>(C.grid_priv.as<unsigned long long>(),
-                                                                      C.grid_grad.as<unsigned long long>());
+    const BwdPlan plan = bwd_plan(C.geom);
+    k_grid_bwd<<<plan.first[kGridLevels], kBwdBlock, 0, st>>>(
+        C.pos.as<float>(), (n + 63u) & ~63u, C.dx0.as<float>(), n, n_dev, C.geom, plan,
+        C.grid_grad.as<unsigned long long>(), C.grid_priv.as<unsigned long long>(), ad);
     AdamP A;
     A.b1 = b1;
     A.b2 = b2;
@@ -1232,8 +1303,8 @@ snkpt_status cache_train_run(snkpt_ctx* ctx, const float* samples, uint32_t n, c
                                                         C.mlp16.as<_Float16>(), C.mlp16t.as<_Float16>(),
                                                         C.mlp_gradf.as<float>(), C.mlp_e32.as<float>(),
                                                         C.mlp_e16.as<_Float16>(), A, ad);
-    // grid: the fixed-point gradient is consumed (and cleared) every call; without
-    // Adam it is kept as floats so it can be read back
+    // grid: the fixed-point gradient is made anew every call; without Adam it is kept
+    // as floats so it can be read back
     float2* gout = nullptr;
     if (!apply) {
         HIPC(C.grid_gradf.reserve(kGridParams * 4));
@@ -1241,8 +1312,9 @@ snkpt_status cache_train_run(snkpt_ctx* ctx, const float* samples, uint32_t n, c
     }
     const size_t entries = (size_t)kGridLevels * kGridT;
     k_grid_adam<<<(uint32_t)((entries + 255) / 256), 256, 0, st>>>(
-        C.grid_grad.as<unsigned long long>(), C.grid32.as<float2>(), C.grid_m.as<float2>(), C.grid_v.as<float2>(),
-        C.grid16.as<__half2>(), gout, C.grid_e32.as<float2>(), C.grid_e16.as<__half2>(), C.geom, A, ad);
+        C.grid_grad.as<unsigned long long>(), C.grid_priv.as<unsigned long long>(), C.grid32.as<float2>(),
+        C.grid_m.as<float2>(), C.grid_v.as<float2>(), C.grid16.as<__half2>(), gout, C.grid_e32.as<float2>(),
+        C.grid_e16.as<__half2>(), C.geom, plan, A, ad);
     C.last_n = n;
     if (loss_out) {
         std::vector<float> lp(chunks);
