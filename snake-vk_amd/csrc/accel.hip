@@ -10,9 +10,9 @@
 //   4. radix sort      LDS-staged stable LSD sort, 4 x 8-bit digits
 //   5. k_karras        binary radix tree (Karras 2012), duplicate keys ordered by index
 //   6. k_bottom_level  boxes, SAH cost and leaf-cluster flags (clusters of <= 3 triangles),
-//                      one tree level per launch
-//   7. collapse        level-synchronous greedy collapse to BVH8 (largest-area child
-//                      expanded first), octant slot order, 8-bit quantised child boxes
+//                      one tree level per launch, the last small levels in one
+//   7. collapse        level-synchronous collapse to BVH8 by SAH costs, octant slot
+//                      order, 8-bit quantised child boxes; three launches per level
 // Every integer output and every FP32 box is reproduced bit for bit by the CPU
 // twin; allocation is by prefix sums, never by atomics, so the layout is
 // deterministic.
@@ -567,6 +567,36 @@ __global__ __launch_bounds__(kUpBlock) void k_bottom_level(BinUp U, const uint32
     }
 }
 
+// The remaining levels in one launch: one block goes on level by level over the few
+// nodes that are still live (block barriers order the levels).  A launch per level
+// costs 2-4 us even when nothing is live: 63 of them took 430 us on 1.02M triangles.
+constexpr int kRestBlock = 1024;
+__global__ __launch_bounds__(kRestBlock) void k_bottom_rest(BinUp U, uint32_t* __restrict__ live_a,
+                                                            uint32_t* __restrict__ live_b,
+                                                            const uint32_t* __restrict__ cnt_in, uint32_t levels) {
+    __shared__ uint32_t cnt;
+    uint32_t total = *cnt_in;
+    uint32_t* in = live_a;
+    uint32_t* out = live_b;
+    for (uint32_t l = 0; l < levels && total > 0u; ++l) {
+        __syncthreads();
+        if (threadIdx.x == 0) cnt = 0u;
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < total; i += kRestBlock) {
+            const uint32_t parent = U.parent_int[in[i]];
+            if (parent != kNone && atomicAdd(&U.flags[parent], 1u) != 0u) {
+                bin_node(U, parent);
+                out[atomicAdd(&cnt, 1u)] = parent;
+            }
+        }
+        __syncthreads();
+        total = cnt;
+        uint32_t* t = in;
+        in = out;
+        out = t;
+    }
+}
+
 // ------------------------------------------------------------- collapse ----
 struct BinView {
     uint32_t n, n_int;
@@ -592,177 +622,191 @@ struct BinView {
     }
 };
 
-// Children of a BVH8 node made from binary node `b`, in slot order.  Every
-// per-child array is indexed only inside fully unrolled loops, so the eight
-// candidates, their areas and centres and the 8x8 octant cost table live in
-// VGPRs (dynamically indexed private arrays go to scratch), and the two
-// children of an expanded node are fetched with independent loads.
-__device__ __forceinline__ void child_info(const BinView& bv, uint32_t t, bool& ex, float& area, float& cx,
-                                           float& cy, float& cz) {
-    const float* bx = bv.box(t);
-    float bb[6];
-#pragma unroll
-    for (int q = 0; q < 6; ++q) bb[q] = bx[q];
-    ex = bv.expandable(t);
-    area = ex ? box_area(bb) : -1.0f;
-    cx = (bb[0] + bb[3]) * 0.5f;
-    cy = (bb[1] + bb[4]) * 0.5f;
-    cz = (bb[2] + bb[5]) * 0.5f;
+// A level of BVH8 nodes: first node, nodes, first leaf triangle.
+struct LevelD {
+    uint32_t start, count, tri, pad;
+};
+constexpr uint32_t kLevelRing = 8;    // levels kept on the device
+constexpr uint32_t kLevelBatch = 4;   // levels launched between two looks at their counts
+constexpr int kExpandBlock = 256;
+constexpr uint32_t kChunk = kExpandBlock / 8;  // nodes per block and chunk
+
+// What the collapse needs of a candidate child; every load is independent, the ones
+// that only an opened candidate needs are made at once too, so that opening one
+// costs one memory latency instead of three.
+struct Child {
+    bool ex;
+    float x, y, z;      // box centre
+    uint32_t k, l, r, n;  // collapse splits, children, triangles
+};
+__device__ __forceinline__ Child child_info(const BinView& bv, uint32_t t) {
+    const float2* bx = (const float2*)bv.box(t);
+    const bool leaf = (t & kLeafTag) != 0u;
+    const uint32_t i = leaf ? 0u : t;
+    const float2 b0 = bx[0], b1 = bx[1], b2 = bx[2];
+    const uint32_t lf = bv.leafify[i];
+    const uint2 c = ((const uint2*)bv.child)[i];
+    Child o;
+    o.k = bv.dpk[i];
+    o.n = leaf ? 1u : bv.count[i];
+    o.ex = !leaf && lf == 0u;
+    o.l = c.x;
+    o.r = c.y;
+    o.x = (b0.x + b1.y) * 0.5f;
+    o.y = (b0.y + b2.x) * 0.5f;
+    o.z = (b1.x + b2.y) * 0.5f;
+    return o;
 }
 
-__global__ __launch_bounds__(128) void k_collapse_expand(BinView bv, const uint32_t* __restrict__ work,
-                                                         uint32_t level_start, uint32_t level_count,
-                                                         uint32_t* __restrict__ slot_child,
-                                                         uint32_t* __restrict__ n_int, uint32_t* __restrict__ n_tri) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= level_count) return;
-    const uint32_t b = work[level_start + i];
-    uint32_t S[8];
-    float A[8], X[8], Y[8], Z[8];
-    uint32_t em = 0;  // bit k: S[k] is expandable
-    int ns;
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-        S[k] = kNone;
-        A[k] = X[k] = Y[k] = Z[k] = 0.0f;
-    }
-    {
-        bool ex;
-        child_info(bv, b, ex, A[0], X[0], Y[0], Z[0]);
-        S[0] = b;
-        ns = 1;
-        if (ex) {
-            // the SAH collapse: the 8 slots are split between b's children as
-            // D(b, 8) chose; then the first candidate that the costs open (its
-            // slot count i > 1 after dropping the i whose cost equals i - 1's)
-            // is replaced by its left child and its right child appended, until
-            // every candidate is a leaf, a BVH8 node of its own (i = 1) or done
-            const uint32_t kb = bv.dpk[b] & 7u;
-            uint32_t I[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) I[k] = 0u;
-            uint32_t l = bv.child[2 * b], r = bv.child[2 * b + 1];
-            bool el, er;
-            child_info(bv, l, el, A[0], X[0], Y[0], Z[0]);
-            child_info(bv, r, er, A[1], X[1], Y[1], Z[1]);
-            S[0] = l;
-            S[1] = r;
-            I[0] = kb;
-            I[1] = 8u - kb;
-            em = (el ? 1u : 0u) | (er ? 2u : 0u);
+// Children of the BVH8 nodes of a level, in slot order, with each node's internal
+// children and triangles as prefix sums within its chunk (local) and the chunk's sums
+// (chunk).  Eight lanes per node: lane k holds candidate k, the two children of an
+// opened candidate are fetched by two lanes at once, and the slots are dealt out over
+// the lanes.  A level's time is one node's latency (12 levels of 1 to 90k nodes at
+// 1.02M triangles): 49 us with a thread per node and three dependent loads per opened
+// candidate, 40 with the loads made at once, 15 with a group (build of 1.02M triangles
+// 2.33, 1.75 and 1.43 ms).
+__device__ __forceinline__ uint32_t ballot8(bool x) {
+    return (uint32_t)(__ballot(x) >> (__lane_id() & 56u)) & 0xFFu;
+}
+__global__ __launch_bounds__(kExpandBlock) void k_collapse_expand(BinView bv, const uint32_t* __restrict__ work,
+                                                                  const LevelD* __restrict__ lv,
+                                                                  uint32_t* __restrict__ slot_child,
+                                                                  uint2* __restrict__ local,
+                                                                  uint2* __restrict__ chunk) {
+    __shared__ uint2 sums[kChunk];
+    const uint32_t level_start = lv->start, level_count = lv->count;
+    const uint32_t k = threadIdx.x & 7u, node = threadIdx.x >> 3;
+    // block-uniform loop, all lanes go round together (ballots and shuffles)
+    for (uint32_t base = blockIdx.x * kChunk; base < level_count; base += gridDim.x * kChunk) {
+        const uint32_t i = base + node;
+        const bool in = i < level_count;
+        const uint32_t b = in ? work[level_start + i] : kLeafTag;
+        const Child root = child_info(bv, b);
+        // lane k's candidate: S its binary node; may it open, into `it` slots, kk of them left
+        uint32_t S = kNone, L = 0, R = 0, N = 0, it = 0, kk = 0;
+        bool ex = false, open = false;
+        float X = 0.0f, Y = 0.0f, Z = 0.0f;
+        // a candidate with `slots` slots: i drops while its cost equals i - 1's
+        auto take = [&](uint32_t t, uint32_t slots) {
+            const Child c = child_info(bv, t);
+            S = t, L = c.l, R = c.r, N = c.n, ex = c.ex, X = c.x, Y = c.y, Z = c.z;
+            it = slots;
+            while (it > 1u && ((c.k >> (3u * (it - 1u))) & 7u) == 0u) --it;
+            open = ex && it > 1u;
+            kk = (c.k >> (3u * (it - 1u))) & 7u;
+        };
+        uint32_t ns = 1;
+        if (root.ex) {
+            // the SAH collapse: the 8 slots are split between b's children as D(b, 8)
+            // chose; then the first candidate that the costs open is replaced by its
+            // left child and its right child appended, until every candidate is a
+            // leaf, a BVH8 node of its own (i = 1) or done
+            const uint32_t kb = root.k & 7u;
+            if (k < 2u) take(k ? root.r : root.l, k ? 8u - kb : kb);
             ns = 2;
-            uint32_t done = 0;  // bit k: candidate k stays as it is
-            while (true) {
-                int cur = -1;
-#pragma unroll
-                for (int k = 7; k >= 0; --k)
-                    if (k < ns && !((done >> k) & 1u)) cur = k;
-                if (cur < 0) break;
-                uint32_t x = 0, i = 0;
-                bool xe = false;
-#pragma unroll
-                for (int k = 0; k < 8; ++k)
-                    if (k == cur) {
-                        x = S[k];
-                        i = I[k];
-                        xe = (em >> k) & 1u;
-                    }
-                if (!xe) {
-                    done |= 1u << cur;
-                    continue;
-                }
-                const uint32_t kx = bv.dpk[x];
-                while (i > 1u && ((kx >> (3u * (i - 1u))) & 7u) == 0u) --i;
-                if (i == 1u) {
-                    done |= 1u << cur;
-                    continue;
-                }
-                const uint32_t kk = (kx >> (3u * (i - 1u))) & 7u;
-                const uint32_t cl = bv.child[2 * x], cr = bv.child[2 * x + 1];
-                bool xl, xr;
-                float al, ar, lx, ly, lz, rx, ry, rz;
-                child_info(bv, cl, xl, al, lx, ly, lz);
-                child_info(bv, cr, xr, ar, rx, ry, rz);
-#pragma unroll
-                for (int k = 0; k < 8; ++k) {
-                    if (k == cur) {
-                        S[k] = cl;
-                        I[k] = kk;
-                        A[k] = al;
-                        X[k] = lx;
-                        Y[k] = ly;
-                        Z[k] = lz;
-                        em = (em & ~(1u << k)) | (xl ? 1u << k : 0u);
-                    }
-                    if (k == ns) {
-                        S[k] = cr;
-                        I[k] = i - kk;
-                        A[k] = ar;
-                        X[k] = rx;
-                        Y[k] = ry;
-                        Z[k] = rz;
-                        em = (em & ~(1u << k)) | (xr ? 1u << k : 0u);
-                    }
-                }
-                ++ns;
-            }
+        } else if (k == 0u) {
+            S = b, N = root.n, X = root.x, Y = root.y, Z = root.z;
         }
-    }
-    // octant slot assignment: greedy on cost[c][s] = sum_a (+-1)(centre_c - centre_node)_a
-    const float* nb = bv.box(b);
-    const float nc0 = (nb[0] + nb[3]) * 0.5f, nc1 = (nb[1] + nb[4]) * 0.5f, nc2 = (nb[2] + nb[5]) * 0.5f;
-    float cost[8][8];
+        while (true) {
+            const uint32_t om = ballot8(open);
+            if (__ballot(open) == 0ull) break;
+            const uint32_t cur = om ? (uint32_t)__builtin_ctz(om) : 0u;
+            const uint32_t cr = __shfl(R, cur, 8), ci = __shfl(it, cur, 8), ck = __shfl(kk, cur, 8);
+            if (om && (k == cur || k == ns)) take(k == cur ? L : cr, k == cur ? ck : ci - ck);
+            if (om) ++ns;
+        }
+        // octant slot assignment: greedy on cost[c][s] = sum_a (+-1)(centre_c - centre_node)_a,
+        // the largest first, ties to the lower child, then the lower slot
+        float cost[8];
+        const float dx = X - root.x, dy = Y - root.y, dz = Z - root.z;
 #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        const float dx = X[c] - nc0, dy = Y[c] - nc1, dz = Z[c] - nc2;
+        for (int s = 0; s < 8; ++s) cost[s] = ((s & 1 ? dx : -dx) + (s & 2 ? dy : -dy)) + (s & 4 ? dz : -dz);
+        uint32_t slot_used = 0, child_used = 0, mine = kNone;
+        for (uint32_t r = 0; r < 8u; ++r) {
+            if (__ballot(r < ns) == 0ull) break;
+            const uint32_t free = ~slot_used & 0xFFu;
+            float v = -__builtin_inff();
+            uint32_t who = 8u * k + (uint32_t)__builtin_ctz(free | 0x100u);
 #pragma unroll
-        for (int s = 0; s < 8; ++s) cost[c][s] = ((s & 1 ? dx : -dx) + (s & 2 ? dy : -dy)) + (s & 4 ? dz : -dz);
-    }
-    uint32_t slot_used = 0, child_used = 0;
-    uint32_t slots[8];
+            for (int s = 0; s < 8; ++s)
+                if (((free >> s) & 1u) && cost[s] > v) {
+                    v = cost[s];
+                    who = 8u * k + (uint32_t)s;
+                }
+            if (k >= ns || ((child_used >> k) & 1u)) {
+                v = -__builtin_inff();
+                who = 64u + k;  // after every candidate
+            }
 #pragma unroll
-    for (int s = 0; s < 8; ++s) slots[s] = kNone;
-    for (int r = 0; r < ns; ++r) {
-        int bc = -1, bs = -1;
-        float bval = 0.0f;
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            if (c >= ns || (child_used & (1u << c))) continue;
-#pragma unroll
-            for (int s = 0; s < 8; ++s) {
-                if (slot_used & (1u << s)) continue;
-                if (bc < 0 || cost[c][s] > bval) {
-                    bval = cost[c][s];
-                    bc = c;
-                    bs = s;
+            for (int o = 1; o < 8; o <<= 1) {
+                const float ov = __shfl_xor(v, o, 64);
+                const uint32_t ow = __shfl_xor(who, o, 64);
+                if (ov > v || (ov == v && ow < who)) {
+                    v = ov;
+                    who = ow;
                 }
             }
+            const uint32_t bc = (who >> 3) & 7u, bs = who & 7u;
+            const uint32_t chosen = __shfl(S, bc, 8);
+            if (r < ns) {
+                child_used |= 1u << bc;
+                slot_used |= 1u << bs;
+                if (k == bs) mine = chosen;
+            }
         }
-        child_used |= 1u << bc;
-        slot_used |= 1u << bs;
-        uint32_t chosen = kNone;
+        const uint32_t ni = (uint32_t)__builtin_popcount(ballot8(ex && k < ns));
+        uint32_t nt = k < ns && !ex ? N : 0u;
 #pragma unroll
-        for (int c = 0; c < 8; ++c)
-            if (c == bc) chosen = S[c];
+        for (int o = 1; o < 8; o <<= 1) nt += __shfl_xor(nt, o, 64);
+        if (in) slot_child[8 * (size_t)i + k] = mine;
+        if (k == 0u) sums[node] = in ? make_uint2(ni, nt) : make_uint2(0u, 0u);
+        __syncthreads();
+        // exclusive prefix sums over the chunk
+        if (threadIdx.x < kChunk) {
+            const uint2 v = sums[threadIdx.x];
+            uint2 p = v;
 #pragma unroll
-        for (int s = 0; s < 8; ++s)
-            if (s == bs) slots[s] = chosen;
-    }
-    uint32_t ni = 0, nt = 0;
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-        slot_child[8 * (size_t)i + s] = slots[s];
-        if (slots[s] == kNone) continue;
-        if (bv.expandable(slots[s]))
-            ++ni;
-        else {
-            uint32_t f, c;
-            bv.range(slots[s], f, c);
-            nt += c;
+            for (uint32_t o = 1; o < kChunk; o <<= 1) {
+                const uint32_t a = __shfl_up(p.x, o, kChunk), c = __shfl_up(p.y, o, kChunk);
+                if (threadIdx.x >= o) p = make_uint2(p.x + a, p.y + c);
+            }
+            if (base + threadIdx.x < level_count) local[base + threadIdx.x] = make_uint2(p.x - v.x, p.y - v.y);
+            if (threadIdx.x == kChunk - 1u) chunk[base / kChunk] = p;
         }
+        __syncthreads();
     }
-    n_int[i] = ni;
-    n_tri[i] = nt;
+}
+
+// Exclusive sums over the level's chunks, in place, and the next level.
+constexpr int kTopBlock = 1024;
+__global__ __launch_bounds__(kTopBlock) void k_collapse_top(const LevelD* __restrict__ lv, uint2* __restrict__ chunk,
+                                                            LevelD* __restrict__ next) {
+    __shared__ uint2 part[kTopBlock / 64];
+    const LevelD L = *lv;
+    const uint32_t n = (L.count + kChunk - 1u) / kChunk;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    uint2 run = make_uint2(0u, 0u);
+    for (uint32_t base = 0; base < n; base += kTopBlock) {
+        const uint32_t i = base + threadIdx.x;
+        const uint2 v = i < n ? chunk[i] : make_uint2(0u, 0u);
+        uint2 p = v;
+#pragma unroll
+        for (uint32_t o = 1; o < 64u; o <<= 1) {
+            const uint32_t a = __shfl_up(p.x, o, 64), c = __shfl_up(p.y, o, 64);
+            if (lane >= o) p = make_uint2(p.x + a, p.y + c);
+        }
+        if (lane == 63u) part[wave] = p;
+        __syncthreads();
+        uint2 before = run;
+        for (uint32_t w = 0; w < kTopBlock / 64; ++w) {
+            if (w < wave) before = make_uint2(before.x + part[w].x, before.y + part[w].y);
+            run = make_uint2(run.x + part[w].x, run.y + part[w].y);
+        }
+        if (i < n) chunk[i] = make_uint2(before.x + p.x - v.x, before.y + p.y - v.y);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) *next = LevelD{L.start + L.count, run.x, L.tri + run.y, 0u};
 }
 
 __device__ __forceinline__ int quant_exp(float lo, float hi) {
@@ -791,62 +835,100 @@ __device__ __forceinline__ uint32_t quant_hi(float c, float p, int e) {
     return (uint32_t)q;
 }
 
-__global__ void k_collapse_emit(BinView bv, uint32_t* __restrict__ work, uint32_t level_start,
-                                uint32_t level_count, const uint32_t* __restrict__ slot_child,
-                                const uint32_t* __restrict__ scan_int, const uint32_t* __restrict__ scan_tri,
-                                uint32_t next_level_start, uint32_t level_tri_start,
-                                const uint32_t* __restrict__ ids, const float4* __restrict__ world,
-                                uint4* __restrict__ nodes, float4* __restrict__ leaf) {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= level_count) return;
-    uint32_t b = work[level_start + i];
-    const float* nb = bv.box(b);
-    float p[3] = {nb[0], nb[1], nb[2]};
-    int e[3];
-    for (int a = 0; a < 3; ++a) e[a] = quant_exp(nb[a], nb[3 + a]);
-    uint32_t child_base = next_level_start + scan_int[i];
-    uint32_t tri_base = level_tri_start + scan_tri[i];
-    uint32_t imask = 0, meta[2] = {0, 0}, ql[3][2] = {{0, 0}, {0, 0}, {0, 0}}, qh[3][2] = {{0, 0}, {0, 0}, {0, 0}};
-    uint32_t ci = 0, toff = 0;
-    for (int s = 0; s < 8; ++s) {
-        uint32_t c = slot_child[8 * (size_t)i + s];
-        if (c == kNone) continue;
-        const float* cb = bv.box(c);
-        int w = s >> 2, sh = 8 * (s & 3);
-        for (int a = 0; a < 3; ++a) {
-            ql[a][w] |= quant_lo(cb[a], p[a], e[a]) << sh;
-            qh[a][w] |= quant_hi(cb[3 + a], p[a], e[a]) << sh;
-        }
-        uint32_t m;
-        if (bv.expandable(c)) {
-            imask |= 1u << s;
-            m = 0x20u | (24u + (uint32_t)s);
-            work[child_base + ci] = c;
-            ++ci;
-        } else {
-            uint32_t f, cnt;
-            bv.range(c, f, cnt);
-            uint32_t unary = (1u << cnt) - 1u;
-            m = (unary << 5) | toff;
-            for (uint32_t k = 0; k < cnt; ++k) {
-                const float4* src = world + 3 * (size_t)ids[f + k];
-                float4* dst = leaf + 3 * (size_t)(tri_base + toff + k);
-                dst[0] = src[0];
-                dst[1] = src[1];
-                dst[2] = src[2];
+// The level's nodes and their leaf triangles, eight lanes per node: lane s quantises
+// the box of slot s (FP64) and copies its triangles; the byte planes are put together
+// over the lanes (one thread per node walked its eight children in turn: 18 us per level).
+__device__ __forceinline__ uint32_t or_quad(uint32_t v) {
+    v |= (uint32_t)__shfl_xor((int)v, 1, 64);
+    return v | (uint32_t)__shfl_xor((int)v, 2, 64);
+}
+constexpr int kEmitBlock = 256;
+__global__ __launch_bounds__(kEmitBlock) void k_collapse_emit(BinView bv, uint32_t* __restrict__ work,
+                                                              const LevelD* __restrict__ lv,
+                                                              const uint32_t* __restrict__ slot_child,
+                                                              const uint2* __restrict__ local,
+                                                              const uint2* __restrict__ chunk,
+                                                              const uint32_t* __restrict__ ids,
+                                                              const float4* __restrict__ world,
+                                                              uint4* __restrict__ nodes, float4* __restrict__ leaf) {
+    const LevelD L = *lv;
+    const uint32_t s = threadIdx.x & 7u, group = threadIdx.x & 56u;
+    // all lanes of a wave go round together: the shuffles need every lane
+    for (uint32_t base = blockIdx.x * (kEmitBlock / 8); base < L.count; base += gridDim.x * (kEmitBlock / 8)) {
+        const uint32_t i = base + (threadIdx.x >> 3);
+        const bool in = i < L.count;
+        uint32_t c = kNone, b = 0;
+        uint2 pre = make_uint2(0u, 0u);
+        float p[3] = {0.0f, 0.0f, 0.0f};
+        int e[3] = {0, 0, 0};
+        if (in) {
+            b = work[L.start + i];
+            c = slot_child[8 * (size_t)i + s];
+            const uint2 lo = local[i], ch = chunk[i / kChunk];
+            pre = make_uint2(L.start + L.count + ch.x + lo.x, L.tri + ch.y + lo.y);
+            const float* nb = bv.box(b);
+            for (int a = 0; a < 3; ++a) {
+                p[a] = nb[a];
+                e[a] = quant_exp(nb[a], nb[3 + a]);
             }
-            toff += cnt;
         }
-        meta[w] |= m << sh;
+        const bool used = c != kNone;
+        const bool inner = used && bv.expandable(c);
+        uint32_t f = 0, cnt = 0;
+        if (used && !inner) bv.range(c, f, cnt);
+        // slots before this one: internal children, triangles
+        const uint32_t im = (uint32_t)(__ballot(inner) >> group) & 0xFFu;
+        uint32_t toff = cnt;
+#pragma unroll
+        for (uint32_t o = 1; o < 8u; o <<= 1) {
+            const uint32_t t = __shfl_up(toff, o, 8);
+            if (s >= o) toff += t;
+        }
+        toff -= cnt;
+        uint32_t m = 0, ql[3] = {0, 0, 0}, qh[3] = {0, 0, 0};
+        const uint32_t sh = 8u * (s & 3u);
+        if (used) {
+            const float* cb = bv.box(c);
+            for (int a = 0; a < 3; ++a) {
+                ql[a] = quant_lo(cb[a], p[a], e[a]) << sh;
+                qh[a] = quant_hi(cb[3 + a], p[a], e[a]) << sh;
+            }
+            if (inner) {
+                m = 0x20u | (24u + s);
+                work[pre.x + (uint32_t)__builtin_popcount(im & ((1u << s) - 1u))] = c;
+            } else {
+                m = (((1u << cnt) - 1u) << 5) | toff;
+                for (uint32_t k = 0; k < cnt; ++k) {
+                    const float4* src = world + 3 * (size_t)ids[f + k];
+                    float4* dst = leaf + 3 * (size_t)(pre.y + toff + k);
+                    const float4 a0 = src[0], a1 = src[1], a2 = src[2];
+                    dst[0] = a0;
+                    dst[1] = a1;
+                    dst[2] = a2;
+                }
+            }
+        }
+        m = or_quad(m << sh);
+        uint32_t hi[7];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            ql[a] = or_quad(ql[a]);
+            qh[a] = or_quad(qh[a]);
+            hi[a] = __shfl_xor(ql[a], 4, 64);
+            hi[3 + a] = __shfl_xor(qh[a], 4, 64);
+        }
+        hi[6] = __shfl_xor(m, 4, 64);
+        if (in && s == 0u) {
+            uint4* o = nodes + (size_t)(L.start + i) * kNodeWords;
+            const uint32_t ew = (uint32_t)(e[0] + 127) | ((uint32_t)(e[1] + 127) << 8) |
+                                ((uint32_t)(e[2] + 127) << 16) | (im << 24);
+            o[0] = make_uint4(__float_as_uint(p[0]), __float_as_uint(p[1]), __float_as_uint(p[2]), ew);
+            o[1] = make_uint4(pre.x, pre.y, m, hi[6]);
+            o[2] = make_uint4(ql[0], hi[0], ql[1], hi[1]);
+            o[3] = make_uint4(ql[2], hi[2], qh[0], hi[3]);
+            o[4] = make_uint4(qh[1], hi[4], qh[2], hi[5]);
+        }
     }
-    uint4* o = nodes + (size_t)(level_start + i) * kNodeWords;
-    uint32_t ew = (uint32_t)(e[0] + 127) | ((uint32_t)(e[1] + 127) << 8) | ((uint32_t)(e[2] + 127) << 16) |
-                  (imask << 24);
-    o[0] = make_uint4(__float_as_uint(p[0]), __float_as_uint(p[1]), __float_as_uint(p[2]), ew);
-    o[1] = make_uint4(child_base, tri_base, meta[0], meta[1]);
-    o[2] = make_uint4(ql[0][0], ql[0][1], ql[1][0], ql[1][1]);
-    o[3] = make_uint4(ql[2][0], ql[2][1], qh[0][0], qh[0][1]);
-    o[4] = make_uint4(qh[1][0], qh[1][1], qh[2][0], qh[2][1]);
 }
 
 inline uint32_t blocks(uint32_t n, uint32_t b) { return n == 0 ? 1 : (n + b - 1) / b; }
@@ -938,14 +1020,15 @@ snkpt_status build_accel(snkpt_ctx* ctx, hipStream_t st) {
     DeviceBuffer &keys2 = A.keys2, &ids2 = A.ids2, &hist = A.hist, &hist_scan = A.hist_scan, &sums = A.sums,
                  &bounds = A.bounds, &first = A.first, &count = A.count, &pint = A.pint, &pleaf = A.pleaf,
                  &flags = A.flags, &up_live = A.up_live, &up_cnt = A.up_cnt, &cost = A.cost, &height = A.height,
-                 &slot_child = A.slot_child, &nint = A.nint, &ntri = A.ntri, &sint = A.sint, &stri = A.stri,
+                 &slot_child = A.slot_child, &nint = A.nint,
                  &work = A.work, &totals = A.totals;
     const uint32_t nb_sort = blocks(n, kSortTile);
     HIP_CHECK(keys2.reserve(nn * 4));
     HIP_CHECK(ids2.reserve(nn * 4));
     HIP_CHECK(hist.reserve((size_t)256 * nb_sort * 4));
     HIP_CHECK(hist_scan.reserve((size_t)256 * nb_sort * 4));
-    HIP_CHECK(sums.reserve((blocks((uint32_t)std::max<size_t>(256ull * nb_sort, nn), kScanTile) + 1) * 4));
+    HIP_CHECK(sums.reserve(std::max<size_t>((blocks((uint32_t)std::max<size_t>(256ull * nb_sort, nn), kScanTile) + 1) * 4,
+                                            (size_t)blocks((uint32_t)nn + 1u, kChunk) * 8)));
     HIP_CHECK(bounds.reserve(12 * 4));
     HIP_CHECK(first.reserve(nn * 4));
     HIP_CHECK(count.reserve(nn * 4));
@@ -957,12 +1040,9 @@ snkpt_status build_accel(snkpt_ctx* ctx, hipStream_t st) {
     HIP_CHECK(cost.reserve(nn * 4));
     HIP_CHECK(height.reserve(nn * 4));
     HIP_CHECK(slot_child.reserve(nn * 32));
-    HIP_CHECK(nint.reserve(nn * 4));
-    HIP_CHECK(ntri.reserve(nn * 4));
-    HIP_CHECK(sint.reserve(nn * 4));
-    HIP_CHECK(stri.reserve(nn * 4));
+    HIP_CHECK(nint.reserve(nn * 8));
     HIP_CHECK(work.reserve((nn + 1) * 4));
-    HIP_CHECK(totals.reserve(16));
+    HIP_CHECK(totals.reserve(kLevelRing * sizeof(LevelD)));
 
     uint32_t hb[12];
     const uint32_t cus = ctx->props.multiProcessorCount > 0 ? (uint32_t)ctx->props.multiProcessorCount : 256u;
@@ -1010,39 +1090,53 @@ snkpt_status build_accel(snkpt_ctx* ctx, hipStream_t st) {
             uint32_t* live[2] = {up_live.as<uint32_t>(), up_live.as<uint32_t>() + n};
             uint32_t* cnt = up_cnt.as<uint32_t>();
             k_bottom_level<true><<<grid(0), kUpBlock, 0, st>>>(U, nullptr, nullptr, live[0], cnt);
-            for (uint32_t l = 1; l < kMaxBinLevels; ++l)
+            // launches until about n / 2^launches nodes are left for the last one
+            uint32_t l = 1;
+            for (; l < kMaxBinLevels && (n >> l) > 64u; ++l)
                 k_bottom_level<false><<<grid(l), kUpBlock, 0, st>>>(U, live[(l - 1) & 1], cnt + (l - 1),
                                                                     live[l & 1], cnt + l);
+            if (l < kMaxBinLevels)
+                k_bottom_rest<<<1, kRestBlock, 0, st>>>(U, live[(l - 1) & 1], live[l & 1], cnt + (l - 1),
+                                                        kMaxBinLevels - l);
         }
         // ---- collapse, one level per iteration
         BinView bv{n, n_int, A.bin_child.as<uint32_t>(), first.as<uint32_t>(), count.as<uint32_t>(),
                    A.bin_aabb.as<float>(), A.bin_leafify.as<uint32_t>(), A.bin_dpk.as<uint32_t>()};
         uint32_t root = n >= 2 ? 0u : kLeafTag;
         HIP_CHECK(hipMemcpyAsync(work.ptr, &root, 4, hipMemcpyHostToDevice, st));
-        uint32_t level_start = 0, level_count = 1, tri_start = 0, depth = 0;
-        while (level_count > 0) {
-            k_collapse_expand<<<blocks(level_count, 128), 128, 0, st>>>(
-                bv, work.as<uint32_t>(), level_start, level_count, slot_child.as<uint32_t>(), nint.as<uint32_t>(),
-                ntri.as<uint32_t>());
-            scan_exclusive(nint.as<uint32_t>(), sint.as<uint32_t>(), level_count, sums.as<uint32_t>(),
-                           totals.as<uint32_t>(), st);
-            scan_exclusive(ntri.as<uint32_t>(), stri.as<uint32_t>(), level_count, sums.as<uint32_t>(),
-                           totals.as<uint32_t>() + 1, st);
-            uint32_t next_start = level_start + level_count;
-            k_collapse_emit<<<blocks(level_count, 128), 128, 0, st>>>(
-                bv, work.as<uint32_t>(), level_start, level_count, slot_child.as<uint32_t>(), sint.as<uint32_t>(),
-                stri.as<uint32_t>(), next_start, tri_start, A.ids.as<uint32_t>(), A.world_tris.as<float4>(),
-                A.nodes.as<uint4>(), A.leaf_tris.as<float4>());
-            uint32_t tot[2];
-            HIP_CHECK(hipMemcpyAsync(tot, totals.ptr, 8, hipMemcpyDeviceToHost, st));
+        // level l is lv[l % kLevelRing]; the counts stay on the device, and the host looks
+        // at them once per kLevelBatch levels (an empty level's launches do nothing)
+        LevelD lv[kLevelRing] = {};
+        lv[0] = LevelD{0u, 1u, 0u, 0u};
+        LevelD* d_lv = totals.as<LevelD>();
+        HIP_CHECK(hipMemcpyAsync(d_lv, lv, sizeof(LevelD), hipMemcpyHostToDevice, st));
+        uint2 *local = nint.as<uint2>(), *chunk = sums.as<uint2>();
+        uint32_t depth = 0;
+        LevelD last = lv[0];
+        while (last.count > 0) {
+            for (uint32_t k = 0; k < kLevelBatch; ++k) {
+                const uint32_t l = depth + k;
+                const LevelD* cur = d_lv + l % kLevelRing;
+                // a level has at most 8 x the nodes of the one before, and n in all
+                const uint64_t most = std::min<uint64_t>(n, (uint64_t)last.count << std::min(3u * k, 32u));
+                const uint32_t eb = std::min(blocks((uint32_t)most, kChunk), cus * 8u);
+                k_collapse_expand<<<eb, kExpandBlock, 0, st>>>(bv, work.as<uint32_t>(), cur,
+                                                               slot_child.as<uint32_t>(), local, chunk);
+                k_collapse_top<<<1, kTopBlock, 0, st>>>(cur, chunk, d_lv + (l + 1) % kLevelRing);
+                k_collapse_emit<<<std::min(blocks((uint32_t)most, kEmitBlock / 8), cus * 16u), kEmitBlock, 0, st>>>(
+                    bv, work.as<uint32_t>(), cur, slot_child.as<uint32_t>(), local, chunk, A.ids.as<uint32_t>(),
+                    A.world_tris.as<float4>(), A.nodes.as<uint4>(), A.leaf_tris.as<float4>());
+            }
+            HIP_CHECK(hipMemcpyAsync(lv, d_lv, sizeof(lv), hipMemcpyDeviceToHost, st));
             HIP_CHECK(hipStreamSynchronize(st));
-            ++depth;
-            tri_start += tot[1];
-            level_start = next_start;
-            level_count = tot[0];
-            if (level_start + level_count > n + 1) return fail(ctx, SNKPT_ERR_CAPACITY, "BVH8 node overflow");
+            for (uint32_t k = 0; k < kLevelBatch && last.count > 0; ++k) {
+                ++depth;
+                last = lv[depth % kLevelRing];
+                if (last.start + last.count > n + 1) return fail(ctx, SNKPT_ERR_CAPACITY, "BVH8 node overflow");
+            }
         }
-        A.num_nodes = level_start;
+        const uint32_t tri_start = last.tri;
+        A.num_nodes = last.start;
         A.depth = depth;
         if (tri_start != n) return fail(ctx, SNKPT_ERR_HIP, "BVH8 collapse lost triangles");
         HIP_CHECK(hipMemcpyAsync(hb, bounds.ptr, 48, hipMemcpyDeviceToHost, st));

@@ -75,7 +75,7 @@ struct Accel {
     DeviceBuffer inst_tri_offset;  // per instance: first global triangle id (n_inst + 1 entries)
     // build scratch, kept between builds so a per-frame rebuild allocates nothing
     DeviceBuffer keys2, ids2, hist, hist_scan, sums, bounds, first, count, pint, pleaf, flags, up_live, up_cnt, cost,
-        height, slot_child, nint, ntri, sint, stri, work, totals;
+        height, slot_child, nint, work, totals;
 };
 
 // Emitter table: one entry per emissive triangle, sampled proportionally to power.
