@@ -84,8 +84,9 @@ __device__ __forceinline__ void path_vertex_surf(const SceneDev& S, const PtPara
     if (ls.ok) {
         float cs = dot(s.ns, ls.wi);
         if (cs > 0.0f && dot(s.ng, ls.wi) > 0.0f) {
-            V3 f = brdf_eval(s.m, s.ns, wo, ls.wi);
-            float w = (last || ls.delta) ? 1.0f : power_heuristic(ls.pdf, brdf_pdf(s.m, s.ns, wo, ls.wi));
+            const V3 h = brdf_half(s.m, wo, ls.wi);
+            V3 f = brdf_eval(s.m, brdf_view(s.m, s.ns, wo), s.ns, wo, ls.wi, h);
+            float w = (last || ls.delta) ? 1.0f : power_heuristic(ls.pdf, brdf_pdf(s.m, s.ns, wo, ls.wi, h));
             o.sh_c = mul(mul(thr, f), ls.le) * (cs * w / ls.pdf);
             if (o.sh_c.x > 0.0f || o.sh_c.y > 0.0f || o.sh_c.z > 0.0f) {
                 o.sh = true;
@@ -96,9 +97,10 @@ __device__ __forceinline__ void path_vertex_surf(const SceneDev& S, const PtPara
     // continuation
     V3 wi;
     if (!last && brdf_sample(s.m, s.ns, wo, ul, us1, us2, wi) && dot(s.ng, wi) > 0.0f) {
-        float pdf = brdf_pdf(s.m, s.ns, wo, wi);
+        const V3 h = brdf_half(s.m, wo, wi);
+        float pdf = brdf_pdf(s.m, s.ns, wo, wi, h);
         if (pdf > 0.0f) {
-            V3 f = brdf_eval(s.m, s.ns, wo, wi);
+            V3 f = brdf_eval(s.m, brdf_view(s.m, s.ns, wo), s.ns, wo, wi, h);
             V3 nt = mul(thr, f) * (dot(s.ns, wi) / pdf);
             bool alive = nt.x > 0.0f || nt.y > 0.0f || nt.z > 0.0f;
             if (alive && P.rr_start > 0 && bounce + 1 >= P.rr_start) {

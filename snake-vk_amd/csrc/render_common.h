@@ -75,7 +75,10 @@ __device__ __forceinline__ Surf surface_at(const SceneDev& S, V3 dir, uint32_t i
     V3 ns = V3{(m0.x * nl.x + m0.y * nl.y) + m0.z * nl.z, (m1.x * nl.x + m1.y * nl.y) + m1.z * nl.z,
                (m2.x * nl.x + m2.y * nl.y) + m2.z * nl.z};
     float l2 = dot(ns, ns);
-    ns = l2 > 1e-20f ? ns * (1.0f / sqrtf(l2)) : ng;
+    if (__builtin_expect(exact_range(l2), 1))
+        ns = l2 > 1e-20f ? ns * rcp_exact(sqrt_exact(l2)) : ng;
+    else
+        ns = l2 > 1e-20f ? ns * (1.0f / sqrtf(l2)) : ng;
     s.nraw = ns;
     if (dot(ng, dir) > 0.0f) ng = ng * -1.0f;  // face the incoming ray
     if (dot(ns, ng) < 0.0f) ns = ns * -1.0f;
@@ -107,8 +110,15 @@ __device__ __forceinline__ void shadow_segment(V3 p, V3 ng, float eps, V3 wi, fl
         return;
     }
     const V3 e = (p + wi * dist) - o;
-    const float l = sqrtf(dot(e, e));
-    d = l > 0.0f ? e * (1.0f / l) : wi;
+    const float l2 = dot(e, e);
+    float l;
+    if (__builtin_expect(exact_range(l2), 1)) {
+        l = sqrt_exact(l2);
+        d = e * rcp_exact(l);
+    } else {
+        l = sqrtf(l2);
+        d = l > 0.0f ? e * (1.0f / l) : wi;
+    }
     tmax = l * (1.0f - 1e-4f);
 }
 
@@ -139,6 +149,25 @@ __device__ __forceinline__ uint32_t emitter_record(const SceneDev& S, uint32_t e
     return e;
 }
 
+// Direction, distance and unsigned cosine at the emitter (two-sided emitters,
+// RayClosestHit.rchit:119-123) of a point at offset d, d2 = |d|^2, on a triangle
+// with normal nl, nl2 = |nl|^2; false for a point or triangle of no extent.
+__device__ __forceinline__ bool seen_from(V3 d, float d2, V3 nl, float nl2, V3& wi, float& dist, float& cosl) {
+    if (__builtin_expect(exact_range(d2) && exact_range(nl2), 1)) {
+        dist = sqrt_exact(d2);
+        wi = d * rcp_exact(dist);
+        cosl = div_exact(fabsf(dot(nl, wi)), sqrt_exact(nl2));
+        return true;
+    }
+    if (!(d2 > 0.0f)) return false;
+    dist = sqrtf(d2);
+    wi = d * (1.0f / dist);
+    const float nll = sqrtf(nl2);
+    if (!(nll > 0.0f)) return false;
+    cosl = fabsf(dot(nl, wi)) / nll;
+    return true;
+}
+
 // Power-proportional emitter choice (alias table), uniform point on it.
 __device__ __forceinline__ LightSample sample_light(const SceneDev& S, V3 p, float u0, float u1, float u2,
                                                     float u3) {
@@ -156,13 +185,9 @@ __device__ __forceinline__ LightSample sample_light(const SceneDev& S, V3 p, flo
     V3 q = A * w0 + B * w1 + C * w2;
     V3 d = q - p;
     float d2 = dot(d, d);
-    if (!(d2 > 0.0f)) return ls;
-    float dist = sqrtf(d2);
-    ls.wi = d * (1.0f / dist);
     V3 nl = cross(B - A, C - A);
-    float nll = sqrtf(dot(nl, nl));
-    if (!(nll > 0.0f)) return ls;
-    float cosl = fabsf(dot(nl, ls.wi)) / nll;  // two-sided emitters (RayClosestHit.rchit:119-123)
+    float dist, cosl;
+    if (!seen_from(d, d2, nl, dot(nl, nl), ls.wi, dist, cosl)) return ls;
     if (cosl <= 0.0f) return ls;
     ls.le = V3{info.x, info.y, info.z};
     ls.pdf = c.w * d2 / (info.w * cosl);

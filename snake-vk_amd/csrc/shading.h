@@ -21,6 +21,8 @@
 
 #include <cstdint>
 
+#include "exact_math.h"
+
 namespace snkpt {
 
 constexpr float kRefPi = 3.1415926f;  // the reference's PI (LightBuffers.glsl:29)
@@ -39,7 +41,12 @@ __device__ __host__ __forceinline__ V3 cross(V3 a, V3 b) {
     return {a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
 }
 __device__ __forceinline__ V3 normalize(V3 a) {
-    float l = sqrtf(dot(a, a));
+    const float l2 = dot(a, a);
+    if (__builtin_expect(exact_range(l2), 1)) {
+        const float l = sqrt_exact(l2), r = rcp_exact(l);
+        return V3{div_signed(a.x, l, r), div_signed(a.y, l, r), div_signed(a.z, l, r)};
+    }
+    const float l = sqrtf(l2);
     return l > 0.0f ? V3{a.x / l, a.y / l, a.z / l} : a;
 }
 __device__ __host__ __forceinline__ float luminance(V3 c) { return (0.2126f * c.x + 0.7152f * c.y) + 0.0722f * c.z; }
@@ -82,7 +89,7 @@ struct Mat {
 // Orthonormal basis around n (Duff et al. 2017).
 __device__ __forceinline__ void onb(V3 n, V3& t, V3& b) {
     float s = copysignf(1.0f, n.z);
-    float a = -1.0f / (s + n.z);
+    float a = -rcp_exact(s + n.z);  // 1 <= |s + n.z| <= 2
     float bb = n.x * n.y * a;
     t = V3{1.0f + s * n.x * n.x * a, s * bb, -s * n.x};
     b = V3{bb, s + n.y * n.y * a, -n.y};
@@ -93,48 +100,81 @@ __device__ __forceinline__ float ggx_d(float ndh, float a2) {
     return a2 / (kRefPi * d * d);
 }
 __device__ __forceinline__ float g1_schlick(float x, float k) { return x / (x * (1.0f - k) + k); }
+// g1_schlick for a cosine of unit vectors and a roughness in [0, 1]: the denominator
+// lies between 1/8 and 1
+__device__ __forceinline__ float g1_exact(float x, float k) { return div_exact(x, x * (1.0f - k) + k); }
+
+// The part of brdf_eval that depends on the surface and wo alone.
+struct BrdfView {
+    V3 f0;
+    float a2, k, nv4, g1v;
+};
+__device__ __forceinline__ BrdfView brdf_view(const Mat& m, V3 n, V3 wo) {
+    BrdfView b;
+    b.f0 = V3{0.04f + (m.albedo.x - 0.04f) * m.metallic, 0.04f + (m.albedo.y - 0.04f) * m.metallic,
+              0.04f + (m.albedo.z - 0.04f) * m.metallic};
+    const float a = m.roughness * m.roughness;
+    b.a2 = a * a;
+    const float r = m.roughness + 1.0f;
+    b.k = (r * r) / 8.0f;
+    const float nv = fmaxf(dot(n, wo), 0.0f);
+    b.nv4 = 4.0f * nv;
+    b.g1v = g1_exact(nv, b.k);
+    return b;
+}
 
 // f(wo, wi) without the cosine; n is the shading normal facing wo.
-__device__ __forceinline__ V3 brdf_eval(const Mat& m, V3 n, V3 wo, V3 wi) {
+// h = brdf_half(m, wo, wi), which brdf_pdf takes too.
+__device__ __forceinline__ V3 brdf_half(const Mat& m, V3 wo, V3 wi) {
+    return (m.flags & 2u) ? wo : normalize(wo + wi);  // the Lambert lobe has no use for it
+}
+__device__ __forceinline__ V3 brdf_eval(const Mat& m, const BrdfView& b, V3 n, V3 wo, V3 wi, V3 h) {
     if (m.flags & 2u) return m.albedo * (1.0f / kRefPi);
-    V3 f0 = V3{0.04f + (m.albedo.x - 0.04f) * m.metallic, 0.04f + (m.albedo.y - 0.04f) * m.metallic,
-               0.04f + (m.albedo.z - 0.04f) * m.metallic};
-    V3 h = normalize(wo + wi);
+    const V3 f0 = b.f0;
     float hv = fmaxf(dot(h, wo), 0.0f);
     float c1 = fminf(fmaxf(1.0f - hv, 0.0f), 1.0f), c2 = c1 * c1;
     float fw = (c2 * c2) * c1;  // pow(x, 5.0)
     V3 F = V3{f0.x + (1.0f - f0.x) * fw, f0.y + (1.0f - f0.y) * fw, f0.z + (1.0f - f0.z) * fw};
-    float a = m.roughness * m.roughness;
-    float D = ggx_d(fmaxf(dot(n, h), 0.0f), a * a);
-    float r = m.roughness + 1.0f;
-    float k = (r * r) / 8.0f;
-    float nv = fmaxf(dot(n, wo), 0.0f), nl = fmaxf(dot(n, wi), 0.0f);
-    float G = g1_schlick(nv, k) * g1_schlick(nl, k);
-    float denom = 4.0f * nv * nl + 0.0001f;
-    V3 spec = F * (D * G / denom);
+    const float ndh = fmaxf(dot(n, h), 0.0f), d = ndh * ndh * (b.a2 - 1.0f) + 1.0f, dd = kRefPi * d * d;
+    float nl = fmaxf(dot(n, wi), 0.0f);
+    const float G = b.g1v * g1_exact(nl, b.k);
+    float denom = b.nv4 * nl + 0.0001f;
+    // d is a multiple of 2^-24, so dd lies in range unless d is 0 (a mirror-like lobe
+    // hit dead centre); denom is at least 1e-4
+    float sp;
+    if (__builtin_expect(exact_range(dd), 1))
+        sp = div_exact(div_exact(b.a2, dd) * G, denom);
+    else
+        sp = b.a2 / dd * G / denom;
+    V3 spec = F * sp;
     float kdm = 1.0f - m.metallic;
     V3 diff = V3{(1.0f - F.x) * kdm * m.albedo.x, (1.0f - F.y) * kdm * m.albedo.y, (1.0f - F.z) * kdm * m.albedo.z} *
               (1.0f / kRefPi);
     return diff + spec;
 }
+__device__ __forceinline__ V3 brdf_eval(const Mat& m, V3 n, V3 wo, V3 wi) {
+    return brdf_eval(m, brdf_view(m, n, wo), n, wo, wi, brdf_half(m, wo, wi));
+}
 
 __device__ __forceinline__ float spec_prob(const Mat& m) { return (m.flags & 2u) ? 0.0f : 0.5f + 0.5f * m.metallic; }
 
 // Solid-angle pdf of brdf_sample producing wi.
-__device__ __forceinline__ float brdf_pdf(const Mat& m, V3 n, V3 wo, V3 wi) {
+__device__ __forceinline__ float brdf_pdf(const Mat& m, V3 n, V3 wo, V3 wi, V3 h) {
     float ci = dot(n, wi);
     if (ci <= 0.0f) return 0.0f;
     float ps = spec_prob(m);
     float pdf = (1.0f - ps) * ci * (1.0f / kPi);
     if (ps > 0.0f) {
-        V3 h = normalize(wo + wi);
         float a = m.roughness * m.roughness;
         float a2 = a * a;
         float nh = fmaxf(dot(n, h), 0.0f);
         float d = nh * nh * (a2 - 1.0f) + 1.0f;
-        float D = a2 / (kPi * d * d);
+        const float dd = kPi * d * d;
         float wh = fabsf(dot(wo, h));
-        if (wh > 0.0f) pdf += ps * D * nh / (4.0f * wh);
+        if (__builtin_expect(exact_range(dd) && wh >= 0x1p-30f, 1))
+            pdf += div_exact(ps * div_exact(a2, dd) * nh, 4.0f * wh);
+        else if (wh > 0.0f)
+            pdf += ps * (a2 / dd) * nh / (4.0f * wh);
     }
     return pdf;
 }
@@ -147,7 +187,7 @@ __device__ __forceinline__ bool brdf_sample(const Mat& m, V3 n, V3 wo, float ul,
     if (ul < ps) {
         float a = m.roughness * m.roughness;
         float a2 = a * a;
-        float c2 = (1.0f - u1) / (1.0f + (a2 - 1.0f) * u1);
+        float c2 = div_exact(1.0f - u1, 1.0f + (a2 - 1.0f) * u1);  // u1 < 1: the denominator is at least a2 / 2
         float ct = sqrtf(fmaxf(c2, 0.0f)), st = sqrtf(fmaxf(1.0f - c2, 0.0f));
         float ph = 2.0f * kPi * u2;
         V3 h = t * (st * cosf(ph)) + b * (st * sinf(ph)) + n * ct;
@@ -163,7 +203,9 @@ __device__ __forceinline__ bool brdf_sample(const Mat& m, V3 n, V3 wo, float ul,
 
 __device__ __forceinline__ float power_heuristic(float a, float b) {
     float a2 = a * a, b2 = b * b;
-    return a2 + b2 > 0.0f ? a2 / (a2 + b2) : 0.0f;
+    const float s2 = a2 + b2;
+    if (__builtin_expect(exact_range(s2), 1)) return div_exact(a2, s2);
+    return s2 > 0.0f ? a2 / s2 : 0.0f;
 }
 
 }  // namespace snkpt

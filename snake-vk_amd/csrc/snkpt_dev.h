@@ -28,6 +28,8 @@
 #include <cstdint>
 #include <type_traits>
 
+#include "exact_math.h"
+
 namespace snkpt {
 
 constexpr int kNodeWords = 5;  // uint4 per BVH8 node
@@ -60,12 +62,6 @@ struct RayPre {
     __device__ __forceinline__ uint32_t par() const { return (bits >> 9) & 7u; }
 };
 
-// a where the mask's bits are set, else b.  V_BITOP3 issues in 2 cycles per wave
-// beside the other pipe; V_CNDMASK takes 4, and a run of them on one VCC measured
-// 15-22 cycles each (the near / far choice and the axis permutation are such runs).
-__device__ __forceinline__ uint32_t bit_sel(uint32_t a, uint32_t b, uint32_t m) {
-    return __builtin_amdgcn_bitop3_b32(a, b, m, 0xE4);
-}
 // x, y or z by the masks of "is x" and "is y".
 __device__ __forceinline__ float sel3(float x, float y, float z, uint32_t mx, uint32_t my) {
     return __uint_as_float(bit_sel(__float_as_uint(x), bit_sel(__float_as_uint(y), __float_as_uint(z), my), mx));
@@ -85,20 +81,6 @@ __device__ __forceinline__ uint32_t byte_mask4(uint32_t m4) {
 constexpr float kParallelEps = 1e-20f;
 __device__ __forceinline__ float safe_inv(float d) {
     return fabsf(d) < kParallelEps ? __builtin_nanf("") : 1.0f / d;
-}
-
-// 1 / d and x / d rounded as IEEE division rounds them, for 2^-60 <= |d| <= 2^60
-// and (quotient) 2^-60 <= |x| <= |d|: one Newton step on V_RCP_F32 gave the
-// correctly rounded reciprocal for each of the 2^23 mantissas, and Markstein's
-// correction then rounds the quotient correctly (no off result in 5e8 random
-// pairs).  3 + 3 instructions where the general division takes about 10.
-__device__ __forceinline__ float rcp_exact(float d) {
-    const float r = __builtin_amdgcn_rcpf(d);
-    return fmaf(fmaf(-d, r, 1.0f), r, r);
-}
-__device__ __forceinline__ float div_exact(float x, float d, float r) {
-    const float q = x * r;
-    return fmaf(fmaf(-q, d, x), r, q);
 }
 
 __device__ __forceinline__ RayPre ray_setup(const Ray& r) {
