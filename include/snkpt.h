@@ -162,8 +162,8 @@ typedef struct snkpt_settings {
                                        running mean (0 = 1); rising weights let a still-learning cache's early frames
                                        fade out of the mean */
     uint32_t tail_bounce;           /* SNKPT_MODE_PT (and the path-traced bounces of ReSTIR and G-buffer frames):
-                                       bounce from which the paths still alive run one thread per path instead of one
-                                       launch per bounce; same radiance bit for bit.  0 = chosen from the context's
+                                       bounce from which the paths still alive run to their ends in one launch instead of
+                                       one launch per bounce; same radiance bit for bit.  0 = chosen from the context's
                                        previous frame (the first bounce with at most 2^22 queued paths); >= max_depth = never */
     uint32_t reserved[1];
 } snkpt_settings;
@@ -203,7 +203,8 @@ typedef struct snkpt_accel_info {
  * snkpt_trace_counted and the extension rays of snkpt_render), [0] closest hit,
  * [1] any hit: a wave hands new rays to its idle lanes once refill_lanes of them
  * are idle, taking steps_per_check traversal steps between two such checks, with
- * blocks_per_cu resident 128-lane blocks per CU.  snkpt_build_accel picks it with
+ * blocks_per_cu pairs of waves resident per CU (launches of at most 2^17 rays use eight lanes
+ * per ray and take no shape).  snkpt_build_accel picks it with
  * an autotuner (timed on 2^20 bounce-like rays leaving the scene's triangles; kept per device,
  * stack size and scene size, so rebuilds of similar scenes reuse it) unless the
  * caller fixed it with snkpt_set_trace_tuning (NULL hands it back to the
@@ -507,7 +508,7 @@ typedef struct snkpt_batch_tuning {
     uint32_t shade_blocks_per_cu; /* persistent shade grid (256-lane blocks) = CUs x this */
     uint32_t queue_capacity;      /* paths per group of views processed together; 0 = all views at once */
     float ms_per_frame;           /* set by snkpt_batch_autotune: best measured frame time */
-    uint32_t tail_bounce;         /* bounce from which the paths still alive run one thread per path (same images
+    uint32_t tail_bounce;         /* bounce from which the paths still alive run to their ends in one launch (same images
                                      bit for bit); 0 = the frame's rr_start, 0xFFFFFFFF (or >= max_depth) = never */
     uint32_t reserved[2];
 } snkpt_batch_tuning;

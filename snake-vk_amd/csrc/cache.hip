@@ -8,8 +8,8 @@
 // D[4(l/16) .. 4(l/16)+3][l%16].
 //
 // Determinism: MLP weight gradients are written as per-wave partials and summed
-// in a fixed order; hash-grid gradients are accumulated with 64-bit fixed-point
-// integer atomics (order independent).  Same seed -> same bits.
+// in a fixed order; hash-grid gradients are sums of 64-bit fixed-point integers
+// (order independent).  Same seed -> same bits.
 #include <hip/hip_fp16.h>
 
 #include <algorithm>

@@ -31,7 +31,7 @@ struct VertexOut {
 // MIS, cache query or training record, NEE (power-heuristic MIS against BRDF
 // sampling), BRDF continuation with Russian roulette.  Eight uniforms are
 // drawn at every non-emissive vertex whether used or not, so the wavefront
-// and the per-thread kernels consume the stream identically.  rad_now: the
+// and the path kernels consume the stream identically.  rad_now: the
 // path's radiance before this vertex (read for training records only).
 template <int KIND>
 __device__ __forceinline__ void path_vertex_surf(const SceneDev& S, const PtParams& P, const ShadeHooks& H,

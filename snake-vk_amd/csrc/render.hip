@@ -48,7 +48,7 @@ __global__ void k_set_counts(uint32_t* c, uint32_t i0, uint32_t v0, uint32_t i1,
 // the shadow rays traced in the previous bounce (count_shadow), then clear the
 // queues this bounce fills.  Counting from the queue sizes keeps per-wave
 // statistics atomics out of the shade kernel.  The queue length of bounce
-// b < kQueueHist goes to stats[kQueueHistAt + b] (the per-thread tail's choice).
+// b < kQueueHist goes to stats[kQueueHistAt + b] (the tail's choice).
 constexpr uint32_t kQueueHist = 16, kQueueHistAt = 16;
 __global__ void k_bounce_begin(uint32_t* c, uint32_t cur, uint32_t nxt, unsigned long long* stats,
                                uint32_t count_ext, uint32_t count_shadow, uint32_t bounce) {
@@ -497,7 +497,7 @@ snkpt_status pt_bounces(snkpt_ctx* ctx, const snkpt_settings* s, int cur, uint32
     float4* rad = H.rad ? H.rad : R.rad.as<float4>();
     uint32_t* counts = R.counts.as<uint32_t>();
     unsigned long long* stats = R.stats.as<unsigned long long>();
-    // bounce from which the surviving paths run one thread per path (0: never)
+    // bounce from which the surviving paths run to their ends in one launch (0: never)
     uint32_t tail_from = 0;
     if (H.kind == 0) {
         const uint32_t t = s->tail_bounce ? s->tail_bounce
