@@ -443,7 +443,9 @@ snkpt_status snkpt_cache_train(snkpt_ctx* ctx, const float* samples, uint32_t n,
 /* which: 0 MLP fp32 weights (17,408: W0..W3 64x64, W4 16x64 row-major [out][in], rows
  * 3..15 of W4 zero), 1 grid fp32 features (16 x 2^19 x 2), 2 MLP gradient of the last
  * train call, 3 grid gradient of the last train call made without Adam,
- * 4 encoded inputs of the last call (fp16, n x 64); of the last cache-mode render
+ * 4 encoded inputs (fp16, n x 64; n of the last infer or train call) as the last encoding
+ * left them, a cache-mode frame's queries included, rows past those it encoded zero;
+ * of the last cache-mode render
  * pass: 5 the queries (16 floats each, target fields unused), 6 their records
  * (float4: throughput rgb at the query vertex, path index as uint32 bits),
  * 7 the training samples built from that pass's training paths. */

@@ -32,6 +32,7 @@ struct CacheState {
     // exponential moving averages of the weights (fp32 and the fp16 copies queries read)
     DeviceBuffer grid_e32, grid_e16, mlp_e32, mlp_e16;
     DeviceBuffer partial, loss_part, x0, pos, rows, dx0, y, mlp_red, grid_priv;  // grid_priv: dense levels' gradient copies
+    DeviceBuffer x0_is;       // Encoded: what x0 holds, written by the encoding itself
     uint32_t cap = 0;         // samples the inference work buffers hold
     uint32_t tcap = 0;        // samples the training work buffers hold
     uint32_t last_n = 0;
@@ -286,15 +287,24 @@ struct EncLevels {
     uint32_t n, l[kGridLevels];
 };
 
+// What an encoding leaves in x0: `n` queries in the layout of `stride` (0: rows of 64
+// inputs).  The kernel that encodes writes it, so that it also follows the replays of
+// a captured frame.
+struct Encoded {
+    uint32_t stride, n;
+};
+
 // The dense levels (1.2 MB of tables together) and the features that need no grid;
 // the normalised positions go to `pos` (three arrays of `stride`) for the levels' pass.
 constexpr int kEncTBlock = 256;
 __global__ __launch_bounds__(kEncTBlock) void k_encode_dense(const float* __restrict__ samples, uint32_t n,
                                                              const uint32_t* __restrict__ n_dev, uint32_t stride,
                                                              GridGeom G, EncLevels L, const __half2* __restrict__ grid,
-                                                             half2v_t* __restrict__ x0t, float* __restrict__ pos) {
+                                                             half2v_t* __restrict__ x0t, float* __restrict__ pos,
+                                                             Encoded* __restrict__ is) {
     if (n_dev) n = min(n, *n_dev);
     const uint32_t i = blockIdx.x * kEncTBlock + threadIdx.x;
+    if (is && i == 0) *is = Encoded{stride, n};
     if (i >= n) return;
     float s[kSampleFloats];
     const float4* q = (const float4*)(samples + (size_t)kSampleFloats * i);
@@ -344,8 +354,10 @@ __global__ __launch_bounds__(kEncTBlock) void k_encode_hashed(const float* __res
 __global__ __launch_bounds__(kEncBlock) void k_encode(const float* __restrict__ samples, uint32_t n,
                                                      const uint32_t* __restrict__ n_dev, GridGeom G,
                                                      const __half2* __restrict__ grid, _Float16* __restrict__ x0,
-                                                     float* __restrict__ pos, uint32_t pos_stride) {
+                                                     float* __restrict__ pos, uint32_t pos_stride,
+                                                     Encoded* __restrict__ is) {
     if (n_dev) n = min(n, *n_dev);
+    if (is && blockIdx.x == 0 && threadIdx.x == 0) *is = Encoded{0u, n};
     if (blockIdx.x * 64 >= n) return;  // the whole block is past the end
     encode_block(samples, n, G, grid, x0, pos, pos_stride);
 }
@@ -359,8 +371,9 @@ inline uint32_t enc_stride(uint32_t n) { return n <= kEncSmall ? 0u : (n + 63u) 
 // Encodes n queries (min(n, *n_dev) with n_dev) into x0t in the layout of
 // enc_stride(n).  pos: receives the normalised positions, three arrays of n rounded up
 // to 64 (null: a large call reads the samples' positions once per level instead).
+// is: receives what x0t then holds (null: not asked for).
 void encode_queries(const float* samples, uint32_t n, const uint32_t* n_dev, const GridGeom& G, const __half2* grid,
-                    _Float16* x0t, float* pos, hipStream_t st) {
+                    _Float16* x0t, float* pos, Encoded* is, hipStream_t st) {
     if (n == 0) return;
     EncLevels d{0, {}}, h{0, {}};
     for (int l = 0; l < kGridLevels; ++l) {
@@ -369,19 +382,26 @@ void encode_queries(const float* samples, uint32_t n, const uint32_t* n_dev, con
     }
     const uint32_t blocks = (n + kEncTBlock - 1) / kEncTBlock, stride = enc_stride(n);
     if (!stride) {
-        k_encode<<<(n + 63) / 64, kEncBlock, 0, st>>>(samples, n, n_dev, G, grid, x0t, pos, (n + 63u) & ~63u);
+        k_encode<<<(n + 63) / 64, kEncBlock, 0, st>>>(samples, n, n_dev, G, grid, x0t, pos, (n + 63u) & ~63u, is);
         return;
     }
-    k_encode_dense<<<blocks, kEncTBlock, 0, st>>>(samples, n, n_dev, stride, G, d, grid, (half2v_t*)x0t, pos);
+    k_encode_dense<<<blocks, kEncTBlock, 0, st>>>(samples, n, n_dev, stride, G, d, grid, (half2v_t*)x0t, pos, is);
     if (h.n)
         k_encode_hashed<<<dim3(blocks, h.n), kEncTBlock, 0, st>>>(samples, pos, n, n_dev, stride, G, h, grid,
                                                                   (half2v_t*)x0t);
 }
 
-// Rows of 64 inputs per query from the encoded queries (for reading them back).
-__global__ void k_rows_of(const half2v_t* __restrict__ x0t, uint32_t n, uint32_t stride, half2v_t* __restrict__ rows) {
+// Rows of 64 inputs of the first n queries of x0 (for reading them back); zero past
+// the queries it holds.  cap: queries the buffer has room for.
+__global__ void k_rows_of(const half2v_t* __restrict__ x0, const Encoded* __restrict__ is, uint32_t cap, uint32_t n,
+                          half2v_t* __restrict__ rows) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, r = blockIdx.y;
-    if (i < n) rows[(size_t)32 * i + r] = x0t[(size_t)r * stride + i];
+    if (i >= n) return;
+    const Encoded e = *is;
+    half2v_t v = to_half2v(0.0f, 0.0f);
+    if (i < min(e.n, cap) && e.stride <= cap)
+        v = e.stride ? x0[(size_t)r * e.stride + i] : x0[(size_t)32 * i + r];
+    rows[(size_t)32 * i + r] = v;
 }
 
 inline uint32_t enc_blocks(uint32_t n) { return n == 0 ? 1u : (n + 63) / 64; }
@@ -1160,6 +1180,10 @@ snkpt_status cache_reset(snkpt_ctx* ctx, uint32_t seed, const float* lo, const f
     HIPC(C.mlp_e32.reserve(kMlpParams * 4));
     HIPC(C.mlp_e16.reserve(kMlpParams * 2));
     HIPC(sync_ema(C, st));
+    if (!C.x0_is.ptr) {
+        HIPC(C.x0_is.reserve(sizeof(Encoded)));
+        HIPC(hipMemsetAsync(C.x0_is.ptr, 0, sizeof(Encoded), st));
+    }
     HIPC(C.adam.reserve(sizeof(AdamDev)));
     k_adam_reset<<<1, 64, 0, st>>>(C.adam.as<AdamDev>());
     HIPC(hipStreamSynchronize(st));
@@ -1173,6 +1197,7 @@ snkpt_status cache_reset(snkpt_ctx* ctx, uint32_t seed, const float* lo, const f
 static snkpt_status ensure_work(snkpt_ctx* ctx, CacheState& C, uint32_t n, bool train) {
     const uint32_t cap = ((n + 63) / 64) * 64;
     if (cap > C.cap) {
+        C.cap = 0;  // a failed growth leaves nothing to use
         HIPC(C.x0.reserve((size_t)cap * 128));
         HIPC(C.pos.reserve((size_t)cap * 12));
         HIPC(C.y.reserve((size_t)cap * 16));
@@ -1194,7 +1219,8 @@ snkpt_status cache_infer(snkpt_ctx* ctx, const float* samples, uint32_t n, float
     if (n == 0) return SNKPT_OK;
     snkpt_status e = ensure_work(ctx, C, n, false);
     if (e != SNKPT_OK) return e;
-    encode_queries(samples, n, nullptr, C.geom, C.grid16.as<__half2>(), C.x0.as<_Float16>(), C.pos.as<float>(), st);
+    encode_queries(samples, n, nullptr, C.geom, C.grid16.as<__half2>(), C.x0.as<_Float16>(), C.pos.as<float>(),
+                   C.x0_is.as<Encoded>(), st);
     const uint32_t waves = (n + 63) / 64;
     k_mlp_infer<<<(waves + kInferWaves - 1) / kInferWaves, 64 * kInferWaves, 0, st>>>(
         C.x0.as<_Float16>(), enc_stride(n), n, nullptr, C.mlp16.as<_Float16>(), (float4*)out);
@@ -1246,7 +1272,7 @@ snkpt_status cache_infer_noalloc(snkpt_ctx* ctx, const float* samples, uint32_t 
     }
     if (!x0) return fail(ctx, SNKPT_ERR_HIP, "cache_infer_noalloc: workspace address not set up for this device");
     CacheState& C = *Cp;
-    encode_queries(samples, n, nullptr, C.geom, C.grid16.as<__half2>(), x0, nullptr, st);
+    encode_queries(samples, n, nullptr, C.geom, C.grid16.as<__half2>(), x0, nullptr, nullptr, st);
     const uint32_t waves = (n + 63) / 64;
     k_mlp_infer<<<(waves + kInferWaves - 1) / kInferWaves, 64 * kInferWaves, 0, st>>>(
         x0, enc_stride(n), n, nullptr, C.mlp16.as<_Float16>(), (float4*)out);
@@ -1277,7 +1303,8 @@ snkpt_status cache_train_run(snkpt_ctx* ctx, const float* samples, uint32_t n, c
     AdamDev* ad = C.adam.as<AdamDev>();
     k_adam_advance<<<1, 64, 0, st>>>(ad, n, n_dev, lr, ema, b1, b2, apply);
     const uint32_t chunks = (n + 63) / 64;
-    encode_queries(samples, n, n_dev, C.geom, C.grid16.as<__half2>(), C.x0.as<_Float16>(), C.pos.as<float>(), st);
+    encode_queries(samples, n, n_dev, C.geom, C.grid16.as<__half2>(), C.x0.as<_Float16>(), C.pos.as<float>(),
+                   C.x0_is.as<Encoded>(), st);
     uint32_t hashed = 0;
     for (int l = 0; l < kGridLevels; ++l)
         if (!C.geom.dense[l]) hashed |= 1u << l;
@@ -1360,19 +1387,18 @@ snkpt_status cache_params(snkpt_ctx* ctx, uint32_t which, void* dst, size_t byte
     if (!dst) return SNKPT_OK;
     if (bytes < sz) return fail(ctx, SNKPT_ERR_INVALID_ARG, "cache_params: destination too small");
     if (which == 3 && !C.grid_gradf.ptr) return fail(ctx, SNKPT_ERR_NOT_BUILT, "cache_params: no gradient-only step yet");
-    const void* src = which == 0   ? C.mlp32.ptr
+    const void* src = which == 0   ? (const void*)C.mlp32.ptr
                       : which == 1 ? C.grid32.ptr
                       : which == 2 ? C.mlp_gradf.ptr
                       : which == 3 ? C.grid_gradf.ptr
-                      : which == 4 ? C.x0.ptr
                       : which == 5 ? C.q_samples.ptr
                       : which == 6 ? C.q_meta.ptr
                                    : C.t_samples.ptr;
     if (sz == 0) return SNKPT_OK;
-    if (which == 4 && enc_stride(C.last_n)) {
+    if (which == 4) {
         HIPC(C.rows.reserve(sz));
-        k_rows_of<<<dim3((C.last_n + 255) / 256, 32), 256, 0, st>>>(C.x0.as<half2v_t>(), C.last_n,
-                                                                   enc_stride(C.last_n), C.rows.as<half2v_t>());
+        k_rows_of<<<dim3((C.last_n + 255) / 256, 32), 256, 0, st>>>(C.x0.as<half2v_t>(), C.x0_is.as<Encoded>(), C.cap,
+                                                                   C.last_n, C.rows.as<half2v_t>());
         src = C.rows.ptr;
     }
     HIPC(hipMemcpyAsync(dst, src, sz, hipMemcpyDeviceToHost, st));
@@ -1548,21 +1574,6 @@ __global__ void k_train_emit(const float* __restrict__ rec, const uint32_t* __re
 
 snkpt_status cache_ensure(snkpt_ctx* ctx, const snkpt_settings* s, hipStream_t st) {
     if (!ctx->cache || !ctx->cache->ready) return cache_reset(ctx, s->seed, nullptr, nullptr, st);
-    return SNKPT_OK;
-}
-
-// Encoding + MLP on n queries (device memory) into y; `averaged`: the weight averages.
-snkpt_status cache_query(snkpt_ctx* ctx, const float* samples, uint32_t n, float4* y, bool averaged,
-                         hipStream_t st) {
-    CacheState& C = *ctx->cache;
-    if (n == 0) return SNKPT_OK;
-    snkpt_status e = ensure_work(ctx, C, n, false);
-    if (e != SNKPT_OK) return e;
-    encode_queries(samples, n, nullptr, C.geom, (averaged ? C.grid_e16 : C.grid16).as<__half2>(),
-                   C.x0.as<_Float16>(), C.pos.as<float>(), st);
-    const uint32_t waves = (n + 63) / 64;
-    k_mlp_infer<<<(waves + kInferWaves - 1) / kInferWaves, 64 * kInferWaves, 0, st>>>(
-        C.x0.as<_Float16>(), enc_stride(n), n, nullptr, (averaged ? C.mlp_e16 : C.mlp16).as<_Float16>(), y);
     return SNKPT_OK;
 }
 
@@ -1798,7 +1809,8 @@ snkpt_status cache_pass(snkpt_ctx* ctx, const CamDev& cd, const snkpt_settings* 
     // 2. query the cache
     const bool avg = s->cache_ema > 0.0f;  // query the weight averages
     encode_queries(C.q_samples.as<float>(), n, qc, C.geom, (avg ? C.grid_e16 : C.grid16).as<__half2>(),
-                   C.x0.as<_Float16>(), C.pos.as<float>(), st);
+                   C.x0.as<_Float16>(), C.pos.as<float>(),
+                   C.x0_is.as<Encoded>(), st);
     const uint32_t waves = (n + 63) / 64;
     k_mlp_infer<<<(waves + kInferWaves - 1) / kInferWaves, 64 * kInferWaves, 0, st>>>(
         C.x0.as<_Float16>(), enc_stride(n), n, qc, (avg ? C.mlp_e16 : C.mlp16).as<_Float16>(), C.y.as<float4>());

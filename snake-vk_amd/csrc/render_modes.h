@@ -211,8 +211,6 @@ constexpr uint64_t kTrainPathsTag = 0x545241494eull;
 constexpr uint64_t kTrainTargetTag = 0x7461726765ull;
 // a cache-mode frame with these settings would allocate nothing (it may be captured)
 bool cache_capture_ready(snkpt_ctx* ctx, const snkpt_settings* s, uint32_t w, uint32_t h);
-snkpt_status cache_query(snkpt_ctx* ctx, const float* samples, uint32_t n, float4* y, bool averaged,
-                         hipStream_t st);
 // Training paths of a context enqueued on `side` (statistics kept per context),
 // then, for several contexts at once, one readback of their sample counts and
 // each one's optimiser step on `st` (their statistics added into `stats`).

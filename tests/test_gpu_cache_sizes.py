@@ -47,3 +47,55 @@ def test_encoding_matches_oracle(net):
     want = O.cache_encode(O.CacheGeom(LO, HI), grid, s[pick])
     # FP16 grid entries and an FP16 result: the tolerance of the row-wise encoding's test
     assert np.allclose(enc[pick].astype(np.float64), want, rtol=4e-3, atol=2e-3)
+
+
+@pytest.mark.parametrize("first,w,h", [(70001, 97, 53), (1000, 300, 200), (70001, 300, 200), (33000, 300, 200)])
+def test_encoded_inputs_after_a_frame(gpu, first, w, h):
+    """The encoded inputs read back after a cache frame without training are those of
+    the frame's queries whatever layout the encodings before and in the frame took, and
+    those of each replay after a captured frame's replay."""
+    import snkpt
+    import torch
+
+    from helpers import make_ctx
+    scene = snkpt.SceneData(1)
+    ctx = make_ctx(scene)
+    info = ctx.accel_info()
+    lo, hi = list(info.scene_lo), list(info.scene_hi)
+    rng = np.random.default_rng(first + w)
+    ctx.cache_reset(3, lo, hi)
+    grid = (rng.uniform(-1, 1, O.GRID_PARAMS) * 0.3).astype(np.float32)
+    ctx.cache_set_params(1, grid)
+    s = np.zeros((first, 16), np.float32)
+    s[:, 0:3] = rng.uniform(lo, hi, (first, 3))
+    s[:, 3:13] = rng.uniform(0.1, 0.9, (first, 10))
+    t = torch.from_numpy(s).cuda()
+    cam = scene.camera(0, w, h)
+    out = torch.zeros(h, w, 4, device="cuda")
+    st = snkpt.default_settings(mode=snkpt.MODE_CACHE, max_depth=4, seed=5, cache_query_depth=1,
+                                flags=snkpt.FLAG_NO_STATS | snkpt.FLAG_NO_TRAIN)
+
+    def check():
+        q = ctx.cache_params(5).reshape(-1, 16)
+        enc = ctx.cache_params(4).reshape(-1, 64).astype(np.float64)
+        assert enc.shape[0] == first and q.shape[0] > 0.3 * w * h
+        k = min(first, q.shape[0])
+        # FP16 grid entries and an FP16 result: the tolerance of the encoding's own test
+        want = O.cache_encode(O.CacheGeom(lo, hi), grid, q[:k])
+        assert np.allclose(enc[:k], want, rtol=4e-3, atol=2e-3)
+        assert not enc[q.shape[0]:].any()
+
+    ctx.cache_infer(t)
+    ctx.render(cam, st, out, w, h)
+    torch.cuda.synchronize()
+    check()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        ctx.render(cam, st, out, w, h)
+    for _ in range(2):
+        ctx.cache_infer(t)
+        enc = ctx.cache_params(4).reshape(-1, 64)[::97].astype(np.float64)
+        assert np.allclose(enc, O.cache_encode(O.CacheGeom(lo, hi), grid, s[::97]), rtol=4e-3, atol=2e-3)
+        g.replay()
+        torch.cuda.synchronize()
+        check()
