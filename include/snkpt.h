@@ -413,7 +413,8 @@ snkpt_status snkpt_oracle_accumulate(snkpt_ctx* ctx, const snkpt_camera* cam,
 /* ---- MLP radiance cache (no reference counterpart) -------------------------
  * A training / query sample is 16 floats: position[3], direction[3] (towards the
  * previous path vertex), normal[3], roughness, albedo[3], target radiance[3]
- * (ignored for queries).  Sample and output pointers are device memory.  The
+ * (ignored for queries).  Sample and output pointers are device memory; samples
+ * need a float's alignment (4 B), outputs 16 B.  The
  * cache is a 16-level hash grid (2 FP16 features, 2^19 entries per level) feeding
  * a 64-wide MLP with 4 hidden ReLU layers and 3 outputs, run on MFMA in FP16
  * with FP32 accumulation; Adam (beta 0.9 / 0.99, eps 1e-15). */

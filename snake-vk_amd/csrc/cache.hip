@@ -113,6 +113,7 @@ __device__ __forceinline__ f32x4_t mfma16(half8_t a, half8_t b, f32x4_t c) {
 
 // ------------------------------------------------------------- encoding ----
 typedef _Float16 half2v_t __attribute__((ext_vector_type(2)));
+typedef float float4_any_t __attribute__((ext_vector_type(4), aligned(4)));
 
 // Position normalised to the cache box, clamped to [0, 1].
 __device__ __forceinline__ void norm_pos(const float* s, const GridGeom& G, float p[3]) {
@@ -306,11 +307,12 @@ __global__ __launch_bounds__(kEncTBlock) void k_encode_dense(const float* __rest
     const uint32_t i = blockIdx.x * kEncTBlock + threadIdx.x;
     if (is && i == 0) *is = Encoded{stride, n};
     if (i >= n) return;
+    // 16 B loads that ask for no more than a float's alignment, which is all the caller owes
     float s[kSampleFloats];
-    const float4* q = (const float4*)(samples + (size_t)kSampleFloats * i);
+    const float4_any_t* q = (const float4_any_t*)(samples + (size_t)kSampleFloats * i);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const float4 v = q[j];
+        const float4_any_t v = q[j];
         s[4 * j] = v.x, s[4 * j + 1] = v.y, s[4 * j + 2] = v.z, s[4 * j + 3] = v.w;
     }
     float p[3];

@@ -49,6 +49,20 @@ def test_encoding_matches_oracle(net):
     assert np.allclose(enc[pick].astype(np.float64), want, rtol=4e-3, atol=2e-3)
 
 
+@pytest.mark.parametrize("n", [65, 70001])
+@pytest.mark.parametrize("shift", [1, 2, 3])
+def test_samples_need_a_floats_alignment_only(net, n, shift):
+    import torch
+    ctx, s, _, full, enc, _ = net
+    buf = torch.zeros(n * 16 + 4, device="cuda")
+    t = buf[shift:shift + n * 16].view(n, 16)
+    t.copy_(torch.from_numpy(s[:n]))
+    assert t.data_ptr() % 16 == 4 * shift
+    y = ctx.cache_infer(t).cpu().numpy()
+    assert np.array_equal(y.view(np.uint32), full[:n].view(np.uint32))
+    assert np.array_equal(ctx.cache_params(4).view(np.uint16), enc[:n].reshape(-1).view(np.uint16))
+
+
 @pytest.mark.parametrize("first,w,h", [(70001, 97, 53), (1000, 300, 200), (70001, 300, 200), (33000, 300, 200)])
 def test_encoded_inputs_after_a_frame(gpu, first, w, h):
     """The encoded inputs read back after a cache frame without training are those of
