@@ -153,12 +153,11 @@ __device__ __forceinline__ uint32_t emitter_record(const SceneDev& S, uint32_t e
 // RayClosestHit.rchit:119-123) of a point at offset d, d2 = |d|^2, on a triangle
 // with normal nl, nl2 = |nl|^2; false for a point or triangle of no extent.
 __device__ __forceinline__ bool seen_from(V3 d, float d2, V3 nl, float nl2, V3& wi, float& dist, float& cosl) {
-    if (__builtin_expect(exact_range(d2) && exact_range(nl2), 1)) {
-        dist = sqrt_exact(d2);
-        wi = d * rcp_exact(dist);
-        cosl = div_exact(fabsf(dot(nl, wi)), sqrt_exact(nl2));
-        return true;
-    }
+    dist = sqrt_exact(d2);
+    wi = d * rcp_exact(dist);
+    const float x = fabsf(dot(nl, wi));
+    cosl = div_exact(x, sqrt_exact(nl2));
+    if (__builtin_expect(exact_range(d2) & exact_range(nl2) & short_range(x), 1)) return true;
     if (!(d2 > 0.0f)) return false;
     dist = sqrtf(d2);
     wi = d * (1.0f / dist);

@@ -108,12 +108,10 @@ __device__ __forceinline__ float target_at(const GSurf& g, const BrdfView& bv, c
     if (!seen_from(d, d2, x.nl, x.nl2, wi, dist, cosl)) return 0.0f;
     float cs = dot(g.ns, wi);
     if (cs <= 0.0f || dot(g.ng, wi) <= 0.0f) return 0.0f;
-    V3 f = brdf_eval(g.m, bv, g.ns, g.wo, wi, brdf_half(g.m, g.wo, wi));
-    float geo;
-    if (__builtin_expect(exact_range(d2), 1))
-        geo = div_exact(cs * cosl, d2);
-    else
-        geo = cs * cosl / d2;
+    V3 f = brdf_eval<true>(g.m, bv, g.ns, g.wo, wi, brdf_half(g.m, g.wo, wi));
+    const float cc2 = cs * cosl;
+    float geo = div_exact(cc2, d2);
+    if (__builtin_expect(!(short_range(cc2) & short_range(d2)), 0)) geo = cc2 / d2;
     V3 cc = mul(f, x.le) * geo;
     if (c_out) *c_out = cc;
     if (wi_out) *wi_out = wi;

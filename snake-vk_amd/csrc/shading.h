@@ -42,7 +42,8 @@ __device__ __host__ __forceinline__ V3 cross(V3 a, V3 b) {
 }
 __device__ __forceinline__ V3 normalize(V3 a) {
     const float l2 = dot(a, a);
-    if (__builtin_expect(exact_range(l2), 1)) {
+    // 2^-50 <= l < 2^50, components zero or 2^-74 <= |x| <= l
+    if (__builtin_expect(exact_range(l2) & short_or_zero(a.x, a.y, a.z), 1)) {
         const float l = sqrt_exact(l2), r = rcp_exact(l);
         return V3{div_signed(a.x, l, r), div_signed(a.y, l, r), div_signed(a.z, l, r)};
     }
@@ -89,7 +90,8 @@ struct Mat {
 // Orthonormal basis around n (Duff et al. 2017).
 __device__ __forceinline__ void onb(V3 n, V3& t, V3& b) {
     float s = copysignf(1.0f, n.z);
-    float a = -rcp_exact(s + n.z);  // 1 <= |s + n.z| <= 2
+    const float sn = s + n.z;  // 1 <= |sn|; at most 2 for a unit vector
+    const float a = __builtin_expect(exact_range(fabsf(sn)), 1) ? -rcp_exact(sn) : -1.0f / sn;
     float bb = n.x * n.y * a;
     t = V3{1.0f + s * n.x * n.x * a, s * bb, -s * n.x};
     b = V3{bb, s + n.y * n.y * a, -n.y};
@@ -100,14 +102,11 @@ __device__ __forceinline__ float ggx_d(float ndh, float a2) {
     return a2 / (kRefPi * d * d);
 }
 __device__ __forceinline__ float g1_schlick(float x, float k) { return x / (x * (1.0f - k) + k); }
-// g1_schlick for a cosine of unit vectors and a roughness in [0, 1]: the denominator
-// lies between 1/8 and 1
-__device__ __forceinline__ float g1_exact(float x, float k) { return div_exact(x, x * (1.0f - k) + k); }
-
 // The part of brdf_eval that depends on the surface and wo alone.
 struct BrdfView {
     V3 f0;
     float a2, k, nv4, g1v;
+    bool shrt;  // a2 lies in short_range
 };
 __device__ __forceinline__ BrdfView brdf_view(const Mat& m, V3 n, V3 wo) {
     BrdfView b;
@@ -115,11 +114,12 @@ __device__ __forceinline__ BrdfView brdf_view(const Mat& m, V3 n, V3 wo) {
               0.04f + (m.albedo.z - 0.04f) * m.metallic};
     const float a = m.roughness * m.roughness;
     b.a2 = a * a;
+    b.shrt = short_range(b.a2);
     const float r = m.roughness + 1.0f;
     b.k = (r * r) / 8.0f;
     const float nv = fmaxf(dot(n, wo), 0.0f);
     b.nv4 = 4.0f * nv;
-    b.g1v = g1_exact(nv, b.k);
+    b.g1v = g1_schlick(nv, b.k);
     return b;
 }
 
@@ -128,6 +128,10 @@ __device__ __forceinline__ BrdfView brdf_view(const Mat& m, V3 n, V3 wo) {
 __device__ __forceinline__ V3 brdf_half(const Mat& m, V3 wo, V3 wi) {
     return (m.flags & 2u) ? wo : normalize(wo + wi);  // the Lambert lobe has no use for it
 }
+// SHORT: quotients in the short form where their operands allow it.  ReSTIR's targets
+// gain by it (a BRDF per pair of input and surface); in the path kernels the range
+// tests cost as much as the short forms save, so they divide in the general form.
+template <bool SHORT = false>
 __device__ __forceinline__ V3 brdf_eval(const Mat& m, const BrdfView& b, V3 n, V3 wo, V3 wi, V3 h) {
     if (m.flags & 2u) return m.albedo * (1.0f / kRefPi);
     const V3 f0 = b.f0;
@@ -137,15 +141,18 @@ __device__ __forceinline__ V3 brdf_eval(const Mat& m, const BrdfView& b, V3 n, V
     V3 F = V3{f0.x + (1.0f - f0.x) * fw, f0.y + (1.0f - f0.y) * fw, f0.z + (1.0f - f0.z) * fw};
     const float ndh = fmaxf(dot(n, h), 0.0f), d = ndh * ndh * (b.a2 - 1.0f) + 1.0f, dd = kRefPi * d * d;
     float nl = fmaxf(dot(n, wi), 0.0f);
-    const float G = b.g1v * g1_exact(nl, b.k);
-    float denom = b.nv4 * nl + 0.0001f;
-    // d is a multiple of 2^-24, so dd lies in range unless d is 0 (a mirror-like lobe
-    // hit dead centre); denom is at least 1e-4
-    float sp;
-    if (__builtin_expect(exact_range(dd), 1))
-        sp = div_exact(div_exact(b.a2, dd) * G, denom);
-    else
-        sp = b.a2 / dd * G / denom;
+    const float gl = nl * (1.0f - b.k) + b.k;
+    const float denom = b.nv4 * nl + 0.0001f;
+    float sp = 0.0f;
+    bool ok = false;
+    if (SHORT) {
+        // out of range: nl = 0, a mirror (a2 = 0) or its lobe hit dead centre (dd = 0), a
+        // roughness or a normal's length that no material has
+        const float DG = div_exact(b.a2, dd) * (b.g1v * div_exact(nl, gl));
+        sp = div_exact(DG, denom);
+        ok = b.shrt & short_range(dd) & short_range(nl) & short_range(gl) & short_range(DG) & short_range(denom);
+    }
+    if (__builtin_expect(!ok, !SHORT)) sp = b.a2 / dd * (b.g1v * (nl / gl)) / denom;
     V3 spec = F * sp;
     float kdm = 1.0f - m.metallic;
     V3 diff = V3{(1.0f - F.x) * kdm * m.albedo.x, (1.0f - F.y) * kdm * m.albedo.y, (1.0f - F.z) * kdm * m.albedo.z} *
@@ -171,10 +178,7 @@ __device__ __forceinline__ float brdf_pdf(const Mat& m, V3 n, V3 wo, V3 wi, V3 h
         float d = nh * nh * (a2 - 1.0f) + 1.0f;
         const float dd = kPi * d * d;
         float wh = fabsf(dot(wo, h));
-        if (__builtin_expect(exact_range(dd) && wh >= 0x1p-30f, 1))
-            pdf += div_exact(ps * div_exact(a2, dd) * nh, 4.0f * wh);
-        else if (wh > 0.0f)
-            pdf += ps * (a2 / dd) * nh / (4.0f * wh);
+        if (wh > 0.0f) pdf += ps * (a2 / dd) * nh / (4.0f * wh);
     }
     return pdf;
 }
@@ -187,7 +191,7 @@ __device__ __forceinline__ bool brdf_sample(const Mat& m, V3 n, V3 wo, float ul,
     if (ul < ps) {
         float a = m.roughness * m.roughness;
         float a2 = a * a;
-        float c2 = div_exact(1.0f - u1, 1.0f + (a2 - 1.0f) * u1);  // u1 < 1: the denominator is at least a2 / 2
+        float c2 = (1.0f - u1) / (1.0f + (a2 - 1.0f) * u1);
         float ct = sqrtf(fmaxf(c2, 0.0f)), st = sqrtf(fmaxf(1.0f - c2, 0.0f));
         float ph = 2.0f * kPi * u2;
         V3 h = t * (st * cosf(ph)) + b * (st * sinf(ph)) + n * ct;
@@ -204,7 +208,6 @@ __device__ __forceinline__ bool brdf_sample(const Mat& m, V3 n, V3 wo, float ul,
 __device__ __forceinline__ float power_heuristic(float a, float b) {
     float a2 = a * a, b2 = b * b;
     const float s2 = a2 + b2;
-    if (__builtin_expect(exact_range(s2), 1)) return div_exact(a2, s2);
     return s2 > 0.0f ? a2 / s2 : 0.0f;
 }
 

@@ -100,6 +100,7 @@ __device__ __forceinline__ RayPre ray_setup(const Ray& r) {
     }
     const float dkx = kx == 0 ? r.dx : (kx == 1 ? r.dy : r.dz);
     const float dky = ky == 0 ? r.dx : (ky == 1 ? r.dy : r.dz);
+    // quotients of at most 1 and at least 2^-120: inside what div_exact asks for
     constexpr float kLo = 0x1p-60f, kHi = 0x1p60f;
     if (fminf(fminf(ax, ay), az) >= kLo && fmaxf(fmaxf(ax, ay), az) <= kHi) {
         p.ix = rcp_exact(r.dx);

@@ -1,5 +1,6 @@
-"""GPU: the shading arithmetic's short forms (operands of ordinary size) and general
-forms (the rest) give the same bits, and so do the two register layouts of ReSTIR's
+"""GPU: frames are the same bits whether the lengths of the vertex normals take the short
+or the general root (test_gpu_exact_math.py holds each function against its general
+form), and so do the two register layouts of ReSTIR's
 spatial pass."""
 import numpy as np
 import pytest
