@@ -364,9 +364,9 @@ __global__ __launch_bounds__(kEncBlock) void k_encode(const float* __restrict__ 
     encode_block(samples, n, G, grid, x0, pos, pos_stride);
 }
 
-// Largest call encoded in one launch: queries of random points take 25 / 39 / 65 /
-// 121 us at 16k / 32k / 65k / 131k in one launch, 37 / 46 / 53 / 77 in two.
-constexpr uint32_t kEncSmall = 1u << 15;
+// Largest call encoded in one launch: calls for random points take 54 / 64 / 81 / 120 us
+// at 32k / 41k / 65k / 100k queries in one launch, 62 / 65 / 69 / 83 in two.
+constexpr uint32_t kEncSmall = 40960u;
 
 // Stride of the level-major encoding of a call for n queries; 0: rows of 64 inputs.
 inline uint32_t enc_stride(uint32_t n) { return n <= kEncSmall ? 0u : (n + 63u) & ~63u; }

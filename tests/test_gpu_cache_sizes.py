@@ -1,5 +1,5 @@
 """GPU: the cache's queries give the same bits whatever the call's size (rows of
-inputs up to 32,768 queries, level by level above), against the FP64 oracle's
+inputs up to 40,960 queries, level by level above), against the FP64 oracle's
 encoding at the line between the two and at ragged sizes."""
 import numpy as np
 import pytest
@@ -33,7 +33,7 @@ def net(gpu):
     return ctx, s, t, full, enc, grid
 
 
-@pytest.mark.parametrize("n", [1, 65, 32767, 32768, 32769, 65535, 70001])
+@pytest.mark.parametrize("n", [1, 65, 32767, 32768, 32769, 40959, 40960, 40961, 65535, 70001])
 def test_same_bits_at_every_size(net, n):
     ctx, _, t, full, enc, _ = net
     y = ctx.cache_infer(t[:n].contiguous()).cpu().numpy()
@@ -43,7 +43,7 @@ def test_same_bits_at_every_size(net, n):
 
 def test_encoding_matches_oracle(net):
     _, s, _, _, enc, grid = net
-    pick = np.r_[0:64, 32700:32800, 69900:70001]
+    pick = np.r_[0:64, 32700:32800, 40900:41000, 69900:70001]
     want = O.cache_encode(O.CacheGeom(LO, HI), grid, s[pick])
     # FP16 grid entries and an FP16 result: the tolerance of the row-wise encoding's test
     assert np.allclose(enc[pick].astype(np.float64), want, rtol=4e-3, atol=2e-3)
@@ -63,7 +63,7 @@ def test_samples_need_a_floats_alignment_only(net, n, shift):
     assert np.array_equal(ctx.cache_params(4).view(np.uint16), enc[:n].reshape(-1).view(np.uint16))
 
 
-@pytest.mark.parametrize("first,w,h", [(70001, 97, 53), (1000, 300, 200), (70001, 300, 200), (33000, 300, 200)])
+@pytest.mark.parametrize("first,w,h", [(70001, 97, 53), (1000, 300, 200), (70001, 300, 200), (41000, 300, 200)])
 def test_encoded_inputs_after_a_frame(gpu, first, w, h):
     """The encoded inputs read back after a cache frame without training are those of
     the frame's queries whatever layout the encodings before and in the frame took, and
