@@ -31,9 +31,14 @@ struct CacheState {
     DeviceBuffer mlp32, mlp16, mlp16t, mlp_m, mlp_v, mlp_gradf, grid_gradf;
     // exponential moving averages of the weights (fp32 and the fp16 copies queries read)
     DeviceBuffer grid_e32, grid_e16, mlp_e32, mlp_e16;
-    DeviceBuffer partial, loss_part, x0, pos, rows, dx0, y, mlp_red, grid_priv;  // grid_priv: dense levels' gradient copies
+    DeviceBuffer partial, loss_part, work, rows, dx0, mlp_red, grid_priv;  // grid_priv: dense levels' gradient copies
     DeviceBuffer x0_is;       // Encoded: what x0 holds, written by the encoding itself
-    uint32_t cap = 0;         // samples the inference work buffers hold
+    // One allocation (a context's first query pays for it): encoded inputs, normalised
+    // positions and network outputs of `cap` samples.
+    uint32_t cap = 0;         // multiple of 64
+    _Float16* x0() const { return work.as<_Float16>(); }
+    float* pos() const { return (float*)(work.as<uint8_t>() + (size_t)cap * 128); }
+    float4* y() const { return (float4*)(work.as<uint8_t>() + (size_t)cap * 140); }
     uint32_t tcap = 0;        // samples the training work buffers hold
     uint32_t last_n = 0;
     uint32_t t_max = 0;       // most training samples the last frame's paths may emit
@@ -1200,9 +1205,7 @@ static snkpt_status ensure_work(snkpt_ctx* ctx, CacheState& C, uint32_t n, bool 
     const uint32_t cap = ((n + 63) / 64) * 64;
     if (cap > C.cap) {
         C.cap = 0;  // a failed growth leaves nothing to use
-        HIPC(C.x0.reserve((size_t)cap * 128));
-        HIPC(C.pos.reserve((size_t)cap * 12));
-        HIPC(C.y.reserve((size_t)cap * 16));
+        HIPC(C.work.reserve((size_t)cap * (128 + 12 + 16)));
         C.cap = cap;
     }
     if (train && cap > C.tcap) {
@@ -1221,11 +1224,11 @@ snkpt_status cache_infer(snkpt_ctx* ctx, const float* samples, uint32_t n, float
     if (n == 0) return SNKPT_OK;
     snkpt_status e = ensure_work(ctx, C, n, false);
     if (e != SNKPT_OK) return e;
-    encode_queries(samples, n, nullptr, C.geom, C.grid16.as<__half2>(), C.x0.as<_Float16>(), C.pos.as<float>(),
+    encode_queries(samples, n, nullptr, C.geom, C.grid16.as<__half2>(), C.x0(), C.pos(),
                    C.x0_is.as<Encoded>(), st);
     const uint32_t waves = (n + 63) / 64;
     k_mlp_infer<<<(waves + kInferWaves - 1) / kInferWaves, 64 * kInferWaves, 0, st>>>(
-        C.x0.as<_Float16>(), enc_stride(n), n, nullptr, C.mlp16.as<_Float16>(), (float4*)out);
+        C.x0(), enc_stride(n), n, nullptr, C.mlp16.as<_Float16>(), (float4*)out);
     C.last_n = n;
     hipError_t le = hipGetLastError();
     if (le != hipSuccess) return hip_fail(ctx, le, "cache_infer launch");
@@ -1305,17 +1308,17 @@ snkpt_status cache_train_run(snkpt_ctx* ctx, const float* samples, uint32_t n, c
     AdamDev* ad = C.adam.as<AdamDev>();
     k_adam_advance<<<1, 64, 0, st>>>(ad, n, n_dev, lr, ema, b1, b2, apply);
     const uint32_t chunks = (n + 63) / 64;
-    encode_queries(samples, n, n_dev, C.geom, C.grid16.as<__half2>(), C.x0.as<_Float16>(), C.pos.as<float>(),
+    encode_queries(samples, n, n_dev, C.geom, C.grid16.as<__half2>(), C.x0(), C.pos(),
                    C.x0_is.as<Encoded>(), st);
     uint32_t hashed = 0;
     for (int l = 0; l < kGridLevels; ++l)
         if (!C.geom.dense[l]) hashed |= 1u << l;
-    k_mlp_train<<<chunks, 64, 0, st>>>(C.x0.as<_Float16>(), enc_stride(n), samples, n, n_dev, C.mlp16.as<_Float16>(),
+    k_mlp_train<<<chunks, 64, 0, st>>>(C.x0(), enc_stride(n), samples, n, n_dev, C.mlp16.as<_Float16>(),
                                        C.mlp16t.as<_Float16>(), C.partial.as<float>(), C.dx0.as<float>(),
                                        C.loss_part.as<float>(), hashed, ad);
     const BwdPlan plan = bwd_plan(C.geom);
     k_grid_bwd<<<plan.first[kGridLevels], kBwdBlock, 0, st>>>(
-        C.pos.as<float>(), (n + 63u) & ~63u, C.dx0.as<float>(), n, n_dev, C.geom, plan,
+        C.pos(), (n + 63u) & ~63u, C.dx0.as<float>(), n, n_dev, C.geom, plan,
         C.grid_grad.as<unsigned long long>(), C.grid_priv.as<unsigned long long>(), ad);
     AdamP A;
     A.b1 = b1;
@@ -1399,8 +1402,8 @@ snkpt_status cache_params(snkpt_ctx* ctx, uint32_t which, void* dst, size_t byte
     if (sz == 0) return SNKPT_OK;
     if (which == 4) {
         HIPC(C.rows.reserve(sz));
-        k_rows_of<<<dim3((C.last_n + 255) / 256, 32), 256, 0, st>>>(C.x0.as<half2v_t>(), C.x0_is.as<Encoded>(), C.cap,
-                                                                   C.last_n, C.rows.as<half2v_t>());
+        k_rows_of<<<dim3((C.last_n + 255) / 256, 32), 256, 0, st>>>((const half2v_t*)C.x0(), C.x0_is.as<Encoded>(),
+                                                                   C.cap, C.last_n, C.rows.as<half2v_t>());
         src = C.rows.ptr;
     }
     HIPC(hipMemcpyAsync(dst, src, sz, hipMemcpyDeviceToHost, st));
@@ -1811,12 +1814,11 @@ snkpt_status cache_pass(snkpt_ctx* ctx, const CamDev& cd, const snkpt_settings* 
     // 2. query the cache
     const bool avg = s->cache_ema > 0.0f;  // query the weight averages
     encode_queries(C.q_samples.as<float>(), n, qc, C.geom, (avg ? C.grid_e16 : C.grid16).as<__half2>(),
-                   C.x0.as<_Float16>(), C.pos.as<float>(),
-                   C.x0_is.as<Encoded>(), st);
+                   C.x0(), C.pos(), C.x0_is.as<Encoded>(), st);
     const uint32_t waves = (n + 63) / 64;
     k_mlp_infer<<<(waves + kInferWaves - 1) / kInferWaves, 64 * kInferWaves, 0, st>>>(
-        C.x0.as<_Float16>(), enc_stride(n), n, qc, (avg ? C.mlp_e16 : C.mlp16).as<_Float16>(), C.y.as<float4>());
-    k_cache_apply<<<grid_for(n, 256), 256, 0, st>>>(C.q_meta.as<float4>(), C.y.as<float4>(), qc, R.rad.as<float4>(),
+        C.x0(), enc_stride(n), n, qc, (avg ? C.mlp_e16 : C.mlp16).as<_Float16>(), C.y());
+    k_cache_apply<<<grid_for(n, 256), 256, 0, st>>>(C.q_meta.as<float4>(), C.y(), qc, R.rad.as<float4>(),
                                                       stats + 3);
     (void)pass;
     if (!train) return SNKPT_OK;
