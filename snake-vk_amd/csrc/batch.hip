@@ -119,10 +119,11 @@ __global__ void k_bbounce_end(uint32_t* c, unsigned long long* stats) {
 // persistent waves with ray refill.
 template <int STACK>
 __global__ __launch_bounds__(64 * kBatchWaves)
-    __attribute__((amdgpu_waves_per_eu(trace_waves_per_simd(STACK), 8))) void k_btrace(
+    __attribute__((amdgpu_waves_per_eu(trace_waves_per_simd(STACK), trace_waves_most(STACK)))) void k_btrace(
         SceneMany ss, const float4* __restrict__ org, const float4* __restrict__ dir,
         const uint32_t* __restrict__ q_path, const uint32_t* __restrict__ count, HitArrays hit) {
-    __shared__ TraceLds<STACK, kBatchWaves> lds;
+    extern __shared__ uint4 trace_mem[];
+    const TraceLds<STACK> lds(trace_mem);
     const uint32_t n = *count;
     auto load = [&](uint32_t i, Ray& ray, const uint4*& nd, const float4*& tr) {
         float4 a = org[i], d = dir[i];
@@ -298,9 +299,10 @@ __global__ void k_bq_apply(const float4* __restrict__ meta, const float4* __rest
 
 template <int STACK>
 __global__ __launch_bounds__(64 * kBatchWaves)
-    __attribute__((amdgpu_waves_per_eu(trace_waves_per_simd(STACK), 8))) void k_bshadow(
+    __attribute__((amdgpu_waves_per_eu(trace_waves_per_simd(STACK), trace_waves_most(STACK)))) void k_bshadow(
         SceneMany ss, ShadowQueue sq, const uint32_t* __restrict__ counts, float4* __restrict__ rad) {
-    __shared__ TraceLds<STACK, kBatchWaves> lds;
+    extern __shared__ uint4 trace_mem[];
+    const TraceLds<STACK> lds(trace_mem);
     const uint32_t n = counts[2];
     auto load = [&](uint32_t i, Ray& ray, const uint4*& nd, const float4*& tr) {
         ray = shadow_ray(sq, i);
@@ -536,12 +538,12 @@ void launch_traces(snkpt_batch* B, const SceneMany& ss, int cur, hipStream_t st,
         if (!shadow) {
             HitArrays hit{B->h_t.as<float>(), B->h_inst.as<uint32_t>(), B->h_prim.as<uint32_t>(),
                           B->h_u.as<float>(), B->h_v.as<float>()};
-            k_btrace<S><<<g.blocks, g.threads, 0, st>>>(ss, B->q_org[cur].as<float4>(), B->q_dir[cur].as<float4>(),
+            k_btrace<S><<<g.blocks, g.threads, g.lds, st>>>(ss, B->q_org[cur].as<float4>(), B->q_dir[cur].as<float4>(),
                                                         B->q_path[cur].as<uint32_t>(),
                                                         B->counts.as<uint32_t>() + cur, hit);
         } else {
             ShadowQueue sq{B->s_org.as<float4>(), B->s_dir.as<float4>(), B->s_contrib.as<float4>()};
-            k_bshadow<S><<<g.blocks, g.threads, 0, st>>>(ss, sq, B->counts.as<uint32_t>(), B->rad.as<float4>());
+            k_bshadow<S><<<g.blocks, g.threads, g.lds, st>>>(ss, sq, B->counts.as<uint32_t>(), B->rad.as<float4>());
         }
     });
 }

@@ -82,11 +82,12 @@ __device__ __forceinline__ void write_contact(const TravState& st, uint32_t id, 
 
 template <int STACK>
 __global__ __launch_bounds__(64 * trace_waves(STACK))
-    __attribute__((amdgpu_waves_per_eu(trace_waves_per_simd(STACK), 8))) void k_contacts(
+    __attribute__((amdgpu_waves_per_eu(trace_waves_per_simd(STACK), trace_waves_most(STACK)))) void k_contacts(
         const float4* __restrict__ org_tmin, const float4* __restrict__ dir_tmax, uint32_t n,
         const uint4* __restrict__ nodes, const float4* __restrict__ tris, ContactScene C, float timestep,
         ContactOut out, uint32_t refill) {
-    __shared__ TraceLds<STACK> lds;
+    extern __shared__ uint4 trace_mem[];
+    const TraceLds<STACK> lds(trace_mem);
     auto load = [&](uint32_t id, Ray& ray, const uint4*& nd, const float4*& tr) {
         const float4 a = org_tmin[id], d = dir_tmax[id];
         ray = Ray{a.x, a.y, a.z, a.w, d.x, d.y, d.z, d.w};
@@ -164,7 +165,7 @@ snkpt_status trace_contacts(snkpt_ctx* ctx, const float4* org_tmin, const float4
                 k_contacts_group<S><<<g.blocks, g.threads, 0, st>>>(org_tmin, dir_tmax, n, nodes, tris, C, timestep, o);
             } else {
                 const TraceGrid g = trace_grid(S, trace_waves(S), (uint32_t)cu_waves(S), cus, n);
-                k_contacts<S><<<g.blocks, g.threads, 0, st>>>(org_tmin, dir_tmax, n, nodes, tris, C, timestep, o,
+                k_contacts<S><<<g.blocks, g.threads, g.lds, st>>>(org_tmin, dir_tmax, n, nodes, tris, C, timestep, o,
                                                              refill);
             }
         });

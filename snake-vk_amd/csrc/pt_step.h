@@ -239,7 +239,7 @@ struct TailLds {
     uint32_t cursor, n_ext, n_sh;
 };
 inline TraceGrid tail_grid(int stack, uint32_t cus, uint32_t n) {
-    return TraceGrid{std::min(cus * 2u, std::max(1u, (n + 7) / 8)), (uint32_t)tail_waves(stack) * 64u};
+    return TraceGrid{std::min(cus * 2u, std::max(1u, (n + 7) / 8)), (uint32_t)tail_waves(stack) * 64u, 0u};
 }
 // Lanes of a wave with a hit to shade at which the wave stops traversing and shades
 // them: it costs about as much as three traversal steps, whatever the number of

@@ -160,10 +160,11 @@ __global__ void k_gbuf_stats(const uint32_t* c, unsigned long long* stats) {
 // Shadow rays: persistent any-hit traversal with ray refill.
 template <int STACK>
 __global__ __launch_bounds__(64 * trace_waves(STACK))
-    __attribute__((amdgpu_waves_per_eu(trace_waves_per_simd(STACK), 8))) void k_shadow(
+    __attribute__((amdgpu_waves_per_eu(trace_waves_per_simd(STACK), trace_waves_most(STACK)))) void k_shadow(
         const uint4* __restrict__ nodes, const float4* __restrict__ tris, ShadowQueue sq,
         const uint32_t* __restrict__ counts, float4* __restrict__ rad) {
-    __shared__ TraceLds<STACK> lds;
+    extern __shared__ uint4 trace_mem[];
+    const TraceLds<STACK> lds(trace_mem);
     const uint32_t nn = counts[2];
     auto load = [&](uint32_t i, Ray& ray, const uint4*& nd, const float4*& tr) {
         ray = shadow_ray(sq, i);
@@ -478,7 +479,7 @@ snkpt_status launch_shadow(snkpt_ctx* ctx, RenderState& R, float4* rad, hipStrea
             return;
         }
         const TraceGrid g = trace_grid(S, trace_waves(S), (uint32_t)cu_waves(S), cus, most);
-        k_shadow<S><<<g.blocks, g.threads, 0, st>>>(A.nodes.as<uint4>(), A.leaf_tris.as<float4>(), shadow_of(R),
+        k_shadow<S><<<g.blocks, g.threads, g.lds, st>>>(A.nodes.as<uint4>(), A.leaf_tris.as<float4>(), shadow_of(R),
                                                     R.counts.as<uint32_t>(), rad);
     });
     if (!ok) return fail(ctx, SNKPT_ERR_CAPACITY, "shadow: BVH8 deeper than the 64-entry traversal stack");

@@ -368,9 +368,9 @@ __device__ __forceinline__ TraceResult traverse(const uint4* __restrict__ nodes,
 __host__ __device__ constexpr int cu_waves(int stack) {
     return stack <= 8 ? 32 : stack <= 10 ? 28 : stack <= 12 ? 24 : stack <= 16 ? 18 : stack <= 32 ? 8 : 4;
 }
-// Waves per block, which share one ray cursor: half a CU's, so that few rays are
+// Most waves per block, which share one ray cursor: half a CU's, so that few rays are
 // left when a block's waves drain (1.24M bounce rays of 1.02M triangles: 12 waves
-// 221 us, 6: 233, 4: 243, 2: 250).  Batches take pairs: frames of several batches
+// 221 us, 6: 233, 4: 243, 2: 250; trace_grid says when it takes fewer).  Batches take pairs: frames of several batches
 // on streams of their own share a CU with finer blocks (64 views, three batches
 // at once / alone: pairs 9.41 / 11.55 ms per frame, 4 waves 9.48 / 11.58, 12 waves
 // 10.24 / 11.13).
@@ -378,7 +378,11 @@ __host__ __device__ constexpr int trace_waves(int stack) {
     return stack <= 8 ? 16 : stack <= 10 ? 14 : stack <= 12 ? 12 : stack <= 16 ? 9 : stack <= 32 ? 4 : 2;
 }
 constexpr int kBatchWaves = 2;
+constexpr uint32_t kFewWaves = 4;
+constexpr uint32_t kFewLanes = 22 * 64;
 __host__ __device__ constexpr int trace_waves_per_simd(int stack) { return stack <= 12 ? cu_waves(stack) / 4 : 1; }
+// (the LDS, which is given at the launch, bounds the waves that the compiler may plan for)
+__host__ __device__ constexpr int trace_waves_most(int stack) { return (cu_waves(stack) + 3) / 4; }
 
 // Calls f(integral_constant<int, STACK>) with the smallest stack variant that holds
 // `need` entries; false when none does.
@@ -401,27 +405,41 @@ bool with_stack(uint32_t need, F f) {
     return true;
 }
 
-// Grid of a persistent traversal launch with `waves_per_cu` waves on each of
-// `cus` CUs (capped by what resides), in blocks of w waves, for at most n rays:
-// not more blocks than groups of 8 rays.
+// Grid and LDS of a persistent traversal launch with `waves_per_cu` waves on each of
+// `cus` CUs (capped by what resides), in blocks of w waves, for at most n rays.
+// While every lane gets one ray at most, there is no cursor worth sharing: blocks of
+// up to kFewWaves waves then, no more than the rays fill, so that a launch on another
+// stream finds room beside this one (a block's LDS comes free when its last wave ends).
+// One launch / two at once, us, large blocks -> four waves: 1.02M triangles 150k rays
+// 87 / 125 -> 82 / 97, 250k 104 / 150 -> 97 / 121, 350k 119 / 169 -> 119 / 145; room 250k
+// 66 / 96 -> 61 / 76, 350k 79 / 110 -> 75 / 95, but 390k 81 / 114 -> 87 / 109: hence
+// kFewLanes.
 struct TraceGrid {
-    uint32_t blocks, threads;
+    uint32_t blocks, threads, lds;
 };
 inline TraceGrid trace_grid(int stack, int w, uint32_t waves_per_cu, uint32_t cus, uint32_t n) {
     const uint32_t most = std::min((uint32_t)cu_waves(stack), std::max(1u, waves_per_cu));
     // large blocks: two on a CU, narrower when fewer waves are asked for
-    const uint32_t waves = std::min((uint32_t)w, (most + 1) / 2);
-    const uint32_t per_cu = std::max(1u, most / waves);
-    return TraceGrid{std::min(cus * per_cu, std::max(1u, (n + 7) / 8)), waves * 64u};
+    uint32_t waves = std::min((uint32_t)w, (most + 1) / 2);
+    // not more blocks than groups of 8 rays
+    uint32_t blocks = std::max(1u, (n + 7) / 8);
+    if (n <= cus * std::min(most * 64u, kFewLanes)) {
+        waves = std::min(waves, kFewWaves);
+        blocks = std::max((n + 64u * waves - 1) / (64u * waves), std::min(cus, blocks));
+    }
+    blocks = std::min(blocks, cus * std::max(1u, most / waves));
+    return TraceGrid{blocks, waves * 64u, 16u + (uint32_t)stack * 512u * waves};
 }
 
-// LDS of a persistent traversal block: each wave's stacks (entries 64 lanes
-// apart, so lanes at equal depth hit distinct banks) and the block's ray cursor.
-template <int STACK, int W = trace_waves(STACK)>
+// LDS of a persistent traversal block (TraceGrid::lds bytes, given at the launch): the
+// block's ray cursor and each wave's stacks (entries 64 lanes apart, so lanes at equal
+// depth hit distinct banks).
+template <int STACK>
 struct TraceLds {
-    uint2 stk[STACK * 64 * W];
-    uint32_t cursor;
-    __device__ __forceinline__ uint2* lane_stack() {
+    uint32_t& cursor;
+    uint2* stk;
+    __device__ __forceinline__ explicit TraceLds(uint4* mem) : cursor(mem->x), stk((uint2*)(mem + 1)) {}
+    __device__ __forceinline__ uint2* lane_stack() const {
         return stk + (threadIdx.x >> 6) * (STACK * 64u) + (threadIdx.x & 63u);
     }
 };
@@ -483,8 +501,8 @@ __device__ __forceinline__ bool trav_steps(const uint4* __restrict__ nodes, cons
 // call per finished lane ran the hit's stores and barycentrics at 1-3 of 64
 // lanes).  Every ray's traversal is the one of traverse(), so results are
 // identical.  All threads of the block must call it.
-template <bool ANY, bool COUNT, int STACK, int STEPS, int W, class Load, class Done>
-__device__ __forceinline__ void refill_trace(uint32_t n, TraceLds<STACK, W>& lds, uint32_t refill, Load load, Done done) {
+template <bool ANY, bool COUNT, int STACK, int STEPS, class Load, class Done>
+__device__ __forceinline__ void refill_trace(uint32_t n, const TraceLds<STACK>& lds, uint32_t refill, Load load, Done done) {
     const RayShare share(n, blockIdx.x, gridDim.x);
     const uint32_t lane = __lane_id();
     const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));

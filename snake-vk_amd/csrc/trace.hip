@@ -65,13 +65,14 @@ __device__ __forceinline__ void write_hit(const TravState& st, const float4* __r
 // Persistent closest / any hit over the ray stream (see refill_trace).
 template <bool ANY, bool COUNT, int STACK, int STEPS>
 __global__ __launch_bounds__(64 * trace_waves(STACK))
-    __attribute__((amdgpu_waves_per_eu(trace_waves_per_simd(STACK), 8))) void k_trace_refill(
+    __attribute__((amdgpu_waves_per_eu(trace_waves_per_simd(STACK), trace_waves_most(STACK)))) void k_trace_refill(
         const float4* __restrict__ org_tmin, const float4* __restrict__ dir_tmax, uint32_t n,
         const uint32_t* __restrict__ count_dev, const uint4* __restrict__ nodes, const float4* __restrict__ tris,
         float* __restrict__ t_out, uint32_t* __restrict__ inst_out, uint32_t* __restrict__ prim_out,
         float* __restrict__ u_out, float* __restrict__ v_out, uint32_t* __restrict__ nvis_out,
         uint32_t* __restrict__ tvis_out, uint32_t refill) {
-    __shared__ TraceLds<STACK> lds;
+    extern __shared__ uint4 trace_mem[];
+    const TraceLds<STACK> lds(trace_mem);
     const uint32_t nn = count_dev ? *count_dev : n;
     auto load = [&](uint32_t id, Ray& ray, const uint4*& nd, const float4*& tr) {
         float4 a = org_tmin[id], d = dir_tmax[id];
@@ -133,10 +134,10 @@ void launch_stack(const TraceShape& sh, uint32_t need, uint32_t cus, hipStream_t
         constexpr int S = decltype(s)::value;
         const TraceGrid g = trace_grid(S, trace_waves(S), 2u * std::max(1u, sh.blocks_per_cu), cus, n);
         if (sh.steps == 3)
-            k_trace_refill<ANY, COUNT, S, 3><<<g.blocks, g.threads, 0, st>>>(
+            k_trace_refill<ANY, COUNT, S, 3><<<g.blocks, g.threads, g.lds, st>>>(
                 o, d, n, cnt, nodes, tris, h.t, h.inst, h.prim, h.u, h.v, nv, tv, sh.refill);
         else
-            k_trace_refill<ANY, COUNT, S, 4><<<g.blocks, g.threads, 0, st>>>(
+            k_trace_refill<ANY, COUNT, S, 4><<<g.blocks, g.threads, g.lds, st>>>(
                 o, d, n, cnt, nodes, tris, h.t, h.inst, h.prim, h.u, h.v, nv, tv, sh.refill);
     });
 }

@@ -151,7 +151,7 @@ struct GroupLds {
 };
 inline TraceGrid group_grid(uint32_t waves_per_cu, uint32_t cus, uint32_t n) {
     return TraceGrid{std::min(cus * (waves_per_cu / kGroupWaves), std::max(1u, (n + kGroupWaves - 1) / kGroupWaves)),
-                     64u * kGroupWaves};
+                     64u * kGroupWaves, 0u};
 }
 
 // refill_trace with a group per ray.  load(id, ray, nodes, tris) and done(id, state)
