@@ -245,8 +245,8 @@ inline TraceGrid tail_grid(int stack, uint32_t cus, uint32_t n) {
 // them: it costs about as much as three traversal steps, whatever the number of
 // lanes.  A quarter of the lanes where a lane sees few paths (frames of 1.02M
 // triangles and of the room at 1080p, tail from bounce 1, 16 / 32 lanes: 1.597 /
-// 1.595 and 0.986 / 0.961 ms; room at 256 x 256 and 400 x 300: 356 / 370 and 394 /
-// 409 us).  Lanes that only need their next ray started (a settled shadow ray, a
+// 1.595 and 0.986 / 0.961 ms; room at 256 x 256 and 400 x 300, measured before a thread
+// per path took such frames: 356 / 370 and 394 / 409 us).  Lanes that only need their next ray started (a settled shadow ray, a
 // path from the queue) are served from an eighth of the lanes on: waiting for the
 // shading with them took 395 us on the 256 x 256 frame, 0.99 ms on the 1080p room.
 constexpr uint32_t kServeLanes = 32;
@@ -385,6 +385,43 @@ __device__ __forceinline__ void tail_paths(const SS& ss, const PtParams& P, cons
     if (threadIdx.x == 0 && (lds.n_ext | lds.n_sh)) {
         atomicAdd(&stats[1], (unsigned long long)lds.n_ext);
         atomicAdd(&stats[2], (unsigned long long)lds.n_sh);
+    }
+}
+
+// tail_paths with each path's loop in a thread of its own, for queues that give a lane
+// about one path: no lane has another path to go on with, and the loop keeps a path's
+// state in registers (119 VGPRs, no spill) where tail_paths keeps it in memory between
+// rays.  Frames of max_depth 4, this / tail_paths, us: room at 256 x 256, 480 x 360, 512
+// x 512: 309 / 353, 371 / 419, 454 / 492; 10,000 emitters 476 / 485, 501 / 562, 636 /
+// 657; two contexts on streams of their own at 512 x 512 658 / 825 and 927 / 1,133.
+template <int STACK, int BLOCK, class SS>
+__device__ __forceinline__ void tail_paths_thread(const SS& ss, const PtParams& P, const ShadeHooks& H, const Queue& in,
+                                                  uint32_t n, const PathState& ps, float4* __restrict__ rad, uint2* stk,
+                                                  unsigned long long* __restrict__ stats, uint32_t* red) {
+    if (threadIdx.x == 0) red[0] = red[1] = 0u;
+    __syncthreads();
+    uint32_t n_ext = 0, n_sh = 0;
+    for (uint32_t i = blockIdx.x * BLOCK + threadIdx.x; i < n; i += gridDim.x * BLOCK) {
+        const uint32_t path = in.path[i];
+        const float4 o = in.org[i], d = in.dir[i];
+        const uint2 rs = ps.rng[path];
+        const Rng rng{(uint64_t)rs.x | ((uint64_t)rs.y << 32), ((uint64_t)ss.stream(path) << 1u) | 1u};
+        rad[path] = path_rest<0, STACK>(ss.at(path), P, H, path, ps.bounce[path],
+                                        Ray{o.x, o.y, o.z, o.w, d.x, d.y, d.z, d.w}, ps.thr[path], rng, stk, BLOCK,
+                                        rad[path], n_ext, n_sh);
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        n_ext += __shfl_xor(n_ext, o, 64);
+        n_sh += __shfl_xor(n_sh, o, 64);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        atomicAdd(&red[0], n_ext);
+        atomicAdd(&red[1], n_sh);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && (red[0] | red[1])) {
+        atomicAdd(&stats[1], (unsigned long long)red[0]);
+        atomicAdd(&stats[2], (unsigned long long)red[1]);
     }
 }
 

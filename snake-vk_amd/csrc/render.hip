@@ -230,13 +230,23 @@ __global__ __launch_bounds__(kMegaBlock) void k_pt_mega(SceneDev S, CamDev cam, 
     }
 }
 
-// The late bounces of the plain path tracer (tail_paths).
+// The late bounces of the plain path tracer (tail_paths, and its forms for smaller queues).
 template <int STACK>
 __global__ __launch_bounds__(64 * tail_waves(STACK)) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_pt_tail(
     SceneDev S, PtParams P, ShadeHooks H, Queue in, const uint32_t* __restrict__ count, PathState ps,
     float4* __restrict__ rad, unsigned long long* __restrict__ stats) {
     __shared__ TailLds<STACK> lds;
     tail_paths<STACK>(SceneOne{S}, P, H, in, *count, ps, rad, lds, stats);
+}
+
+template <int STACK>
+__global__ __launch_bounds__(kMegaBlock) void k_pt_tail_thread(SceneDev S, PtParams P, ShadeHooks H, Queue in,
+                                                               const uint32_t* __restrict__ count, PathState ps,
+                                                               float4* __restrict__ rad,
+                                                               unsigned long long* __restrict__ stats) {
+    __shared__ uint2 stk[STACK * kMegaBlock];
+    __shared__ uint32_t red[2];
+    tail_paths_thread<STACK, kMegaBlock>(SceneOne{S}, P, H, in, *count, ps, rad, &stk[threadIdx.x], stats, red);
 }
 
 template <int STACK>
@@ -286,6 +296,14 @@ __global__ void k_add_f64(const float4* __restrict__ rad, double* __restrict__ a
 }
 
 inline uint32_t nblk(uint32_t n, uint32_t b) { return n == 0 ? 1 : (n + b - 1) / b; }
+// Blocks per CU of the thread-per-path kernel (119 VGPRs: 4 waves per SIMD), and the most
+// queued paths per CU it takes: a quarter more than its resident lanes.  Thread per path
+// / staged lanes, us: 640 x 480 (307k paths) room 458 / 483, 10,000 emitters 651 / 665,
+// 286k triangles 795 / 756, 1.02M triangles 770 / 804, two contexts at once 633 / 828,
+// 891 / 1,099 and 1,059 / 1,393 (1.02M); 720 x 540 (389k) 501 / 507, 706 / 681, 877 / 793,
+// 829 / 847.
+constexpr uint32_t kThreadBlocksPerCu = 8;
+constexpr uint32_t kThreadPathsPerCu = 1280;
 constexpr uint32_t kTailNever = 0xFFFFFFFFu;
 // Longest queue the path kernel takes from the wavefront.  From bounce 1 on it
 // beats a launch per bounce at 65k, 1.3M and 1.9M paths (1.02M-triangle frame at
@@ -451,10 +469,16 @@ snkpt_status launch_tail(snkpt_ctx* ctx, RenderState& R, const SceneDev& S, cons
     unsigned long long* stats = R.stats.as<unsigned long long>();
     const bool ok = with_stack(need, [&](auto s) {
         constexpr int SK = decltype(s)::value;
-        if (n_max <= group_paths(std::min(A.depth, 64u))) {
+        if (n_max <= group_paths(A.depth)) {
             const TraceGrid g = group_grid(16u, cus, n_max);
             k_pt_tail_group<SK><<<g.blocks, g.threads, 0, st>>>(S, P, H, queue_of(R, cur), count, paths_of(R), rad,
                                                                 stats);
+            return;
+        }
+        if (n_max <= cus * kThreadPathsPerCu) {
+            const uint32_t grid = std::min(nblk(n_max, kMegaBlock), cus * kThreadBlocksPerCu);
+            k_pt_tail_thread<SK><<<grid, kMegaBlock, 0, st>>>(S, P, H, queue_of(R, cur), count, paths_of(R), rad,
+                                                              stats);
             return;
         }
         const TraceGrid g = tail_grid(SK, cus, n_max);

@@ -134,12 +134,16 @@ constexpr uint32_t kGroupCuWaves = 24;
 // take 17.9 / 27.5 / 71 us with groups and 34 / 38 / 50 us with a lane per ray, on
 // 1.02M triangles 14.8 us (16k) and 46.8 (262k) against 20.4 and 35.7.
 constexpr uint32_t kGroupRays = 1u << 17;
-// Largest queue whose paths run a group each, by the tree's depth (deeper trees
-// take more steps per ray, and their latency is what a group shortens): frames of
-// the room (depth 7) at 160 x 120 / 256 x 256 take 234 / 397 us with groups and 296 /
-// 356 us with lanes, 1.02M triangles (depth 12) at 160 x 120, 256 x 256, 400 x 300
-// and 640 x 480 433, 554, 722 and 1,094 us against 554, 688, 771 and 887.
-inline uint32_t group_paths(uint32_t depth) { return 1024u * depth * depth; }
+// Largest queue whose paths run a group each, by the tree's depth (deeper trees take
+// more steps per ray, and their latency is what a group shortens).  Frames with a group
+// / a thread per path, us, on both sides of the line: depth 7 (line 35,840 paths) 32k 256 /
+// 267, 50k 344 / 289; depth 8 (40,960) 32k 299 / 353, 50k 398 / 389; depth 10 (52,000)
+// 50k 458 / 459, 65k 581 / 490; depth 12 (89,856), on two scenes, 77k 555 / 624 and 592 /
+// 596, 101k 659 / 652 and 689 / 654.  Deeper trees, not measured, share depth 12's line.
+inline uint32_t group_paths(uint32_t depth) {
+    const uint32_t d = std::min(depth, 12u);
+    return std::max(5120u * d, 52u * d * d * d);
+}
 template <int STACK>
 struct GroupLds {
     uint2 stk[kGroupWaves * STACK * 64 / 8];

@@ -1,5 +1,5 @@
-"""GPU: paths run to their ends by the path kernels (a lane or a group of eight
-lanes per path, chosen by the frame's size and the tree's depth) give the frame
+"""GPU: paths run to their ends by the path kernels (a group of eight lanes per path, a
+thread per path, or lanes in stages, chosen by the frame's size and the tree's depth) give the frame
 and the ray counts of the launch-per-bounce wavefront bit for bit."""
 import numpy as np
 import pytest
@@ -8,7 +8,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("config,rr", [(1, 0), (5, 2)])
-@pytest.mark.parametrize("w,h", [(1, 1), (9, 7), (160, 120), (258, 255), (420, 301)])
+@pytest.mark.parametrize("w,h", [(1, 1), (9, 7), (160, 120), (256, 140), (256, 141), (256, 160), (256, 161),
+                                 (258, 255), (420, 301), (640, 512), (641, 512)])
 def test_path_kernels_match_wavefront(gpu, config, rr, w, h):
     import snkpt
     import torch
