@@ -203,8 +203,8 @@ typedef struct snkpt_accel_info {
  * snkpt_trace_counted and the extension rays of snkpt_render), [0] closest hit,
  * [1] any hit: a wave hands new rays to its idle lanes once refill_lanes of them
  * are idle, taking steps_per_check traversal steps between two such checks, with
- * blocks_per_cu pairs of waves resident per CU (launches of at most 2^17 rays use eight lanes
- * per ray and take no shape).  snkpt_build_accel picks it with
+ * blocks_per_cu pairs of waves resident per CU (small launches, of at most 2^17 rays, use
+ * eight lanes per ray and take no shape).  snkpt_build_accel picks it with
  * an autotuner (timed on 2^20 bounce-like rays leaving the scene's triangles; kept per device,
  * stack size and scene size, so rebuilds of similar scenes reuse it) unless the
  * caller fixed it with snkpt_set_trace_tuning (NULL hands it back to the

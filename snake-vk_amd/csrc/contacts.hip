@@ -160,7 +160,7 @@ snkpt_status trace_contacts(snkpt_ctx* ctx, const float4* org_tmin, const float4
         const ContactOut o{out.t, nrm, pos, vel, out.inst, out.prim};
         with_stack(need, [&](auto s) {
             constexpr int S = decltype(s)::value;
-            if (n <= kGroupRays) {
+            if (n <= group_rays(A.depth)) {
                 const TraceGrid g = group_grid(kGroupCuWaves, cus, n);
                 k_contacts_group<S><<<g.blocks, g.threads, 0, st>>>(org_tmin, dir_tmax, n, nodes, tris, C, timestep, o);
             } else {

@@ -496,7 +496,7 @@ snkpt_status launch_shadow(snkpt_ctx* ctx, RenderState& R, float4* rad, hipStrea
     const uint32_t most = n_max ? n_max : R.w * R.h;
     const bool ok = with_stack(need, [&](auto s) {
         constexpr int S = decltype(s)::value;
-        if (most <= kGroupRays) {
+        if (most <= group_rays(A.depth)) {
             const TraceGrid g = group_grid(kGroupCuWaves, cus, most);
             k_shadow_group<S><<<g.blocks, g.threads, 0, st>>>(A.nodes.as<uint4>(), A.leaf_tris.as<float4>(),
                                                               shadow_of(R), R.counts.as<uint32_t>(), rad);

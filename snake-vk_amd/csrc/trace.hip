@@ -287,7 +287,7 @@ snkpt_status launch_trace(snkpt_ctx* ctx, const float4* org_tmin, const float4* 
         uint32_t need = A.depth > 0 ? A.depth - 1 : 0;
         if (need > 64) return fail(ctx, SNKPT_ERR_CAPACITY, "trace: BVH8 deeper than the 64-entry traversal stack");
         bool count = node_visits || tri_visits;
-        if (!count && n <= kGroupRays) {
+        if (!count && n <= group_rays(A.depth)) {
             with_stack(need, [&](auto s) {
                 constexpr int S = decltype(s)::value;
                 const TraceGrid g = group_grid(kGroupCuWaves, ctx->props.multiProcessorCount > 0 ? (uint32_t)ctx->props.multiProcessorCount : 256u, n);

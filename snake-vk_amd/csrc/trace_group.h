@@ -130,10 +130,12 @@ __device__ __forceinline__ bool group_step(const uint4* __restrict__ nodes, cons
 // Waves per block; a small call gives each wave few rays (down to one).
 constexpr int kGroupWaves = 4;
 constexpr uint32_t kGroupCuWaves = 24;
-// Largest call with a group per ray: 16k / 65k / 262k collision rays in the room
-// take 17.9 / 27.5 / 71 us with groups and 34 / 38 / 50 us with a lane per ray, on
-// 1.02M triangles 14.8 us (16k) and 46.8 (262k) against 20.4 and 35.7.
-constexpr uint32_t kGroupRays = 1u << 17;
+// Largest call with a group per ray, by the tree's depth.  A group / a lane per ray, us
+// (closest hit; contacts): depth 7 82k 41 / 45 and 43 / 45, 98k 43 / 45 and 47 / 44, 131k
+// 51 / 45 and 56 / 43, two calls at once 72 / 56 and 79 / 54; depth 8 131k 56 / 62 and 60 /
+// 63, 197k 77 / 72 and 87 / 63; depth 10 131k 72 / 98 and 78 / 77; depth 12 131k 69 / 87
+// and 73 / 74, 164k 75 / 99 and 87 / 87, two at once 101 / 116 and 116 / 98.
+inline uint32_t group_rays(uint32_t depth) { return depth < 8u ? 81920u : 1u << 17; }
 // Largest queue whose paths run a group each, by the tree's depth (deeper trees take
 // more steps per ray, and their latency is what a group shortens).  Frames with a group
 // / a thread per path, us, on both sides of the line: depth 7 (line 35,840 paths) 32k 256 /
