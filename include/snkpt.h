@@ -507,7 +507,8 @@ snkpt_status snkpt_scene_view(uint32_t config, uint32_t view, uint32_t* out_vari
 typedef struct snkpt_batch snkpt_batch;
 typedef struct snkpt_batch_tuning {
     uint32_t trace_block;         /* lanes per traversal block: 64 or 128 (extension and shadow rays) */
-    uint32_t trace_blocks_per_cu; /* persistent traversal grid = CUs x this */
+    uint32_t trace_blocks_per_cu; /* persistent traversal grid = CUs x this, at most what resides at once (by the
+                                     stack's LDS) and what the queue fills */
     uint32_t shade_blocks_per_cu; /* persistent shade grid (256-lane blocks) = CUs x this */
     uint32_t queue_capacity;      /* paths per group of views processed together; 0 = all views at once */
     float ms_per_frame;           /* set by snkpt_batch_autotune: best measured frame time */

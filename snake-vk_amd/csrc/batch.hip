@@ -115,10 +115,13 @@ __global__ void k_bbounce_end(uint32_t* c, unsigned long long* stats) {
     }
 }
 
+// Most lanes of a traversal block (snkpt_batch_tuning.trace_block).
+constexpr uint32_t kBatchLanes = 128;
+
 // Closest hit of the queued rays, each against its own scene's BVH8:
 // persistent waves with ray refill.
 template <int STACK>
-__global__ __launch_bounds__(64 * kBatchWaves)
+__global__ __launch_bounds__(kBatchLanes)
     __attribute__((amdgpu_waves_per_eu(trace_waves_per_simd(STACK), trace_waves_most(STACK)))) void k_btrace(
         SceneMany ss, const float4* __restrict__ org, const float4* __restrict__ dir,
         const uint32_t* __restrict__ q_path, const uint32_t* __restrict__ count, HitArrays hit) {
@@ -298,7 +301,7 @@ __global__ void k_bq_apply(const float4* __restrict__ meta, const float4* __rest
 }
 
 template <int STACK>
-__global__ __launch_bounds__(64 * kBatchWaves)
+__global__ __launch_bounds__(kBatchLanes)
     __attribute__((amdgpu_waves_per_eu(trace_waves_per_simd(STACK), trace_waves_most(STACK)))) void k_bshadow(
         SceneMany ss, ShadowQueue sq, const uint32_t* __restrict__ counts, float4* __restrict__ rad) {
     extern __shared__ uint4 trace_mem[];
@@ -530,11 +533,10 @@ snkpt_status prepare(snkpt_batch* B, hipStream_t st) {
 }
 
 void launch_traces(snkpt_batch* B, const SceneMany& ss, int cur, hipStream_t st, bool shadow) {
-    // trace_block lanes x trace_blocks_per_cu blocks, as waves per CU
-    const uint32_t waves = (B->tuning.trace_block == 64 ? 1u : 2u) * std::max(1u, B->tuning.trace_blocks_per_cu);
     with_stack(B->stack, [&](auto s) {
         constexpr int S = decltype(s)::value;
-        const TraceGrid g = trace_grid(S, kBatchWaves, waves, (uint32_t)B->cus, B->cap);
+        const TraceGrid g = batch_grid(S, B->tuning.trace_block, B->tuning.trace_blocks_per_cu, (uint32_t)B->cus,
+                                       B->cap);
         if (!shadow) {
             HitArrays hit{B->h_t.as<float>(), B->h_inst.as<uint32_t>(), B->h_prim.as<uint32_t>(),
                           B->h_u.as<float>(), B->h_v.as<float>()};
@@ -1012,8 +1014,16 @@ snkpt_status batch_autotune(snkpt_batch* B, const snkpt_settings* s, hipStream_t
     const uint32_t spc[] = {2, 4, 8, 16};
     const uint64_t caps[] = {0, total / 2, total / 4};
     for (int pass = 0; pass < 2; ++pass) {
+        // (block sizes and counts that launch alike are timed once)
+        uint32_t stack = 64u;
+        with_stack(B->stack, [&](auto k) { stack = (uint32_t)decltype(k)::value; });
         for (uint32_t a : tbs)
             for (uint32_t c : tpc) {
+                const uint32_t per_cu = batch_blocks_per_cu((int)stack, a, c);
+                if (c > tpc[0] && per_cu == batch_blocks_per_cu((int)stack, a, c / 2u)) continue;
+                if (a == best.trace_block &&
+                    per_cu == batch_blocks_per_cu((int)stack, a, best.trace_blocks_per_cu))
+                    continue;
                 snkpt_batch_tuning t = best;
                 t.trace_block = a;
                 t.trace_blocks_per_cu = c;

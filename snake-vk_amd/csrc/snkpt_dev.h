@@ -370,14 +370,13 @@ __host__ __device__ constexpr int cu_waves(int stack) {
 }
 // Most waves per block, which share one ray cursor: half a CU's, so that few rays are
 // left when a block's waves drain (1.24M bounce rays of 1.02M triangles: 12 waves
-// 221 us, 6: 233, 4: 243, 2: 250; trace_grid says when it takes fewer).  Batches take pairs: frames of several batches
-// on streams of their own share a CU with finer blocks (64 views, three batches
-// at once / alone: pairs 9.41 / 11.55 ms per frame, 4 waves 9.48 / 11.58, 12 waves
-// 10.24 / 11.13).
+// 221 us, 6: 233, 4: 243, 2: 250; trace_grid says when it takes fewer).  Batches take
+// one or two (their tuning): frames of several batches on streams of their own share a
+// CU with finer blocks (64 views, three batches at once / alone: pairs 9.41 / 11.55 ms
+// per frame, 4 waves 9.48 / 11.58, 12 waves 10.24 / 11.13).
 __host__ __device__ constexpr int trace_waves(int stack) {
     return stack <= 8 ? 16 : stack <= 10 ? 14 : stack <= 12 ? 12 : stack <= 16 ? 9 : stack <= 32 ? 4 : 2;
 }
-constexpr int kBatchWaves = 2;
 constexpr uint32_t kFewWaves = 4;
 constexpr uint32_t kFewLanes = 22 * 64;
 __host__ __device__ constexpr int trace_waves_per_simd(int stack) { return stack <= 12 ? cu_waves(stack) / 4 : 1; }
@@ -429,6 +428,17 @@ inline TraceGrid trace_grid(int stack, int w, uint32_t waves_per_cu, uint32_t cu
     }
     blocks = std::min(blocks, cus * std::max(1u, most / waves));
     return TraceGrid{blocks, waves * 64u, 16u + (uint32_t)stack * 512u * waves};
+}
+
+// The same for a batch: blocks of `lanes` (64 or 128) lanes, blocks_per_cu on each CU,
+// capped by what resides and by what n rays fill.
+inline uint32_t batch_blocks_per_cu(int stack, uint32_t lanes, uint32_t blocks_per_cu) {
+    return std::min(std::max(1u, blocks_per_cu), (uint32_t)cu_waves(stack) * 64u / lanes);
+}
+inline TraceGrid batch_grid(int stack, uint32_t lanes, uint32_t blocks_per_cu, uint32_t cus, uint32_t n) {
+    const uint32_t fill = std::max(n / lanes + 1u, std::min(cus, std::max(1u, n / 8u)));
+    return TraceGrid{std::min(cus * batch_blocks_per_cu(stack, lanes, blocks_per_cu), fill), lanes,
+                     16u + (uint32_t)stack * 8u * lanes};
 }
 
 // LDS of a persistent traversal block (TraceGrid::lds bytes, given at the launch): the

@@ -39,6 +39,45 @@ def _run(tmp_path, program, args):
     return [[int(x) for x in line.split()] for line in out.splitlines()]
 
 
+BATCH = r"""
+#include <cstdio>
+#include <cstdlib>
+#include "snkpt_dev.h"
+using namespace snkpt;
+int main(int argc, char** argv) {
+    for (int i = 1; i + 3 < argc; i += 4) {
+        const uint32_t need = (uint32_t)atoi(argv[i]), lanes = (uint32_t)atoi(argv[i + 1]),
+                       per_cu = (uint32_t)atoi(argv[i + 2]), n = (uint32_t)strtoul(argv[i + 3], nullptr, 10);
+        with_stack(need, [&](auto s) {
+            constexpr int S = decltype(s)::value;
+            const TraceGrid g = batch_grid(S, lanes, per_cu, 256, n);
+            printf("%u %u %u %d %d %u %u %u\n", lanes, per_cu, n, S, cu_waves(S), g.blocks, g.threads, g.lds);
+        });
+    }
+    return 0;
+}
+"""
+
+
+@pytest.mark.skipif(HIPCC is None, reason="needs hipcc")
+def test_batch_grid(tmp_path):
+    cus = 256
+    cases = [(need, lanes, per_cu, n) for need in (6, 9, 11, 15, 30, 60) for lanes in (64, 128)
+             for per_cu in (1, 4, 8, 16, 32, 64) for n in (1, 100, 38400, 500000, 15000000)]
+    rows = _run(tmp_path, BATCH, [x for c in cases for x in c])
+    assert len(rows) == len(cases)
+    for lanes, per_cu, n, stack, cu_waves, blocks, threads, lds in rows:
+        resident = cu_waves * 64 // lanes
+        assert threads == lanes  # the block size asked for
+        assert lds == 16 + stack * 8 * lanes and min(per_cu, resident) * lds <= 160 * 1024
+        most = cus * min(per_cu, resident)
+        assert 1 <= blocks <= most
+        if n >= most * lanes:
+            assert blocks == most  # the grid asked for
+        else:
+            assert blocks <= max(n // lanes + 1, cus)
+
+
 @pytest.mark.skipif(HIPCC is None, reason="needs hipcc")
 def test_trace_grid(tmp_path):
     cus = 256
