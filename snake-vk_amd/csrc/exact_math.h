@@ -23,6 +23,13 @@ __device__ __forceinline__ uint32_t bit_sel(uint32_t a, uint32_t b, uint32_t m) 
     return __builtin_amdgcn_bitop3_b32(a, b, m, 0xE4);
 }
 
+// Whether every test holds, without a branch between them (with && the path kernels
+// spilled twice as many registers).
+template <class... B>
+__device__ __forceinline__ bool every(B... b) {
+    return (... & b);
+}
+
 // 2^-100 <= x < 2^100 (false for negative numbers and NaN), in one compare.
 __device__ __forceinline__ bool exact_range(float x) { return __float_as_uint(x) - 0x0D800000u < 0x64000000u; }
 

@@ -157,7 +157,7 @@ __device__ __forceinline__ bool seen_from(V3 d, float d2, V3 nl, float nl2, V3& 
     wi = d * rcp_exact(dist);
     const float x = fabsf(dot(nl, wi));
     cosl = div_exact(x, sqrt_exact(nl2));
-    if (__builtin_expect(exact_range(d2) & exact_range(nl2) & short_range(x), 1)) return true;
+    if (__builtin_expect(every(exact_range(d2), exact_range(nl2), short_range(x)), 1)) return true;
     if (!(d2 > 0.0f)) return false;
     dist = sqrtf(d2);
     wi = d * (1.0f / dist);

@@ -111,7 +111,7 @@ __device__ __forceinline__ float target_at(const GSurf& g, const BrdfView& bv, c
     V3 f = brdf_eval<true>(g.m, bv, g.ns, g.wo, wi, brdf_half(g.m, g.wo, wi));
     const float cc2 = cs * cosl;
     float geo = div_exact(cc2, d2);
-    if (__builtin_expect(!(short_range(cc2) & short_range(d2)), 0)) geo = cc2 / d2;
+    if (__builtin_expect(!every(short_range(cc2), short_range(d2)), 0)) geo = cc2 / d2;
     V3 cc = mul(f, x.le) * geo;
     if (c_out) *c_out = cc;
     if (wi_out) *wi_out = wi;

@@ -43,7 +43,7 @@ __device__ __host__ __forceinline__ V3 cross(V3 a, V3 b) {
 __device__ __forceinline__ V3 normalize(V3 a) {
     const float l2 = dot(a, a);
     // 2^-50 <= l < 2^50, components zero or 2^-74 <= |x| <= l
-    if (__builtin_expect(exact_range(l2) & short_or_zero(a.x, a.y, a.z), 1)) {
+    if (__builtin_expect(every(exact_range(l2), short_or_zero(a.x, a.y, a.z)), 1)) {
         const float l = sqrt_exact(l2), r = rcp_exact(l);
         return V3{div_signed(a.x, l, r), div_signed(a.y, l, r), div_signed(a.z, l, r)};
     }
@@ -150,7 +150,7 @@ __device__ __forceinline__ V3 brdf_eval(const Mat& m, const BrdfView& b, V3 n, V
         // roughness or a normal's length that no material has
         const float DG = div_exact(b.a2, dd) * (b.g1v * div_exact(nl, gl));
         sp = div_exact(DG, denom);
-        ok = b.shrt & short_range(dd) & short_range(nl) & short_range(gl) & short_range(DG) & short_range(denom);
+        ok = every(b.shrt, short_range(dd), short_range(nl), short_range(gl), short_range(DG), short_range(denom));
     }
     if (__builtin_expect(!ok, !SHORT)) sp = b.a2 / dd * (b.g1v * (nl / gl)) / denom;
     V3 spec = F * sp;
