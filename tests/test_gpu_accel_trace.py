@@ -264,9 +264,9 @@ def test_rebuild_after_new_transforms_matches_cpu_twin(gpu):
 
 
 def test_ray_counts_around_band_edges(gpu):
-    """The persistent traversal deals the rays out in bands of (resident waves x
-    64) and splits the last, partial band evenly; ray counts at and around the
-    chunk and band edges (closest and any hit) must each trace every ray once,
+    """The persistent traversal deals the rays out in bands of (blocks x 64) and
+    splits the last, partial band evenly; ray counts at and around the chunk and band
+    edges, of four-wave blocks (up to 22 x 64 rays per CU) and of two large blocks per CU, (closest and any hit) must each trace every ray once,
     bit-identical to the CPU twin."""
     import torch
 
@@ -276,10 +276,10 @@ def test_ray_counts_around_band_edges(gpu):
     ctx = make_ctx(scene)
     world = scene_world(scene)
     b = O.Bvh(world)
-    assert b.depth - 1 <= 10  # the 10-entry stack variant: 16 resident blocks of 2 waves per CU
+    assert b.depth - 1 <= 8  # the 8-entry stack variant: two blocks of 16 waves per CU
     cus = torch.cuda.get_device_properties(0).multi_processor_count
-    band = cus * 16 * 2 * 64
-    counts = sorted({1, 63, 64, 65, 1000, band - 1, band, band + 1, band + 777, 2 * band + 4097})
+    band = 16 * cus * 2 * 64  # 16 bands of the large blocks; cus * 256 rays fill a four-wave block per CU
+    counts = sorted({1, 63, 64, 65, 1000, cus * 256 - 1, cus * 256, cus * 256 + 1, cus * 1024 + 63, band - 1, band, band + 1, band + 777, 2 * band + 4097})
     lo, hi = world[:, :9].reshape(-1, 3).min(0), world[:, :9].reshape(-1, 3).max(0)
     org, dr = raysets.random_rays(counts[-1], lo, hi, seed=21)
     rays = np.concatenate([org, dr], 1)

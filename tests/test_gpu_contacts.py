@@ -55,9 +55,10 @@ def _trace(ctx, rays, dt):
     return [x.cpu().numpy() for x in out]
 
 
-def test_contacts_match_oracle_any_hit_and_restatement(gpu):
+@pytest.mark.parametrize("n", [20000, 81920, 81921, 90001])  # eight lanes per ray up to 81,920 (depth 7)
+def test_contacts_match_oracle_any_hit_and_restatement(gpu, n):
     scene, ctx, arrs, b = _room()
-    rays = _particle_rays(20000, 3)
+    rays = _particle_rays(n, 3)
     dt = 1.0 / 120.0
     t, nw, cp, vel, inst, prim = _trace(ctx, rays, dt)
     ct, ci, cpr, cu, cv, _, _ = b.trace(rays, any_hit=True)
@@ -73,7 +74,8 @@ def test_contacts_match_oracle_any_hit_and_restatement(gpu):
     assert not nw[~hit].any() and not vel[~hit].any() and (inst.view(np.uint32)[~hit] == 0xFFFFFFFF).all()
 
 
-def test_contacts_on_the_deep_bvh_match_oracle(gpu):
+@pytest.mark.parametrize("n", [131072, 200000])  # the largest call with eight lanes per ray, a lane per ray
+def test_contacts_on_the_deep_bvh_match_oracle(gpu, n):
     """The 1.02M-triangle scene (BVH8 depth 12: the 12-entry stack variant, held
     to 80 VGPRs): particle rays over its volume, first hit bit for bit against the
     oracle's any-hit traversal, contact record against the restatement."""
@@ -85,7 +87,6 @@ def test_contacts_on_the_deep_bvh_match_oracle(gpu):
     assert 11 <= ctx.accel_info().depth <= 13
     arrs = O.scene_arrays(scene)
     b = O.Bvh(O.flatten(arrs[0], arrs[1], arrs[2], arrs[3]))
-    n = 200000
     rng = np.random.default_rng(11)
     p = np.stack([rng.uniform(-50, 50, n), rng.uniform(0.0, 12.0, n), rng.uniform(-50, 50, n)], 1)
     d = rng.normal(size=(n, 3))

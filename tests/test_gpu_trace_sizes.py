@@ -1,7 +1,8 @@
 """GPU parity of the ray hand-out: the same rays traced in calls of every size
-class (one ray, part of a wave, the edges of a block's 64-ray chunks and of a
-band of the launch) and with directions whose inverses leave the range of the
-short reciprocal return the hits of the CPU BVH8 traversal bit for bit."""
+class (one ray, part of a wave, the edges of 64-ray chunks, of the blocks and bands of
+a launch, and of the lines between eight lanes per ray, small blocks and large blocks)
+and with directions whose inverses leave the range of the short reciprocal return the
+hits of the CPU BVH8 traversal bit for bit.  A counted call always has a lane per ray."""
 import numpy as np
 import pytest
 
@@ -18,23 +19,36 @@ def room(gpu):
     scene = snkpt.SceneData(1)
     ctx = make_ctx(scene)
     bvh = O.Bvh(scene_world(scene))
-    org, dr = raysets.random_rays(70000, [-1, 0, -1], [1, 2, 1], seed=5)
+    org, dr = raysets.random_rays(400003, [-1, 0, -1], [1, 2, 1], seed=5)
     rays = np.concatenate([org, dr], 1)
     return ctx, bvh, rays, bvh.trace(rays, any_hit=False), bvh.trace(rays, any_hit=True)
 
 
-def _trace(ctx, rays, any_hit):
+@pytest.fixture(scope="module")
+def field(gpu):
+    """1.02M triangles: a deeper tree, another stack variant, the groups' line at 2^17."""
+    import raysets
+    import snkpt
+    scene = snkpt.SceneData(2)
+    ctx = make_ctx(scene)
+    bvh = O.Bvh(scene_world(scene))
+    assert bvh.depth == ctx.accel_info().depth >= 8
+    info = ctx.accel_info()
+    org, dr = raysets.random_rays(360449, list(info.scene_lo), list(info.scene_hi), seed=6)
+    rays = np.concatenate([org, dr], 1)
+    return ctx, rays, bvh.trace(rays, any_hit=False), bvh.trace(rays, any_hit=True)
+
+
+def _trace(ctx, rays, any_hit, counted=False):
     import torch
     o = torch.from_numpy(np.ascontiguousarray(rays[:, :4])).cuda()
     d = torch.from_numpy(np.ascontiguousarray(rays[:, 4:])).cuda()
-    return [None if a is None else a.cpu().numpy() for a in ctx.trace(o, d, any_hit=any_hit)]
+    return [None if a is None else a.cpu().numpy() for a in ctx.trace(o, d, any_hit=any_hit, counted=counted)]
 
 
-@pytest.mark.parametrize("n", [1, 7, 8, 9, 63, 65, 1000, 4097, 32768, 32769, 70000])
-def test_call_sizes(room, n):
-    ctx, _, rays, closest, first = room
+def _check(ctx, rays, n, closest, first, counted):
     for any_hit, want in ((False, closest), (True, first)):
-        got = _trace(ctx, rays[:n], any_hit)
+        got = _trace(ctx, rays[:n], any_hit, counted)
         for k, name in enumerate(["t", "inst", "prim"]):
             assert_bits_equal(got[k], want[k][:n], f"{name}, {n} rays, any hit {any_hit}")
         if not any_hit:
@@ -42,7 +56,32 @@ def test_call_sizes(room, n):
                 assert_bits_equal(got[k], want[k][:n], f"{name}, {n} rays")
 
 
-def test_extreme_directions(room):
+# counted: a lane per ray from the first ray on; blocks of 4 waves take 256 rays, a band of
+# them is 64 rays a block
+@pytest.mark.parametrize("counted", [False, True])
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 63, 65, 1000, 4097, 32768, 32769, 65535, 65536, 65537, 70000])
+def test_call_sizes(room, n, counted):
+    ctx, _, rays, closest, first = room
+    _check(ctx, rays, n, closest, first, counted)
+
+
+# on both sides of the groups' line (81,920 in a tree of depth 7) and of the small blocks'
+# (22 waves' lanes on each of 256 CUs), then of bands of two large blocks per CU
+@pytest.mark.parametrize("n", [81919, 81920, 81921, 100003, 360447, 360448, 360449, 393215, 393217, 400003])
+def test_call_sizes_around_the_lines(room, n):
+    ctx, bvh, rays, closest, first = room
+    assert bvh.depth == 7
+    _check(ctx, rays, n, closest, first, False)
+
+
+@pytest.mark.parametrize("n", [5, 16385, 131071, 131072, 131073, 200003, 360448, 360449])
+def test_call_sizes_of_a_deeper_tree(field, n):
+    ctx, rays, closest, first = field
+    _check(ctx, rays, n, closest, first, False)
+
+
+@pytest.mark.parametrize("counted", [False, True])
+def test_extreme_directions(room, counted):
     """Components at and beyond both ends of the short reciprocal's range, zeros of
     both signs, unnormalised rays, and rays that miss at once (zero, NaN, empty)."""
     ctx, bvh, rays, _, _ = room
@@ -57,6 +96,6 @@ def test_extreme_directions(room):
     r[2, 3], r[2, 7] = 2.0, 1.0
     for any_hit in (False, True):
         want = bvh.trace(r, any_hit=any_hit)
-        got = _trace(ctx, r, any_hit)
+        got = _trace(ctx, r, any_hit, counted)
         for k, name in enumerate(["t", "inst", "prim"]):
             assert_bits_equal(got[k], want[k], f"{name}, any hit {any_hit}")
