@@ -1236,12 +1236,13 @@ snkpt_status cache_infer(snkpt_ctx* ctx, const float* samples, uint32_t n, float
 }
 
 // ---------------------------------------------- queries without allocation ----
-// Workspace of cache_infer_noalloc: the encoded query rows (64 FP16 network
-// inputs = 128 B per query) for at most kNoAllocQueries queries; 8 MiB held on
+// Workspace of cache_infer_noalloc: the encoded queries (64 FP16 network inputs =
+// 128 B per query, in the layout of enc_stride) for at most kNoAllocQueries queries; 8 MiB held on
 // every GPU the library runs on until the process ends.  Every call on a GPU
 // shares that GPU's copy, so calls that overlap on one GPU (any context, any
-// stream) race.  Nothing in it has to start at zero: k_encode writes every row
-// below n before k_mlp_infer reads rows below n only.
+// stream) race.  Nothing in it has to start at zero: the encoding writes all inputs of
+// the queries below n (k_encode in rows, k_encode_dense and k_encode_hashed between them
+// all 32 level-major pairs) before k_mlp_infer reads those of queries below n only.
 static __device__ __align__(256) _Float16 scratch[(size_t)kNoAllocQueries * 64];
 
 namespace {
@@ -1262,7 +1263,7 @@ snkpt_status cache_scratch_init(int device) {
     return SNKPT_OK;
 }
 
-// cache_infer with the encoded rows in `scratch`: no allocation, same kernels,
+// cache_infer with the encoded queries in `scratch`: no allocation, same kernels,
 // bit-identical outputs.
 snkpt_status cache_infer_noalloc(snkpt_ctx* ctx, const float* samples, uint32_t n, float* out, hipStream_t st) {
     CacheState* Cp = ctx->cache;

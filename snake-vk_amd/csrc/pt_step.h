@@ -263,8 +263,10 @@ constexpr uint32_t kServeGroups = 2;
 // path's trace, shade and shadow in its own loop had 8.5 of 64 lanes active per
 // VALU instruction: 774 us for the 367k paths of the 1.02M-triangle frame.)
 // What a path holds between rays stays in its queue slot and path state
-// (in.org / in.dir: its next ray; ps: throughput and random stream), so the
-// traversal loop keeps few registers.  Contributions are added to rad[path] in
+// (in.org / in.dir: its next ray; ps: throughput and random stream).  The traversal
+// state of lanes still under way stays live across the shading of the others, though:
+// at 128 VGPRs (four waves per SIMD) 13 to 20 of them spill, 40 to 52 B a lane; with
+// eight lanes per path 21 (56 B).  Contributions are added to rad[path] in
 // the wavefront's order (emission, then the unoccluded shadow ray, vertex by
 // vertex), so the radiance is bit-identical.  The first ray of each entry was
 // counted when it was queued; stats[1] / stats[2] get the rest.

@@ -457,8 +457,8 @@ PathState paths_of(RenderState& R) {
     return PathState{R.p_thr.as<float4>(), R.p_rng.as<uint2>(), R.p_bounce.as<uint32_t>()};
 }
 
-// The rest of every path queued in `cur` (up to n_max of them), one thread per
-// path on a persistent grid.
+// The rest of every path queued in `cur` (up to n_max of them) in one launch: eight
+// lanes per path, a thread per path or lanes in stages, by n_max.
 snkpt_status launch_tail(snkpt_ctx* ctx, RenderState& R, const SceneDev& S, const PtParams& P, const ShadeHooks& H,
                          int cur, float4* rad, hipStream_t st, uint32_t n_max) {
     const Accel& A = ctx->accel;

@@ -478,8 +478,10 @@ struct RayShare {
     // Lanes of a wave that take rays: all of them, or, when the block's rays do not
     // fill kSpreadWaves waves, an even part of them (at least 8): a small call then
     // uses more SIMDs, and a wave waits for fewer rays.  Waves per block, 65k paths of
-    // a 256 x 256 room frame / 16k collision rays: 2: 455 / 33.6 us, 3: 457 / 35.7,
-    // 4: 471 / 32.9, 6: 500 / 31.4; one 64-ray chunk per wave over the chip 478 / 39.5.
+    // a 256 x 256 room frame / 16k collision rays (while a lane carried each; such calls
+    // take other kernels now, queues shorter than the host's bound and counted calls
+    // still come here): 2: 455 / 33.6 us, 3: 457 / 35.7, 4: 471 / 32.9, 6: 500 / 31.4;
+    // one 64-ray chunk per wave over the chip 478 / 39.5.
     __device__ __forceinline__ uint32_t lanes() const {
         const uint32_t waves = min(kSpreadWaves, blockDim.x >> 6);
         return min(64u, max(8u, (end + waves - 1u) / waves));

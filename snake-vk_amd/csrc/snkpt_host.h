@@ -47,7 +47,7 @@ struct DeviceBuffer {
 // Acceleration structure built by build_accel().
 // Launch shape of the persistent traversal kernel (refill_trace): refill once
 // `refill` lanes of a wave are idle, `steps` traversal steps between two
-// refill checks (3 or 4), `blocks_per_cu` resident 128-lane blocks per CU.
+// refill checks (3 or 4), `blocks_per_cu` resident pairs of waves per CU.
 // refill == 0: not set (the defaults apply).
 struct TraceShape {
     uint32_t refill = 0, steps = 4, blocks_per_cu = 16;

@@ -100,7 +100,7 @@ def test_grouping_and_launch_shapes_do_not_change_images(gpu):
 
 
 def test_tail_bounce_does_not_change_images_or_ray_counts(gpu):
-    """The paths still alive from any bounce on run one thread per path: the
+    """The paths still alive from any bounce on run to their ends in one launch: the
     images and ray counts of the launch-per-bounce frame, bit for bit."""
     import snkpt
     scenes, ctxs, b, outs, cams = _setup()

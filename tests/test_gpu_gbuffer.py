@@ -103,8 +103,8 @@ def test_gbuffer_whole_paths_flag_keeps_the_wavefront_image(gpu):
 
 
 def test_gbuffer_tail_bounces_keep_the_wavefront_image(gpu):
-    """The bounces after the G-buffer vertex, run one thread per path from
-    any bounce on: the wavefront's image bit for bit."""
+    """The bounces after the G-buffer vertex, run in one launch from any
+    bounce on: the wavefront's image bit for bit."""
     w = h = 40
     scene, ctx, arrs, b, cam, gb = _scene_gbuffer(1, w, h)
     gbd = _dev(gb)

@@ -156,8 +156,9 @@ def test_whole_path_kernel_matches_wavefront(gpu, config, w, h):
 
 @pytest.mark.parametrize("config,w,h", [(1, 96, 64), (4, 160, 90), (2, 128, 72), (4, 640, 360)])
 def test_per_thread_tail_matches_wavefront(gpu, config, w, h):
-    """From any bounce on, the paths still alive can run one thread per path
-    instead of a launch per bounce: the image and the ray counts stay those of
+    """From any bounce on, the paths still alive can run to their ends in one launch (a
+    group of lanes or, at 640 x 360, a thread per path) instead of a launch per bounce:
+    the image and the ray counts stay those of
     the pure wavefront bit for bit, for every tail bounce and for the bounce the
     context picks itself from the previous frame's queue lengths."""
     import torch
