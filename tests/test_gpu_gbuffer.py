@@ -102,10 +102,11 @@ def test_gbuffer_whole_paths_flag_keeps_the_wavefront_image(gpu):
     assert np.array_equal(a, c)
 
 
-def test_gbuffer_tail_bounces_keep_the_wavefront_image(gpu):
+# by size: eight lanes per path, a thread per path, lanes in stages
+@pytest.mark.parametrize("w,h", [(40, 40), (257, 161), (700, 500)])
+def test_gbuffer_tail_bounces_keep_the_wavefront_image(gpu, w, h):
     """The bounces after the G-buffer vertex, run in one launch from any
     bounce on: the wavefront's image bit for bit."""
-    w = h = 40
     scene, ctx, arrs, b, cam, gb = _scene_gbuffer(1, w, h)
     gbd = _dev(gb)
     a = _render_gb(ctx, cam, gbd, w, h, max_depth=5, rr_start=3, seed=2, tail_bounce=0xFFFFFFFF)

@@ -28,3 +28,24 @@ def test_path_kernels_match_wavefront(gpu, config, rr, w, h):
     for g in got[1:]:
         assert np.array_equal(g[0].view(np.uint32), got[0][0].view(np.uint32))
         assert g[1:] == got[0][1:]
+
+
+@pytest.mark.parametrize("w,h", [(64, 48), (257, 161), (700, 500)])
+def test_path_kernels_after_restir(gpu, w, h):
+    """The bounces after ReSTIR's primary vertex, by the same kernels."""
+    import snkpt
+    import torch
+    from helpers import make_ctx
+    scene = snkpt.SceneData(1)
+    cam = scene.camera(0, w, h)
+    got = []
+    for tail in (5, 1, 0):
+        ctx = make_ctx(scene)  # no history
+        out = torch.zeros(h, w, 4, device="cuda")
+        s = snkpt.default_settings(mode=snkpt.MODE_RESTIR, max_depth=5, seed=3, tail_bounce=tail)
+        ctx.render(cam, s, out, w, h)
+        st = ctx.frame_stats()
+        got.append((out.cpu().numpy(), st.extension_rays, st.shadow_rays))
+    for g in got[1:]:
+        assert np.array_equal(g[0].view(np.uint32), got[0][0].view(np.uint32))
+        assert g[1:] == got[0][1:]
